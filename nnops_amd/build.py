@@ -27,6 +27,9 @@ DIAG_LIB = os.path.join(PKG, "libnnops_amd_diag.so")
 
 SOURCES = [
     "csrc/kernels/gemm_i8.hip",
+    "csrc/kernels/gemm_i8_nk.hip",
+    "csrc/kernels/gemm_i8_trb.hip",
+    "csrc/kernels/gemm_f16.hip",
     "csrc/kernels/gemm_i8_noalloc.hip",
     "csrc/kernels/q4_1.hip",
     "csrc/kernels/q4_1_codec.hip",

@@ -1,0 +1,181 @@
+// ---------------------------------------------------------------------------
+// The ring over f16 operands (nnops_hip_gemm_fp's large shapes): the same
+// byte staging, K and the row pitches in bytes; B [N][K] rows in place, or a
+// [K][N] B transposed into the workspace first. RING_FP writes alpha * acc
+// straight to C; K splits write f32 partials that ring_f16_reduce sums.
+// ---------------------------------------------------------------------------
+#include "gemm_i8_ring.hpp"
+
+namespace nnops_amd {
+namespace {
+
+// The same for 2-byte elements (an f16 [K][N] B staged as [N][Kp]).
+__global__ __launch_bounds__(256) void transpose_b16(const uint16_t* src, int64_t lds_, int R, int C,
+                                                    uint16_t* dst, int64_t ldd, int Rp)
+{
+    __shared__ uint16_t tile[64][65];
+    const int r0 = blockIdx.y * 64;
+    const int c0 = blockIdx.x * 64;
+    const int tx = threadIdx.x & 63;
+    const int ty = threadIdx.x >> 6;
+    for (int i = ty; i < 64; i += 4) {
+        const int r = r0 + i, c = c0 + tx;
+        tile[i][tx] = (r < R && c < C) ? src[(int64_t)r * lds_ + c] : (uint16_t)0;
+    }
+    __syncthreads();
+    for (int i = ty; i < 64; i += 4) {
+        const int c = c0 + i, r = r0 + tx;
+        if (c < C && r < Rp) {
+            dst[(int64_t)c * ldd + r] = tile[tx][i];
+        }
+    }
+}
+
+// C = alpha * (the f16 ring's f32 partials summed in split order)
+__global__ __launch_bounds__(256) void ring_f16_reduce(GemmI8Kern p, RingSplit sk)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)p.m * p.n) {
+        return;
+    }
+    const int64_t slab = (int64_t)p.m * p.n;
+    float v = 0.0f;
+    for (int sp = 0; sp < sk.splits; ++sp) {
+        v += __builtin_bit_cast(float, sk.part[sp * slab + i]);
+    }
+    v = __fmul_rn(v, p.ep.s_a_scalar);
+    const int m = (int)(i / p.n);
+    const int n = (int)(i - (int64_t)m * p.n);
+    char* crow = static_cast<char*>(p.c) + (int64_t)m * p.ldc_bytes;
+    if (p.ep.out_kind == NNOPS_OUT_F16) {
+        reinterpret_cast<_Float16*>(crow)[n] = (_Float16)v;
+    } else {
+        reinterpret_cast<float*>(crow)[n] = v;
+    }
+}
+
+struct F16Plan {
+    RingPlan ring;          // mode < 0: the ring does not take the call
+    bool stage_b = false;
+    int64_t kp = 0;         // staged B row bytes
+    size_t part_off = 0, total = 0;
+};
+
+F16Plan plan_f16(const NnopsGemmFpArgs& g)
+{
+    F16Plan f;
+    if (!g.in_f16 || g.m < 64 || 2 * g.k > INT32_MAX || g.m > INT32_MAX || g.n > INT32_MAX) {
+        return f;
+    }
+    NnopsGemmI8Args x{};
+    x.m = g.m;
+    x.n = g.n;
+    x.k = 2 * g.k;
+    x.trans_b = 1;
+    x.a = g.a;
+    x.lda = 2 * g.lda;
+    x.c = g.c;
+    x.ldc = g.ldc;
+    x.out_kind = g.out_f16 ? NNOPS_OUT_F16 : NNOPS_OUT_F32;
+    x.act = NNOPS_ACT_NONE;
+    x.s_a_scalar = g.alpha;
+    x.s_b_scalar = 1.0f;
+    const int8_t* b = static_cast<const int8_t*>(g.b);
+    int64_t ldb = 2 * g.ldb;
+    size_t off = 0;
+    if (!g.trans_b) {
+        f.stage_b = true;
+        f.kp = (2 * g.k + 127) / 128 * 128;
+        off += align_up((size_t)g.n * (size_t)f.kp);
+        b = nullptr;          // the staged copy: 256-byte aligned, 128-byte rows
+        ldb = f.kp;
+    }
+    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb);
+    if (f.ring.mode != RING_FP && f.ring.mode != RING_PART) {
+        f.ring = RingPlan{};
+        return f;
+    }
+    // f32 partials cost 8 bytes of traffic per output and split: where
+    // 128 x 256 tiles alone nearly fill the CUs, take them unsplit (512 x
+    // 14336 x 4096: 89.6 us split in two over 256 x 256 tiles)
+    const int64_t tiles128 = ((g.m + 127) / 128) * ((g.n + 255) / 256);
+    const bool c_ok = (uintptr_t)g.c % 16 == 0 && (g.ldc * (g.out_f16 ? 2 : 4)) % 16 == 0;
+    if (f.ring.splits > 1 && g.m > 128 && tiles128 >= 192 && c_ok) {
+        f.ring.bm = 128;
+        f.ring.bn = 256;
+        f.ring.splits = 1;
+        f.ring.mode = RING_FP;
+    }
+    if (f.ring.mode == RING_PART) {
+        f.part_off = off;
+        off += align_up((size_t)f.ring.splits * (size_t)g.m * (size_t)g.n * 4);
+    }
+    f.total = off;
+    return f;
+}
+
+}  // namespace
+
+bool ring_gemm_f16_ok(const NnopsGemmFpArgs& g)
+{
+    return plan_f16(g).ring.mode >= 0;
+}
+
+size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g)
+{
+    // the destination's alignment (which a size query may not see) picks
+    // between the fused output and the split partials: room for either
+    NnopsGemmFpArgs x = g;
+    const size_t a = plan_f16(x).total;
+    x.c = reinterpret_cast<void*>(uintptr_t{2});
+    return std::max(a, plan_f16(x).total);
+}
+
+int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s)
+{
+    const F16Plan f = plan_f16(g);
+    if (f.ring.mode < 0) {
+        return NNOPS_UNSUPPORTED;
+    }
+    if (f.total > 0 && (workspace == nullptr || ws_bytes < f.total)) {
+        return NNOPS_NOT_INITIALIZED;
+    }
+    if ((uintptr_t)workspace % 16 != 0) {
+        return NNOPS_INVALID_ARGUMENT;   // staged operands and partials are 16-byte vectors
+    }
+    char* ws = static_cast<char*>(workspace);
+    GemmI8Kern k{};
+    k.m = (int)g.m;
+    k.n = (int)g.n;
+    k.k = (int)(2 * g.k);
+    k.a = static_cast<const int8_t*>(g.a);
+    k.lda = 2 * g.lda;
+    k.c = g.c;
+    k.ldc_bytes = g.ldc * (g.out_f16 ? 2 : 4);
+    if (f.stage_b) {
+        uint16_t* bt = reinterpret_cast<uint16_t*>(ws);
+        const dim3 grid((unsigned)((g.n + 63) / 64), (unsigned)((f.kp / 2 + 63) / 64));
+        NNOPS_LAUNCH(transpose_b16, grid, dim3(256), 0, s, static_cast<const uint16_t*>(g.b), g.ldb,
+                           (int)g.k, (int)g.n, bt, f.kp / 2, (int)(f.kp / 2));
+        k.b = reinterpret_cast<const int8_t*>(bt);
+        k.ldb = f.kp;
+    } else {
+        k.b = static_cast<const int8_t*>(g.b);
+        k.ldb = 2 * g.ldb;
+    }
+    EpiParams& e = k.ep;
+    e.s_a_scalar = g.alpha;
+    e.s_b_scalar = 1.0f;
+    e.out_kind = g.out_f16 ? NNOPS_OUT_F16 : NNOPS_OUT_F32;
+    e.act = NNOPS_ACT_NONE;
+    e.min_clip = -INFINITY;
+    e.max_clip = INFINITY;
+    const RingSplit sk = ring_split(k, f.ring, reinterpret_cast<int32_t*>(ws + f.part_off));
+    launch_ring_tiles<true, false>(k, f.ring, sk, s);
+    if (f.ring.mode == RING_PART) {
+        NNOPS_LAUNCH(ring_f16_reduce, dim3((unsigned)(((int64_t)k.m * k.n + 255) / 256)), dim3(256), 0, s, k, sk);
+    }
+    return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
+}
+
+}  // namespace nnops_amd
