@@ -30,6 +30,7 @@ SOURCES = [
     "csrc/kernels/gemm_i8_nk.hip",
     "csrc/kernels/gemm_i8_trb.hip",
     "csrc/kernels/gemm_f16.hip",
+    "csrc/kernels/ring_plan.hip",
     "csrc/kernels/gemm_i8_noalloc.hip",
     "csrc/kernels/q4_1.hip",
     "csrc/kernels/q4_1_codec.hip",

@@ -528,11 +528,13 @@ Status run_i8(const QuantCall& q, const Geometry& g, TensorView& out, const Tens
     if (!st.ok) {
         return Status::not_initialized;
     }
-    const size_t need = nnops_hip_gemm_i8_workspace_size(&x);
-    if (need > 0 && (workspace == nullptr || ws_bytes < stage_cap + need)) {
+    // all that lies past the staged tables: the plan that the call's pointers
+    // select takes what it needs of it
+    if (workspace == nullptr || ws_bytes < stage_cap) {
         return Status::not_initialized;
     }
-    void* ws = need > 0 ? static_cast<char*>(workspace) + stage_cap : nullptr;
+    void* ws = static_cast<char*>(workspace) + stage_cap;
+    const size_t ws_left = ws_bytes - stage_cap;
 
     const int64_t a_rows_per = g.trans_a ? g.k : g.m;
     const int64_t b_rows_per = g.trans_b ? g.n : g.k;
@@ -550,7 +552,7 @@ Status run_i8(const QuantCall& q, const Geometry& g, TensorView& out, const Tens
             xb.s_a = x.s_a != nullptr ? x.s_a + row_base : nullptr;
             xb.zp_a = x.zp_a != nullptr ? x.zp_a + row_base : nullptr;
         }
-        const int rc = nnops_hip_gemm_i8(&xb, ws, need, stream);
+        const int rc = nnops_hip_gemm_i8(&xb, ws, ws_left, stream);
         if (rc != NNOPS_OK) {
             return from_code(rc);
         }
@@ -784,11 +786,13 @@ Status run_quant(const QuantCall& q, TensorView& out, std::span<const TensorView
         x.ldb = b.row_stride_elems();
         x.ldc = pass ? g.n : out.row_stride_elems();
         const size_t tmp = q4_1_pass_bytes(g, q);
-        const size_t need = nnops_hip_gemm_fp_workspace_size(&x);
-        if ((need > 0 || tmp > 0) && (workspace == nullptr || ws_bytes < tmp + align_up(need))) {
+        if (tmp > 0 && (workspace == nullptr || ws_bytes < tmp)) {
             return Status::not_initialized;
         }
-        char* gemm_ws = static_cast<char*>(workspace) + tmp;
+        // the product's own workspace is what follows (it says itself when
+        // that is too little)
+        char* gemm_ws = workspace != nullptr ? static_cast<char*>(workspace) + tmp : nullptr;
+        const size_t ws_left = workspace != nullptr ? ws_bytes - tmp : 0;
         NnopsFpOutArgs fo = fp_pass_args(q, g, out, bias, workspace);
         const int64_t a_mat = a_rows_per * a.pitch();
         const int64_t b_mat = b_rows_per * b.pitch();
@@ -799,7 +803,7 @@ Status run_quant(const QuantCall& q, TensorView& out, std::span<const TensorView
             xb.b = b.ptr<const char>() + batch_offset(bi, g, g.b_batch, b_mat);
             char* cb = out.ptr<char>() + batch_offset(bi, g, g.out_batch, c_mat);
             xb.c = pass ? workspace : static_cast<void*>(cb);
-            const int rc = nnops_hip_gemm_fp(&xb, gemm_ws, need, stream);
+            const int rc = nnops_hip_gemm_fp(&xb, gemm_ws, ws_left, stream);
             if (rc != NNOPS_OK) {
                 return from_code(rc);
             }

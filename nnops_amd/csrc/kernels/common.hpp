@@ -90,6 +90,10 @@ inline uint64_t next_launch_epoch()
 // ---------------------------------------------------------------------------
 // Epilogue parameters, resolved once on the host (device pointers only).
 // ---------------------------------------------------------------------------
+// The least workspace nnops_hip_gemm_i8 runs a call with (its plan without K
+// splits; nnops_hip_gemm_i8_workspace_size is what the full plan takes).
+size_t gemm_i8_least_workspace(const NnopsGemmI8Args& g);
+
 struct EpiParams {
     const int32_t* bias;       // [N] int32 (integer outputs) or nullptr
     const int32_t* r_a;        // [M] sum_k A (true values), or nullptr

@@ -22,8 +22,8 @@
 //                         64 x 64, v_mfma_f32_32x32x2f32 with A and B staged
 //                         in LDS as f32 (32-deep k stages). Bound: f32 MFMA.
 //   fp_split_sum          C = alpha * (sum of the K splits in split order).
-// The f16 operands of large aligned shapes take the int8 ring GEMM's byte
-// staging with f16 MFMA instead (gemm_i8.hip, nnops_amd::ring_gemm_f16).
+// The f16 operands of aligned shapes past a few rows take the int8 ring GEMM's byte
+// staging with f16 MFMA instead (gemm_f16.hip, nnops_amd::ring_gemm_f16).
 #include "common.hpp"
 
 #include <algorithm>
@@ -31,9 +31,9 @@
 
 namespace nnops_amd {
 
-// gemm_i8.hip: the ring GEMM over f16 operands (C = alpha A B^T, f32 or f16
-// C; B [N][K] rows), or false when the shape / alignment does not fit it.
-bool ring_gemm_f16_ok(const NnopsGemmFpArgs& g);
+// gemm_f16.hip: the ring GEMM over f16 operands (C = alpha A B, f32 or f16 C),
+// or NNOPS_UNSUPPORTED, nothing launched, where the shape, the alignment or
+// (below 64 rows) the workspace does not fit it.
 int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s);
 size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g);
 
@@ -545,6 +545,17 @@ bool use_gemv_fp(const NnopsGemmFpArgs& g)
     return g.m <= kGemvMaxM;
 }
 
+// the [K][N] GEMV's K-split partials
+size_t gemv_fp_workspace(const NnopsGemmFpArgs& g)
+{
+    if (g.trans_b) {
+        return 0;
+    }
+    const int splits = kn_splits_fp(g.n, g.k, g.in_f16 != 0);
+    const int64_t rows = std::min<int64_t>(g.m, kGemvRows);
+    return splits > 1 ? (size_t)splits * (size_t)rows * (size_t)g.n * sizeof(float) : 0;
+}
+
 }  // namespace
 }  // namespace nnops_amd
 
@@ -555,20 +566,10 @@ extern "C" size_t nnops_hip_gemm_fp_workspace_size(const NnopsGemmFpArgs* g)
     if (g == nullptr || g->m <= 0 || g->n <= 0 || g->k <= 0) {
         return 0;
     }
-    if (use_gemv_fp(*g)) {
-        if (g->trans_b) {
-            return 0;
-        }
-        const int splits = kn_splits_fp(g->n, g->k, g->in_f16 != 0);
-        const int64_t rows = std::min<int64_t>(g->m, kGemvRows);
-        return splits > 1 ? (size_t)splits * (size_t)rows * (size_t)g->n * sizeof(float) : 0;
-    }
-    if (g->in_f16) {
-        // room for the ring's plan, which pointer alignment (not seen by a
-        // size query) may rule out in favour of the tile kernel (none)
-        return ring_gemm_f16_workspace(*g);
-    }
-    return 0;
+    const size_t gemv = use_gemv_fp(*g) ? gemv_fp_workspace(*g) : 0;
+    // room for the ring's plan, which pointer alignment (not seen by a size
+    // query) may rule out in favour of the GEMV or the tile kernel
+    return g->in_f16 ? std::max(gemv, ring_gemm_f16_workspace(*g)) : gemv;
 }
 
 extern "C" int nnops_hip_gemm_fp(const NnopsGemmFpArgs* g, void* workspace, size_t ws_bytes, void* stream)
@@ -592,12 +593,18 @@ extern "C" int nnops_hip_gemm_fp(const NnopsGemmFpArgs* g, void* workspace, size
     if (g->lda < g->k || g->ldc < g->n || g->ldb < (g->trans_b ? g->k : g->n)) {
         return NNOPS_INVALID_ARGUMENT;
     }
-    const size_t need = nnops_hip_gemm_fp_workspace_size(g);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool f16 = g->in_f16 != 0;
+    if (f16 && g->k > 0) {
+        // the f16 ring, where it takes the call
+        if (const int rc = ring_gemm_f16(*g, workspace, ws_bytes, s); rc != NNOPS_UNSUPPORTED) {
+            return rc;
+        }
+    }
+    const size_t need = use_gemv_fp(*g) ? gemv_fp_workspace(*g) : 0;
     if (need > 0 && (workspace == nullptr || ws_bytes < need)) {
         return NNOPS_NOT_INITIALIZED;
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool f16 = g->in_f16 != 0;
     const int es = f16 ? 2 : 4;
     FpKern k{};
     k.a = g->a;
@@ -647,9 +654,6 @@ extern "C" int nnops_hip_gemm_fp(const NnopsGemmFpArgs* g, void* workspace, size
             }
         }
         return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
-    }
-    if (f16 && ring_gemm_f16_ok(*g)) {
-        return ring_gemm_f16(*g, workspace, ws_bytes, s);
     }
     const int64_t tiles = ((g->m + 127) / 128) * ((g->n + 127) / 128);
     if (tiles > INT32_MAX) {

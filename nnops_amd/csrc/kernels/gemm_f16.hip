@@ -31,26 +31,41 @@ __global__ __launch_bounds__(256) void transpose_b16(const uint16_t* src, int64_
     }
 }
 
-// C = alpha * (the f16 ring's f32 partials summed in split order)
+// C = alpha * (the f16 ring's f32 partials summed in split order): 4 columns
+// per thread (N % 4 == 0), grid.y walking the rows; a group's splits are loaded
+// four at a time ahead of their sum. Bound: HBM / MALL.
 __global__ __launch_bounds__(256) void ring_f16_reduce(GemmI8Kern p, RingSplit sk)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t)p.m * p.n) {
+    const int nb = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
+    if (nb >= p.n) {
         return;
     }
+    const bool f16 = p.ep.out_kind == NNOPS_OUT_F16;
     const int64_t slab = (int64_t)p.m * p.n;
-    float v = 0.0f;
-    for (int sp = 0; sp < sk.splits; ++sp) {
-        v += __builtin_bit_cast(float, sk.part[sp * slab + i]);
-    }
-    v = __fmul_rn(v, p.ep.s_a_scalar);
-    const int m = (int)(i / p.n);
-    const int n = (int)(i - (int64_t)m * p.n);
-    char* crow = static_cast<char*>(p.c) + (int64_t)m * p.ldc_bytes;
-    if (p.ep.out_kind == NNOPS_OUT_F16) {
-        reinterpret_cast<_Float16*>(crow)[n] = (_Float16)v;
-    } else {
-        reinterpret_cast<float*>(crow)[n] = v;
+    for (int m = (int)blockIdx.y; m < p.m; m += (int)gridDim.y) {
+        const float* src = reinterpret_cast<const float*>(sk.part) + (int64_t)m * p.n + nb;
+        v4f v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        int sp = 0;
+        for (; sp + 3 < sk.splits; sp += 4) {
+            const v4f x0 = *reinterpret_cast<const v4f*>(src + sp * slab);
+            const v4f x1 = *reinterpret_cast<const v4f*>(src + (sp + 1) * slab);
+            const v4f x2 = *reinterpret_cast<const v4f*>(src + (sp + 2) * slab);
+            const v4f x3 = *reinterpret_cast<const v4f*>(src + (sp + 3) * slab);
+            v = (((v + x0) + x1) + x2) + x3;
+        }
+        for (; sp < sk.splits; ++sp) {
+            v += *reinterpret_cast<const v4f*>(src + sp * slab);
+        }
+        char* crow = static_cast<char*>(p.c) + (int64_t)m * p.ldc_bytes;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float y = __fmul_rn(v[e], p.ep.s_a_scalar);
+            if (f16) {
+                reinterpret_cast<_Float16*>(crow)[nb + e] = (_Float16)y;
+            } else {
+                reinterpret_cast<float*>(crow)[nb + e] = y;
+            }
+        }
     }
 }
 
@@ -61,10 +76,15 @@ struct F16Plan {
     size_t part_off = 0, total = 0;
 };
 
-F16Plan plan_f16(const NnopsGemmFpArgs& g)
+// From 3 rows over [N][K] rows of B (4096 x 4096: 3 rows 13.7 us against the
+// GEMV's 19.6, 16 rows 13.7 against 21.4; 2 rows stay with the GEMV, 9.7) and
+// from 17 over a [K][N] B, whose transposed copy the GEMV needs not (17 to 63
+// rows on gemm_fp_tile, in f32: 475 us). lean: the plan for a workspace too
+// small for the full one, without K splits.
+F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
 {
     F16Plan f;
-    if (!g.in_f16 || g.m < 64 || 2 * g.k > INT32_MAX || g.m > INT32_MAX || g.n > INT32_MAX) {
+    if (!g.in_f16 || g.m < (g.trans_b ? 3 : 17) || 2 * g.k > INT32_MAX || g.m > INT32_MAX || g.n > INT32_MAX) {
         return f;
     }
     NnopsGemmI8Args x{};
@@ -90,21 +110,11 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g)
         b = nullptr;          // the staged copy: 256-byte aligned, 128-byte rows
         ldb = f.kp;
     }
-    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb);
+    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb, false, lean ? 1 : 16);
     if (f.ring.mode != RING_FP && f.ring.mode != RING_PART) {
         f.ring = RingPlan{};
+        f.stage_b = false;
         return f;
-    }
-    // f32 partials cost 8 bytes of traffic per output and split: where
-    // 128 x 256 tiles alone nearly fill the CUs, take them unsplit (512 x
-    // 14336 x 4096: 89.6 us split in two over 256 x 256 tiles)
-    const int64_t tiles128 = ((g.m + 127) / 128) * ((g.n + 255) / 256);
-    const bool c_ok = (uintptr_t)g.c % 16 == 0 && (g.ldc * (g.out_f16 ? 2 : 4)) % 16 == 0;
-    if (f.ring.splits > 1 && g.m > 128 && tiles128 >= 192 && c_ok) {
-        f.ring.bm = 128;
-        f.ring.bn = 256;
-        f.ring.splits = 1;
-        f.ring.mode = RING_FP;
     }
     if (f.ring.mode == RING_PART) {
         f.part_off = off;
@@ -115,11 +125,6 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g)
 }
 
 }  // namespace
-
-bool ring_gemm_f16_ok(const NnopsGemmFpArgs& g)
-{
-    return plan_f16(g).ring.mode >= 0;
-}
 
 size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g)
 {
@@ -133,14 +138,21 @@ size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g)
 
 int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s)
 {
-    const F16Plan f = plan_f16(g);
+    if (workspace == nullptr || (g.m < 64 && (uintptr_t)workspace % 16 != 0)) {
+        ws_bytes = 0;
+    }
+    F16Plan f = plan_f16(g);
+    if (ws_bytes < f.total) {
+        f = plan_f16(g, true);
+    }
     if (f.ring.mode < 0) {
         return NNOPS_UNSUPPORTED;
     }
-    if (f.total > 0 && (workspace == nullptr || ws_bytes < f.total)) {
-        return NNOPS_NOT_INITIALIZED;
+    if (ws_bytes < f.total) {
+        // below 64 rows the caller has kernels that need none
+        return g.m < 64 ? NNOPS_UNSUPPORTED : NNOPS_NOT_INITIALIZED;
     }
-    if ((uintptr_t)workspace % 16 != 0) {
+    if (g.m >= 64 && (uintptr_t)workspace % 16 != 0) {
         return NNOPS_INVALID_ARGUMENT;   // staged operands and partials are 16-byte vectors
     }
     char* ws = static_cast<char*>(workspace);
@@ -173,7 +185,8 @@ int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hi
     const RingSplit sk = ring_split(k, f.ring, reinterpret_cast<int32_t*>(ws + f.part_off));
     launch_ring_tiles<true, false>(k, f.ring, sk, s);
     if (f.ring.mode == RING_PART) {
-        NNOPS_LAUNCH(ring_f16_reduce, dim3((unsigned)(((int64_t)k.m * k.n + 255) / 256)), dim3(256), 0, s, k, sk);
+        const dim3 grid((unsigned)((k.n / 4 + 255) / 256), (unsigned)std::min(k.m, 65535));
+        NNOPS_LAUNCH(ring_f16_reduce, grid, dim3(256), 0, s, k, sk);
     }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }

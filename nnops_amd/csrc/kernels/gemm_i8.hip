@@ -1594,7 +1594,6 @@ struct WsPlan {
     KnPlan kn;
 };
 
-inline bool aligned16(const void* p, int64_t ld) { return ((uintptr_t)p % 16 == 0) && (ld % 16 == 0); }
 
 // M <= 16 with a [K,N] B: 16-byte (M <= 2) or 4-byte column groups per lane,
 // K % 16 == 0, dword-aligned A rows (scalar loads), no term that needs the
@@ -1654,85 +1653,9 @@ KnPlan plan_kn(const NnopsGemmI8Args& g)
 }
 
 
-}  // namespace
-
-// The ring kernel needs 64-byte k steps, 16-byte-aligned k-contiguous rows,
-// N % 4 == 0 (int32 groups), and 32-bit buffer offsets within a row panel.
-// Tile shape by M: a 257..384-row problem takes two 192x128 tiles (384x128 when
-// K % 128 != 0), 128x256 and 256x128 the small ones, 256x256 the rest. K is split when the
-// tiles alone do not fill the 256 CUs (at least 8 k steps per split). The
-// fused output modes need row-uniform parameters, no zero-point terms,
-// half-away rounding, 16-byte-aligned tables and destination, and no split;
-// everything else writes raw partials and runs gemm_i8_reduce.
-// trb: B is the caller's [K,N] (row pitch ldb), read in place (its whole
-// span within 32-bit buffer offsets). small_tiles: grids of fewer than 32
-// tiles take 64 x 64 tiles of 4 waves instead (config 1, 128 x 1024 x 1024:
-// 32 workgroups in place of 4).
-RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
-                   bool trb, bool small_tiles)
-{
-    RingPlan r;
-    if (g.m <= 16 || g.k % 64 != 0 || g.n % 4 != 0 || g.m < 64 || !aligned16(a, lda) || !aligned16(b, ldb)) {
-        return r;
-    }
-    if (trb && (g.k * ldb + g.n >= (int64_t)INT32_MAX || ldb < g.n)) {
-        return r;
-    }
-    r.trb = trb;
-    if (g.m > 256 && g.m <= 384 && g.k % 128 == 0) {
-        // two 192-row tiles: twice the tiles of one 384-row tile, so half the
-        // K splits (and half the partial-sum traffic) fill the CUs
-        r.bm = 192; r.bn = 128;
-    } else if (g.m > 256 && g.m <= 384) {
-        r.bm = 384; r.bn = 128;
-    } else if (g.m <= 128) {
-        r.bm = 128; r.bn = 256;
-    } else if (g.m <= 256) {
-        r.bm = 256; r.bn = 128;
-    } else {
-        r.bm = 256; r.bn = 256;
-    }
-    if (small_tiles && ((g.m + r.bm - 1) / r.bm) * ((g.n + r.bn - 1) / r.bn) < 32) {
-        r.bm = 64; r.bn = 64;
-    }
-    if ((int64_t)r.bm * lda >= (int64_t)INT32_MAX || (!trb && (int64_t)r.bn * ldb >= (int64_t)INT32_MAX)) {
-        r = RingPlan{};
-        return r;
-    }
-    const int64_t tiles = ((g.m + r.bm - 1) / r.bm) * ((g.n + r.bn - 1) / r.bn);
-    r.bk = (g.k % 128 == 0) ? 128 : 64;
-    const int kt = (int)(g.k / r.bk);
-    // at least 512 k per split, and no split below 16 k steps: a short ring
-    // gains less from splitting than the reduce launch costs (config 1,
-    // 128x1024x1024 s32: 10.5 + 3.9 us in two splits, 12.4 us unsplit)
-    r.splits = kt < 16 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(256 / tiles, kt / (512 / r.bk)));
-    // (the 64 x 64 tiles of config 1 split 4 ways: 4.2 us ring + 3.4 us
-    // reduce against 6.4 us unsplit)
-    const bool compensate = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0 || g.zp_b != nullptr ||
-                            g.zp_b_scalar != 0;
-    const bool tables16 = ((uintptr_t)g.bias % 16 == 0) && ((uintptr_t)g.s_b % 16 == 0);
-    const bool fp_out = g.out_kind == NNOPS_OUT_F32 || g.out_kind == NNOPS_OUT_F16;
-    const bool plain = !compensate && g.s_out_rows == nullptr && g.zp_out_rows == nullptr && !g.float_ep &&
-                       !g.round_even && !fp_out && tables16 && ((uintptr_t)g.c % 16 == 0);
-    r.mode = RING_PART;
-    const size_t ebytes = g.out_kind == NNOPS_OUT_F16 ? 2 : 4;
-    if (r.splits == 1 && fp_out && !compensate && (g.act == NNOPS_ACT_NONE || g.act == NNOPS_ACT_RELU) &&
-        (uintptr_t)g.c % 16 == 0 && (g.ldc * ebytes) % 16 == 0 &&
-        ((uintptr_t)g.s_b % 16) == 0 && (g.bias_fp == nullptr || (uintptr_t)g.bias_fp % (4 * ebytes) == 0)) {
-        r.mode = RING_FP;      // dequantizing output pass fused
-    } else if (r.splits == 1 && plain) {
-        if (g.out_kind == NNOPS_OUT_S32 && (g.ldc * 4) % 16 == 0) {
-            r.mode = RING_S32;
-        } else if (g.out_kind != NNOPS_OUT_S32 && g.s_a == nullptr && g.ldc % 16 == 0 && g.n % 16 == 0) {
-            r.mode = RING_S8;
-        }
-    }
-    return r;
-}
-
-namespace {
-
-WsPlan plan_workspace(const NnopsGemmI8Args& g)
+// lean: the plan for a workspace too small for the full one: no K split, and
+// below 64 rows no ring (gemm_i8_mfma writes no partials).
+WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
 {
     WsPlan w;
     size_t off = 0;
@@ -1760,16 +1683,20 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g)
     // a [K,N] B goes to the ring in place when it takes it and no column
     // sums of B are needed (they are summed over the staged copy's rows)
     const bool need_rb = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0;
-    if (!g.trans_b && !need_rb) {
-        w.ring = plan_ring(g, a, lda, b, ldb, true, true);
+    // (from 17 rows: 24 x 11008 x 4096 s8 15.8 us on 64 x 64 tiles in four
+    // splits, 52 us on gemm_i8_mfma's 64 workgroups of the whole K)
+    const bool ring = g.m > 16 && !(lean && g.m < 64);
+    const int max_splits = lean ? 1 : 16;
+    if (!g.trans_b && !need_rb && ring) {
+        w.ring = plan_ring(g, a, lda, b, ldb, true, max_splits);
     }
     if (!g.trans_b && w.ring.mode < 0) {
         w.b_t = off; off += align_up((size_t)g.n * (size_t)w.kp);
         b = nullptr;
         ldb = w.kp;
     }
-    if (!w.ring.trb) {
-        w.ring = plan_ring(g, a, lda, b, ldb, false, true);
+    if (!w.ring.trb && ring) {
+        w.ring = plan_ring(g, a, lda, b, ldb, false, max_splits);
     }
     if (w.ring.mode == RING_PART) {
         w.part = off; off += align_up((size_t)w.ring.splits * (size_t)g.m * (size_t)g.n * 4);
@@ -1986,6 +1913,11 @@ extern "C" size_t nnops_hip_gemm_i8_workspace_size(const NnopsGemmI8Args* g)
     return plan_workspace(*g).total;
 }
 
+size_t nnops_amd::gemm_i8_least_workspace(const NnopsGemmI8Args& g)
+{
+    return plan_workspace(g, true).total;
+}
+
 extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, void* stream)
 {
     const TimingDisarm disarm;
@@ -2021,7 +1953,10 @@ extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size
     if (g->lda < min_lda || g->ldb < min_ldb || g->ldc < g->n) {
         return NNOPS_INVALID_ARGUMENT;
     }
-    const WsPlan w = plan_workspace(*g);
+    WsPlan w = plan_workspace(*g);
+    if (ws_bytes < w.total) {
+        w = plan_workspace(*g, true);
+    }
     if (w.total > 0 && (workspace == nullptr || ws_bytes < w.total)) {
         return NNOPS_NOT_INITIALIZED;
     }

@@ -43,9 +43,12 @@ struct RingPlan {
     bool trb = false;       // B is [K,N] row-major, read in place (TRB)
 };
 
-// The ring plan of an int8 call (gemm_i8.hip).
-RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
-                   bool trb = false, bool small_tiles = false);
+// The ring plan of an int8 call (ring_plan.hip); an f16 call asks with its K and
+// row pitches in bytes.
+RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, bool trb,
+                   int max_splits);
+
+inline bool aligned16(const void* p, int64_t ld) { return ((uintptr_t)p % 16 == 0) && (ld % 16 == 0); }
 
 // The ring of a plan over [N,K] rows of B (gemm_i8_nk.hip) and over a [K,N] B
 // in place (gemm_i8_trb.hip).
@@ -312,7 +315,7 @@ __device__ __forceinline__ void ring_coords(int tiles_m, int tiles_n, int& tm, i
 // fragment: k rows +0..7 and +8..15 of the lane's 16). No transposed copy.
 template <int BM, int BN, int WM, int WN, int BK, int NS, int MODE, bool FLIP, bool F16 = false, bool TRB = false>
 __global__ __launch_bounds__(WM * WN * 64)
-__attribute__((amdgpu_waves_per_eu((WM * WN + 3) / 4, (WM * WN + 3) / 4)))
+__attribute__((amdgpu_waves_per_eu((WM * WN + 3) / 4, BM + BN <= 192 ? 4 : (WM * WN + 3) / 4)))
 void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
 {
     static_assert(!F16 || MODE == RING_FP || MODE == RING_PART, "f16 operands: fp or partial outputs");
@@ -1183,10 +1186,13 @@ void launch_ring_cfg(const GemmI8Kern& k, const RingSplit& sk, int bk, int mode,
 {
     if (bk == 128) {
         // three stage slots where the LDS holds them (config 5's 192x128 tiles:
-        // 33.7 -> 32.9 us), two for the 256x256 tile; the 64 x 64 tiles of
-        // small grids keep 8 stages in flight (their latency is the call's)
+        // 33.7 -> 32.9 us), two for the 256x256 tile, four for the tiles of
+        // 128 columns and rows or fewer; the 64 x 64 tiles of small grids keep
+        // 8 stages in flight (their latency is the call's)
         if constexpr (BM + BN <= 128) {
             launch_ring_bk<BM, BN, WM, WN, 128, 8, F16, TRB>(k, sk, mode, flip, s);
+        } else if constexpr (BM + BN <= 256) {
+            launch_ring_bk<BM, BN, WM, WN, 128, 4, F16, TRB>(k, sk, mode, flip, s);
         } else if constexpr ((BM + BN) * 128 * 3 <= 160 * 1024 && BM + BN < 512) {
             launch_ring_bk<BM, BN, WM, WN, 128, 3, F16, TRB>(k, sk, mode, flip, s);
         } else {
@@ -1202,18 +1208,19 @@ template <bool F16, bool TRB>
 void launch_ring_tiles(const GemmI8Kern& k, const RingPlan& r, const RingSplit& sk, hipStream_t s)
 {
     const bool flip = k.a_xor != 0u;
-    if (r.bm == 384) {
-        launch_ring_cfg<384, 128, 4, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
-    } else if (r.bm == 192) {
+    auto is = [&](int bm, int bn) { return r.bm == bm && r.bn == bn; };
+    if (is(64, 64)) {
+        launch_ring_cfg<64, 64, 2, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+    } else if (is(128, 64)) {
+        launch_ring_cfg<128, 64, 2, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+    } else if (is(128, 128)) {
+        launch_ring_cfg<128, 128, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+    } else if (is(192, 128)) {
         launch_ring_cfg<192, 128, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
-    } else if (r.bm == 128) {
-        launch_ring_cfg<128, 256, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
-    } else if (r.bm == 64) {
-        if constexpr (!F16) {
-            launch_ring_cfg<64, 64, 2, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
-        }
-    } else if (r.bn == 128) {
+    } else if (is(256, 128)) {
         launch_ring_cfg<256, 128, 4, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+    } else if (is(128, 256)) {
+        launch_ring_cfg<128, 256, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
     } else {
         launch_ring_cfg<256, 256, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
     }

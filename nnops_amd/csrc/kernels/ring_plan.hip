@@ -1,0 +1,120 @@
+// Which tile and K split a call of the LDS-ring GEMM takes (host code).
+#include "gemm_i8_ring.hpp"
+
+namespace nnops_amd {
+namespace {
+
+// The ring's tile shapes and the time of one 128-byte k step of one
+// workgroup, with one workgroup on every CU (the loop's time over its steps,
+// at 512 x 4096 x 4096 and up, int8 and f16 operands alike: the step moves
+// the same bytes and runs as many matrix-core cycles).
+struct RingTile {
+    int bm, bn;
+    float step_us;
+    bool narrow;        // has a form with 64-byte k steps (K % 128 != 0)
+};
+constexpr RingTile kRingTiles[] = {
+    {64, 64, 0.38f, true},    {128, 64, 0.48f, true},   {128, 128, 0.68f, true},  {192, 128, 0.82f, false},
+    {256, 128, 1.08f, true},  {128, 256, 1.08f, true},  {256, 256, 1.80f, true},
+};
+
+}  // namespace
+
+// The ring kernel needs 64-byte k steps, 16-byte-aligned k-contiguous rows,
+// N % 4 == 0 (int32 groups), and 32-bit buffer offsets within a row panel.
+// The tile and the K split are the cheapest by
+//   rounds of 256 workgroups x k steps x the tile's step time
+//   + (partials: 3 us, and their bytes written and read at 3.5 TB/s),
+// since every sweep of tiles and splits (int8 and f16, 24 to 4096 rows) was
+// won by a grid just under one workgroup per CU, whichever tile gives it, and
+// a second workgroup on a CU doubles the time: 512 x 4096 x 4096 s8 18.4 us on
+// 256 tiles of 128 x 64, 21 on 128 of 128 x 128, 27 on 512 of 64 x 64, 35 in
+// eight K splits of 256 x 256; 1024 x 4096 x 4096 24.7 us on 256 tiles of
+// 128 x 128, 42 on 256 x 256 in four splits. The estimate is within 20 % of
+// the measured time where the matrix work or the staging bounds it. Partials
+// stay under 32 MiB, a split keeps at least 512 bytes of k, a k of fewer than
+// 16 steps is not split (the reduce costs more than it gains), and a problem
+// of few rows is split over small tiles only, which bounds the partials (and
+// so the workspace) by those of one tile per CU. max_splits 1: no split, for
+// a workspace too small for the partials.
+// The fused output modes need row-uniform parameters, no zero-point terms,
+// half-away rounding, 16-byte-aligned tables and destination, and no split;
+// everything else writes raw partials and runs gemm_i8_reduce.
+// trb: B is the caller's [K,N] (row pitch ldb), read in place (its whole
+// span within 32-bit buffer offsets).
+RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, bool trb,
+                   int max_splits)
+{
+    RingPlan r;
+    if (g.m < 1 || g.n < 4 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX || g.k < 64 || g.k % 64 != 0 || g.n % 4 != 0 || !aligned16(a, lda) || !aligned16(b, ldb)) {
+        return r;
+    }
+    if (trb && (g.k * ldb + g.n >= (int64_t)INT32_MAX || ldb < g.n)) {
+        return r;
+    }
+    const bool compensate = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0 || g.zp_b != nullptr ||
+                            g.zp_b_scalar != 0;
+    const bool tables16 = ((uintptr_t)g.bias % 16 == 0) && ((uintptr_t)g.s_b % 16 == 0);
+    const bool fp_out = g.out_kind == NNOPS_OUT_F32 || g.out_kind == NNOPS_OUT_F16;
+    const bool plain = !compensate && g.s_out_rows == nullptr && g.zp_out_rows == nullptr && !g.float_ep &&
+                       !g.round_even && !fp_out && tables16 && ((uintptr_t)g.c % 16 == 0);
+    const size_t ebytes = g.out_kind == NNOPS_OUT_F16 ? 2 : 4;
+    int fused = RING_PART;
+    if (fp_out && !compensate && (g.act == NNOPS_ACT_NONE || g.act == NNOPS_ACT_RELU) &&
+        (uintptr_t)g.c % 16 == 0 && (g.ldc * ebytes) % 16 == 0 &&
+        ((uintptr_t)g.s_b % 16) == 0 && (g.bias_fp == nullptr || (uintptr_t)g.bias_fp % (4 * ebytes) == 0)) {
+        fused = RING_FP;       // dequantizing output pass fused
+    } else if (plain) {
+        if (g.out_kind == NNOPS_OUT_S32 && (g.ldc * 4) % 16 == 0) {
+            fused = RING_S32;
+        } else if (g.out_kind != NNOPS_OUT_S32 && g.s_a == nullptr && g.ldc % 16 == 0 && g.n % 16 == 0) {
+            fused = RING_S8;
+        }
+    }
+    const int bk = (g.k % 128 == 0) ? 128 : 64;
+    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)(g.k / bk);
+    const float out_bytes = 4.0f * (float)m * (float)n;
+    const float step_scale = (float)bk / 128.0f;
+    const uint32_t most = std::min(16u, std::min(kt * (uint32_t)bk / 512u, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)));
+    const int split_area = m <= 256 ? 256 * 128 : m <= 384 ? 192 * 128 : 256 * 256;
+    float best = 0.0f;
+    for (const RingTile& t : kRingTiles) {
+        if ((bk == 64 && !t.narrow) || t.bm * lda >= (int64_t)INT32_MAX ||
+            (!trb && t.bn * ldb >= (int64_t)INT32_MAX)) {
+            continue;
+        }
+        const uint64_t tiles = (uint64_t)((m + t.bm - 1) / (uint32_t)t.bm) * ((n + t.bn - 1) / (uint32_t)t.bn);
+        const float step = t.step_us * step_scale;
+        auto consider = [&](uint32_t sp, uint64_t rounds) {
+            const uint32_t steps = kt - (sp - 1) * (kt / sp);       // the last split's, the longest
+            const bool part = sp > 1 || fused == RING_PART;
+            const float us = (float)rounds * (float)steps * step +
+                             (part ? 3.0f + 2.0f * (float)sp * out_bytes / 3.5e6f : 0.0f);
+            if (r.bm == 0 || us < best) {
+                best = us;
+                r.bm = t.bm;
+                r.bn = t.bn;
+                r.splits = (int)sp;
+                r.mode = part ? RING_PART : fused;
+            }
+        };
+        consider(1, (tiles + 255) / 256);
+        if (tiles <= 128 && max_splits > 1 && kt >= 16 && t.bm * t.bn <= split_area) {
+            // the split that fills the CUs, and half of it
+            const uint32_t sp = std::min(most, 256u / (uint32_t)tiles);
+            if (sp > 1) {
+                consider(sp, 1);
+            }
+            if (sp > 3) {
+                consider(sp / 2, 1);
+            }
+        }
+    }
+    if (r.bm != 0) {
+        r.bk = bk;
+        r.trb = trb;
+    }
+    return r;
+}
+
+}  // namespace nnops_amd

@@ -1,0 +1,126 @@
+"""The LDS-ring GEMM at the sizes where its plan changes: every tile shape,
+ragged last tiles in both directions, the smallest row counts that take it,
+64-byte k steps, K splits, and a workspace too small for the splits.
+
+int8: bit-exact against the oracle. f16: the normalized error of one f16
+rounding (2^-11 of the value) and of an f32 sum over K <= 11008 terms in any
+order (2^-24 sqrt(K) of the rms, far below it): 2e-3, as in test_gpu_fp."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+import datagen as dg
+import nnops_amd as na
+from nnops_amd import ops
+from gpu_util import dev, host, announce, norm_err
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): the tile that the shape's plan takes
+SHAPES = [
+    (17, 704, 68),          # 64 x 64, 64-byte k steps
+    (63, 8192, 132),        # 64 x 64, K split
+    (65, 4096, 260),        # 64 x 64 split, one row past a tile
+    (500, 256, 4000),       # 128 x 64
+    (130, 4160, 1028),      # 64-byte k steps, split
+    (500, 256, 4100),       # 128 x 128, last tile 4 columns wide
+    (300, 2048, 1024),      # split over several tiles of rows
+    (384, 256, 16000),      # 192 x 128
+    (500, 128, 16100),      # 256 x 128
+    (640, 128, 11776),      # 128 x 256
+    (1000, 128, 16132),     # 256 x 256
+]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("out", ["s8", "s8_tokens", "f16"])
+def test_i8_tiles(M, K, N, trans_b, out):
+    """s8: the fused requant; s8 with a scale per row: partials and the
+    reduce; f16: the fused dequantizing output."""
+    announce(f"ring i8 {M}x{K}x{N} tb={trans_b} {out}")
+    seed = M + K + N
+    a = dg.act_s8(seed, (M, K))
+    w = dg.ints(seed + 1, (N, K), -127, 127)
+    sb = dg.uniform(seed + 2, (N,), 0.001, 0.01)
+    kind, dt = (na.OUT_F16, np.float16) if out == "f16" else (na.OUT_S8, np.int8)
+    s_a = dg.uniform(seed + 3, (M,), 0.01, 0.03) if out == "s8_tokens" else 0.02
+    bias = dg.ints(seed + 4, (N,), -5000, 5000, np.int32) if out != "f16" else None
+    c = dev(np.zeros((M, N), dt))
+    b = w if trans_b else np.ascontiguousarray(w.T)
+    na.gemm_i8(dev(a), dev(b), c, trans_b=trans_b, out_kind=kind, bias=None if bias is None else dev(bias),
+               s_a=dev(s_a) if out == "s8_tokens" else s_a, s_b=dev(sb), s_out=0.4,
+               act=na.ACT_RELU if out == "s8" else na.ACT_NONE)
+    got = host(c)
+
+    def rows(r0, r1):
+        return oracle.gemm_i8(a[r0:r1], w, trans_b=True, bias=bias,
+                              out_kind=oracle.OUT_F16 if out == "f16" else oracle.OUT_S8,
+                              s_a=s_a[r0:r1] if out == "s8_tokens" else s_a, s_b=sb, s_out=0.4,
+                              act=oracle.ACT_RELU if out == "s8" else oracle.ACT_NONE)
+    # the rows around every tile edge (a row's result depends on that row only)
+    edges = sorted({r for e in (0, 64, 128, 192, 256, 384, 512, M) for r in range(e - 2, e + 2) if 0 <= r < M})
+    for r in edges:
+        assert np.array_equal(got[r:r + 1].view(np.uint8), rows(r, r + 1).view(np.uint8)), r
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
+                                   (500, 128, 4000), (500, 128, 4100), (384, 128, 16000)])
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("out_f16", [True, False])
+def test_f16_tiles(M, K, N, trans_b, out_f16):
+    import torch
+    announce(f"ring f16 {M}x{K}x{N} tb={trans_b} f16={out_f16}")
+    a = dg.normal(M + K, (M, K)).astype(np.float16)
+    w = dg.normal(N + K, (N, K)).astype(np.float16)
+    c = torch.zeros((M, N), dtype=torch.float16 if out_f16 else torch.float32, device="cuda")
+    na.gemm_fp(dev(a), dev(w if trans_b else np.ascontiguousarray(w.T)), c, trans_b=trans_b, alpha=0.5)
+    got = host(c).astype(np.float32)
+    want = 0.5 * oracle.gemm_fp(a, w)
+    if out_f16:
+        want = want.astype(np.float16).astype(np.float32)
+    assert norm_err(got, want) <= (2e-3 if out_f16 else 2e-5)
+
+
+@pytest.mark.parametrize("M", [3, 24, 40])
+def test_f16_without_workspace(M):
+    """Calls of fewer than 64 rows need no workspace: without one they take
+    the kernels that split nothing."""
+    import torch
+    announce(f"f16 no workspace M={M}")
+    K, N = 4096, 256
+    a = dg.normal(M, (M, K)).astype(np.float16)
+    w = dg.normal(5, (N, K)).astype(np.float16)
+    da, dw = dev(a), dev(w)
+    c = torch.zeros((M, N), dtype=torch.float16, device="cuda")
+    g = na.GemmFpArgs()
+    g.a, g.b, g.c, g.m, g.n, g.k = da.data_ptr(), dw.data_ptr(), c.data_ptr(), M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b, g.in_f16, g.out_f16, g.alpha = K, K, N, 1, 1, 1, 1.0
+    assert na.lib().nnops_hip_gemm_fp_workspace_size(C.byref(g)) > 0
+    assert na.lib().nnops_hip_gemm_fp(C.byref(g), None, 0, ops._stream_ptr(None)) == na.OK
+    want = oracle.gemm_fp(a, w).astype(np.float16).astype(np.float32)
+    assert norm_err(host(c).astype(np.float32), want) <= 2e-3
+
+
+def test_i8_least_workspace():
+    """24 rows with the row and column sums' room alone (what the call took
+    before its K was split): the unsplit kernel, the same bits."""
+    import torch
+    announce("i8 least workspace")
+    M, K, N = 24, 8192, 512
+    a, w = dg.act_s8(1, (M, K)), dg.ints(2, (N, K), -127, 127)
+    c = dev(np.zeros((M, N), np.int32))
+    da, dw = dev(a), dev(w)
+    g = na.GemmI8Args()
+    g.a, g.b, g.c, g.m, g.n, g.k = da.data_ptr(), dw.data_ptr(), c.data_ptr(), M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b, g.out_kind = K, K, N, 1, na.OUT_S32
+    g.s_a_scalar = g.s_b_scalar = g.s_out = 1.0
+    least = 256 + (N * 4 + 255) // 256 * 256
+    assert na.lib().nnops_hip_gemm_i8_workspace_size(C.byref(g)) > least
+    ws = torch.empty(least, dtype=torch.uint8, device="cuda")
+    assert na.lib().nnops_hip_gemm_i8(C.byref(g), ws.data_ptr(), least, ops._stream_ptr(None)) == na.OK
+    assert np.array_equal(host(c), oracle.gemm_i8(a, w, trans_b=True))
