@@ -19,6 +19,12 @@
 #include <cstring>
 #include <limits>
 
+namespace nnops_amd {
+// q4_1.hip: the K splits of a Q4_1 product, summed by its output pass.
+int gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace, size_t ws_bytes,
+                         hipStream_t stream);
+}  // namespace nnops_amd
+
 namespace nnops {
 namespace {
 
@@ -725,11 +731,13 @@ Status run_quant(const QuantCall& q, TensorView& out, std::span<const TensorView
             x.ldb_bytes = b.pitch();
         }
         const size_t tmp = q4_1_pass_bytes(g, q);
-        const size_t need = nnops_hip_gemm_q4_1_workspace_size(&x);
-        if ((need > 0 || tmp > 0) && (workspace == nullptr || ws_bytes < tmp + align_up(need))) {
+        if (tmp > 0 && (workspace == nullptr || ws_bytes < tmp)) {
             return Status::not_initialized;
         }
-        char* gemm_ws = static_cast<char*>(workspace) + tmp;
+        // the product's own workspace is what follows (it says itself when
+        // that is too little)
+        char* gemm_ws = workspace != nullptr ? static_cast<char*>(workspace) + tmp : nullptr;
+        const size_t ws_left = workspace != nullptr ? ws_bytes - tmp : 0;
         NnopsFpOutArgs fo = fp_pass_args(q, g, out, bias, workspace);
         const int64_t a_mat = a_rows_per * a.pitch();
         const int64_t b_mat = b_rows_per * b.pitch();
@@ -741,10 +749,14 @@ Status run_quant(const QuantCall& q, TensorView& out, std::span<const TensorView
             char* cb = out.ptr<char>() + batch_offset(bi, g, g.out_batch, c_mat);
             xb.c = pass ? workspace : static_cast<void*>(cb);
             if (pass) {
-                // the output pass in the GEMM's write-back where its route
-                // takes it, else the GEMM into the workspace and the pass
+                // K splits that the output pass sums, or the pass in the
+                // GEMM's write-back, where the call's route takes them, else
+                // the GEMM into the workspace and the pass
                 fo.out = cb;
-                const int rf = nnops_hip_gemm_q4_1_fused(&xb, &fo, stream);
+                int rf = nnops_amd::gemm_q4_1_split_pass(xb, fo, gemm_ws, ws_left, stream);
+                if (rf == NNOPS_UNSUPPORTED) {
+                    rf = nnops_hip_gemm_q4_1_fused(&xb, &fo, stream);
+                }
                 if (rf == NNOPS_OK) {
                     continue;
                 }
@@ -752,7 +764,7 @@ Status run_quant(const QuantCall& q, TensorView& out, std::span<const TensorView
                     return from_code(rf);
                 }
             }
-            const int rc = nnops_hip_gemm_q4_1(&xb, gemm_ws, need, stream);
+            const int rc = nnops_hip_gemm_q4_1(&xb, gemm_ws, ws_left, stream);
             if (rc != NNOPS_OK) {
                 return from_code(rc);
             }

@@ -94,6 +94,12 @@ inline uint64_t next_launch_epoch()
 // splits; nnops_hip_gemm_i8_workspace_size is what the full plan takes).
 size_t gemm_i8_least_workspace(const NnopsGemmI8Args& g);
 
+// The Q4_1 GEMM as K splits whose partials, in the workspace, the output pass
+// sums (one launch and one staging fewer than the product and then the pass);
+// NNOPS_UNSUPPORTED, nothing launched, where another route is the call's.
+int gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace, size_t ws_bytes,
+                         hipStream_t stream);
+
 struct EpiParams {
     const int32_t* bias;       // [N] int32 (integer outputs) or nullptr
     const int32_t* r_a;        // [M] sum_k A (true values), or nullptr

@@ -24,10 +24,15 @@ struct FpOut {
     float gate_alpha, gate_beta, gate_limit;
     int mm;                     // MatMul's order: alpha P + T(beta old + bias)
     float alpha, beta;
+    int splits;                 // K splits to sum: src + s * slab, s = 0 .. splits - 1
+    int64_t slab;
 };
 
 // Checks the arguments and fills the device form (NNOPS_OK or the status).
 int make_fp_out(const NnopsFpOutArgs* a, FpOut& p);
+
+// The pass over p (its src and splits set).
+void launch_fp_out_pass(const FpOut& p, hipStream_t s);
 
 __device__ __forceinline__ float round_out(bool f16, float x)
 {

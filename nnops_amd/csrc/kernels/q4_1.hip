@@ -63,7 +63,12 @@ struct Q41Kern {
     FpOut fo;            // the fused gated combine (gemm_q4_1_ring with GATED)
     const float* row_scale;  // SPLIT ring: [M] power-of-two factor of each row of A
     int64_t plane;           // SPLIT ring: bytes from the hi plane of A to the lo plane
+    int kt_per;              // QOUT_PART ring: 64-k stages per K split (the last takes the rest)
 };
+
+// What the blocks-along-K ring writes: C in f32 or f16, or the f32 partials of
+// its K split (p.partial, [splits][M][N]).
+enum { QOUT_F32 = 0, QOUT_F16 = 1, QOUT_PART = 2 };
 
 __device__ __forceinline__ float h2f(uint32_t bits16)
 {
@@ -2468,8 +2473,8 @@ __device__ __forceinline__ v8h decode8_f16(uint32_t lo0, uint32_t lo1, v2h d2, v
 // activation -- measured slower than the separate pass: 108 against 98 us at
 // 512 x 14336 x 4096, the pass's arithmetic then running with the matrix
 // cores idle; the gated form saves the larger staging: 196 -> 184 us.)
-template <bool OUT16, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256>
-__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
+template <int OUT, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
 {
     static_assert(!GATED || (WM == 1 && WN == 8 && BM == 128 && BN == 256),
                   "gated: one wave per 32 columns, halves 4 waves apart");
@@ -2490,6 +2495,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
     if ((nb & 7) == 0) {
         bid = (bid & 7) * (nb >> 3) + (bid >> 3);     // consecutive logical tiles on one XCD
     }
+    int sp = 0;
+    if constexpr (OUT == QOUT_PART) {
+        // splits outermost: a band of one XCD shares one K range of A
+        const int tiles = tiles_m * ((p.n + BN - 1) / BN);
+        sp = bid / tiles;
+        bid -= sp * tiles;
+    }
     const int tm = bid % tiles_m, tn = bid / tiles_m; // the M tiles of a column band share B in L2
     const int m0 = tm * BM;
     const int n0 = GATED ? tn * (BN / 2) : tn * BN;   // gated: output columns; the weight has 2 p.fo.n rows
@@ -2497,20 +2509,22 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn0 = (wave % WN) * TN;
     const int wm0 = (wave / WN) * TM;
-    const int kt = p.k / 64;
+    // this split's stages of 64 k
+    const int kt0 = OUT == QOUT_PART ? sp * p.kt_per : 0;
+    const int kt = OUT == QOUT_PART && sp < p.splits - 1 ? p.kt_per : p.k / 64 - kt0;
 
     // A: rows 8 * (4 * wave + i) + lane / 8; B raw: rows 16 * (4 * wave + i) + lane / 4
-    const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda, 0x7fffffffu);
+    const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda + (int64_t)kt0 * 64, 0x7fffffffu);
     const int64_t b_bytes = (int64_t)(p.n - (GATED ? 0 : n0)) * p.ldb;
-    const QBufRsrc rsb = q_buffer_rsrc(p.b + (GATED ? 0 : (int64_t)n0 * p.ldb),
-                                       (uint32_t)std::min<int64_t>(b_bytes, 0x7fffffff));
+    const QBufRsrc rsb = q_buffer_rsrc(p.b + (GATED ? 0 : (int64_t)n0 * p.ldb) + (int64_t)kt0 * 40,
+                                       (uint32_t)std::min<int64_t>(b_bytes - (int64_t)kt0 * 40, 0x7fffffff));
     int a_off[QA], b_off[QB];
 #pragma unroll
     for (int i = 0; i < QA; ++i) {
         // SPLIT: staged rows 128..255 are the lo plane's rows 0..127
         const int ra = 8 * (QA * wave + i) + (lane >> 3);
         const int ca = (lane & 7) ^ ((ra >> 1) & 7);
-        a_off[i] = min(ra & (BM - 1), p.m - 1 - m0) * (int)p.lda * 2 + ca * 16 + (ra >= BM ? (int)p.plane : 0);
+        a_off[i] = min(SPLIT ? ra & (BM - 1) : ra, p.m - 1 - m0) * (int)p.lda * 2 + ca * 16 + (ra >= BM ? (int)p.plane : 0);
     }
 #pragma unroll
     for (int i = 0; i < QB; ++i) {
@@ -2703,7 +2717,10 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
                 if (m < p.m) {
                     // SPLIT: the row's power-of-two factor (exact)
                     const float v = SPLIT ? acc[i][j][r] * p.row_scale[m] : acc[i][j][r];
-                    if constexpr (OUT16) {
+                    if constexpr (OUT == QOUT_PART) {
+                        // read back by the pass that sums the splits
+                        p.partial[((int64_t)sp * p.m + m) * p.n + n] = v;
+                    } else if constexpr (OUT == QOUT_F16) {
                         __builtin_nontemporal_store((_Float16)v, static_cast<_Float16*>(p.c) + (int64_t)m * p.ldc + n);
                     } else {
                         __builtin_nontemporal_store(v, static_cast<float*>(p.c) + (int64_t)m * p.ldc + n);
@@ -3156,9 +3173,180 @@ inline size_t split_ws_bytes(const NnopsGemmQ41Args& g)
     return align_up((size_t)g.m * (size_t)g.k * 4) + align_up((size_t)g.m * 4);
 }
 
+// The blocks-along-K ring's conditions (f16 A; any M).
+inline bool ring_ok(const NnopsGemmQ41Args& g)
+{
+    return g.trans_b && !g.b_soa && g.a_f16 && g.k >= 64 && g.k % 64 == 0 && (g.lda % 8) == 0 &&
+           ((uintptr_t)g.a & 15) == 0;
+}
+
+// The ring's tile shapes and the time of one 64-k step of one workgroup with
+// one workgroup per CU. The 128-column tiles have 4 waves and leave room for
+// two workgroups on a CU, which then take 1.55 times one's time together.
+struct Q41RingTile {
+    int bm, bn;
+    float step_us;
+};
+constexpr Q41RingTile kQ41RingTiles[] = {
+    {32, 128, 0.39f}, {64, 128, 0.51f}, {96, 128, 0.62f}, {128, 128, 0.83f}, {64, 256, 0.82f}, {128, 256, 1.17f},
+};
+
+// The tile and K split of a call and what it is estimated to take.
+struct Q41RingPlan {
+    int bm = 0, bn = 0, splits = 1;
+    float us = 0.0f;
+};
+
+// The cheapest of the tiles and a few splits by steps x the grid's rounds on
+// the CUs, plus, with partials, 3 us and their bytes written and read at 3.5
+// TB/s. One 128 x 256 tile per column band, unsplit, had left most CUs idle
+// below 57344 outputs of a row band: K = 4096, N = 4096 took 60 us for any M
+// up to 512 (77 rows now 17 us, 512 rows 36), K = 14336 205-215 us (128 rows
+// 38, 512 rows 86). Estimates are within 10 % of those sweeps. max_splits 1:
+// no split (a workspace too small for the partials).
+inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
+{
+    Q41RingPlan r;
+    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)(g.k / 64);
+    const float out_bytes = 4.0f * (float)m * (float)n;
+    const uint32_t most = std::min({(uint32_t)max_splits, kt / 4, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)});
+    for (const Q41RingTile& t : kQ41RingTiles) {
+        const uint64_t tiles = (uint64_t)((m + t.bm - 1) / (uint32_t)t.bm) * ((n + t.bn - 1) / (uint32_t)t.bn);
+        const bool pairs = t.bn == 128;
+        auto consider = [&](uint32_t sp) {
+            const uint64_t rounds = (tiles * sp + 255) / 256;
+            const float passes = pairs ? 1.55f * (float)(rounds / 2) + (float)(rounds % 2) : (float)rounds;
+            const uint32_t steps = kt - (sp - 1) * (kt / sp);
+            const float us = passes * (float)steps * t.step_us + (sp > 1 ? 3.0f + 2.0f * (float)sp * out_bytes / 3.5e6f
+                                                                         : 0.0f);
+            if (r.bm == 0 || us < r.us) {
+                r = Q41RingPlan{t.bm, t.bn, (int)sp, us};
+            }
+        };
+        consider(1);
+        const uint32_t cap = pairs ? 512 : 256;
+        if (tiles * 2 <= cap && most > 1) {
+            const uint32_t sp = std::min(most, cap / (uint32_t)tiles);
+            consider(sp);
+            if (sp > 3) {
+                consider(sp / 2);
+            }
+        }
+    }
+    return r;
+}
+
+// bytes of a plan's partials
+inline size_t q41_ring_bytes(const NnopsGemmQ41Args& g, const Q41RingPlan& r)
+{
+    return r.splits > 1 ? align_up((size_t)r.splits * (size_t)g.m * (size_t)g.n * sizeof(float)) : 0;
+}
+
+template <int OUT>
+void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
+{
+    const int64_t tiles = (int64_t)((k.m + r.bm - 1) / r.bm) * ((k.n + r.bn - 1) / r.bn);
+    const dim3 grid((unsigned)(tiles * r.splits));
+    if (r.bn == 128) {
+        if (r.bm == 32) {
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 32, 128>), grid, dim3(256), 0, s, k);
+        } else if (r.bm == 64) {
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 64, 128>), grid, dim3(256), 0, s, k);
+        } else if (r.bm == 96) {
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 96, 128>), grid, dim3(256), 0, s, k);
+        } else {
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 1, 4, false, false, 128, 128>), grid, dim3(256), 0, s, k);
+        }
+    } else if (r.bm == 64) {
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8, false, false, 64, 256>), grid, dim3(512), 0, s, k);
+    } else {
+        // 8 waves (2 per SIMD), each 128 x 32: one wave's decode and stalls
+        // overlap the other's matrix-core work, and no B row is decoded twice
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8>), grid, dim3(512), 0, s, k);
+    }
+}
+
+// Whether the ring may split K: past the skinny kernel's rows, or where its K
+// condition rules that kernel out. (The skinny kernel streams the weight once
+// per 16 rows: 24 rows at K = 4096, N = 14336 take it 30 us, the ring 22; it
+// keeps 17 to 48 rows where the splits have no workspace.)
+inline bool ring_splits(const NnopsGemmQ41Args& g)
+{
+    return ring_ok(g) && (g.m > 16 || (g.m > 2 && g.k % 256 != 0));
+}
+
+// The kernel arguments of a checked call.
+inline Q41Kern q41_kern(const NnopsGemmQ41Args& g)
+{
+    Q41Kern k{};
+    k.a = g.a;
+    k.b = g.b;
+    k.c = g.c;
+    k.m = (int)g.m;
+    k.n = (int)g.n;
+    k.k = (int)g.k;
+    k.lda = g.lda;
+    k.ldc = g.ldc;
+    k.ldb = g.ldb_bytes;
+    k.out_f16 = g.out_kind == NNOPS_OUT_F16;
+    k.bdm = g.b_soa ? g.b_dm : nullptr;
+    k.ldbdm = g.b_soa ? g.ldb_dm : 0;
+    return k;
+}
+
+// The plan's partials, then the pass over their sum.
+inline void run_q41_split(const NnopsGemmQ41Args& g, const Q41RingPlan& r, FpOut& fo, void* ws, hipStream_t s)
+{
+    Q41Kern k = q41_kern(g);
+    k.partial = static_cast<float*>(ws);
+    k.splits = r.splits;
+    k.kt_per = (k.k / 64) / r.splits;
+    launch_q41_ring<QOUT_PART>(k, r, s);
+    fo.src = k.partial;
+    fo.ld_src = k.n;
+    fo.splits = r.splits;
+    fo.slab = (int64_t)k.m * k.n;
+    launch_fp_out_pass(fo, s);
+}
+
+// the pass that only sums and stores
+inline FpOut q41_store_pass(const NnopsGemmQ41Args& g)
+{
+    FpOut fo{};
+    fo.out = g.c;
+    fo.ld_out = g.ldc;
+    fo.rows = g.m;
+    fo.n = (int)g.n;
+    fo.out_f16 = g.out_kind == NNOPS_OUT_F16;
+    fo.ep.min_clip = -INFINITY;
+    fo.ep.max_clip = INFINITY;
+    fo.ep.out_kind = fo.out_f16 ? NNOPS_OUT_F16 : NNOPS_OUT_F32;
+    return fo;
+}
+
 // the prepacked planes' block-column pitches: nibbles in bytes, d|m in dwords
 inline int64_t prepack_q41_nib_pitch(int64_t k) { return (k + 7) / 8 * 128; }
 inline int64_t prepack_q41_dm_pitch(int64_t k) { return (k + 63) / 64 * 64; }
+
+// What a call cannot run without (the ring's K splits can: they are what
+// nnops_hip_gemm_q4_1_workspace_size adds).
+inline size_t least_workspace(const NnopsGemmQ41Args& g)
+{
+    if (split_ok(g)) {
+        return split_ws_bytes(g);
+    }
+    if (g.trans_b || !use_gemv(g) || bcm_ok(g)) {
+        return 0;
+    }
+    // pointer alignment, which a size query may not see, picks between the
+    // two blocks-along-N GEMVs: room for either
+    const size_t split_bytes = align_up((size_t)kn_splits(g) * (size_t)g.m * (size_t)g.n * sizeof(float));
+    const KnDmaPlan kd = plan_kn_dma(g);
+    if (kd.groups > 0) {
+        return std::max(split_bytes, align_up(kn_dma_part_bytes(kd)) + align_up((size_t)kd.groups * kd.splits * 8));
+    }
+    return split_bytes;
+}
 
 }  // namespace
 }  // namespace nnops_amd
@@ -3167,20 +3355,13 @@ using namespace nnops_amd;
 
 extern "C" size_t nnops_hip_gemm_q4_1_workspace_size(const NnopsGemmQ41Args* g)
 {
-    if (g != nullptr && split_ok(*g)) {
-        return split_ws_bytes(*g);
-    }
-    if (g == nullptr || g->trans_b || !use_gemv(*g) || bcm_ok(*g)) {
+    if (g == nullptr) {
         return 0;
     }
-    // pointer alignment, which a size query may not see, picks between the
-    // two blocks-along-N GEMVs: room for either
-    const size_t split_bytes = align_up((size_t)kn_splits(*g) * (size_t)g->m * (size_t)g->n * sizeof(float));
-    const KnDmaPlan kd = plan_kn_dma(*g);
-    if (kd.groups > 0) {
-        return std::max(split_bytes, align_up(kn_dma_part_bytes(kd)) + align_up((size_t)kd.groups * kd.splits * 8));
+    if (ring_splits(*g) && g->n > 0 && g->m <= INT32_MAX && g->n <= INT32_MAX && g->k <= INT32_MAX) {
+        return q41_ring_bytes(*g, plan_q41_ring(*g, 16));
     }
-    return split_bytes;
+    return least_workspace(*g);
 }
 
 extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, size_t ws_bytes, void* stream)
@@ -3213,27 +3394,31 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
                      g->ldb_dm != prepack_q41_dm_pitch(g->k))) {
         return NNOPS_INVALID_ARGUMENT;
     }
-    const size_t need = nnops_hip_gemm_q4_1_workspace_size(g);
+    const size_t need = least_workspace(*g);
     if (need > 0 && (workspace == nullptr || ws_bytes < need)) {
         return NNOPS_NOT_INITIALIZED;
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    Q41Kern k{};
-    k.a = g->a;
-    k.b = g->b;
-    k.c = g->c;
-    k.m = (int)g->m;
-    k.n = (int)g->n;
-    k.k = (int)g->k;
-    k.lda = g->lda;
-    k.ldc = g->ldc;
-    k.ldb = g->ldb_bytes;
-    k.out_f16 = g->out_kind == NNOPS_OUT_F16;
-    k.bdm = g->b_soa ? g->b_dm : nullptr;
-    k.ldbdm = g->b_soa ? g->ldb_dm : 0;
+    if (workspace == nullptr || ((uintptr_t)workspace & 15) != 0) {
+        ws_bytes = 0;            // (below: room for the ring's partials, 16-byte vectors)
+    }
+    // the ring's plan: its K splits, or without room for them no split
+    Q41RingPlan ring;
+    bool starved = !ring_splits(*g);
+    if (ring_ok(*g) && g->m > 2) {
+        ring = plan_q41_ring(*g, starved ? 1 : 16);
+        if (q41_ring_bytes(*g, ring) > ws_bytes) {
+            ring = plan_q41_ring(*g, 1);
+            starved = true;
+        }
+    }
+    const Q41Kern k = q41_kern(*g);
     const bool soa = g->b_soa != 0;
 
-    if (skinny_ok(*g)) {
+    if (ring.splits > 1) {
+        FpOut fo = q41_store_pass(*g);
+        run_q41_split(*g, ring, fo, workspace, s);
+    } else if (skinny_ok(*g) && starved) {
         // a few rows of A: the weight streams once per 16 rows
         for (int m0 = 0; m0 < k.m; m0 += 16) {
             Q41Kern kk = k;
@@ -3396,9 +3581,9 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
         kk.row_scale = rs;
         const unsigned tiles = (unsigned)(((g->m + 127) / 128) * ((g->n + 255) / 256));
         if (g->trans_b && k.out_f16) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<true, 3, 1, 8, false, true>), dim3(tiles), dim3(512), 0, s, kk);
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F16, 3, 1, 8, false, true>), dim3(tiles), dim3(512), 0, s, kk);
         } else if (g->trans_b) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<false, 3, 1, 8, false, true>), dim3(tiles), dim3(512), 0, s, kk);
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 3, 1, 8, false, true>), dim3(tiles), dim3(512), 0, s, kk);
         } else if (soa && k.out_f16) {
             NNOPS_LAUNCH((gemm_q4_1_kn_ring<true, 3, true, true>), dim3(tiles), dim3(512), 0, s, kk);
         } else if (soa) {
@@ -3417,15 +3602,12 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
         } else {
             NNOPS_LAUNCH(gemm_q4_1_f32<1>, dim3(tiles), dim3(256), 0, s, k);
         }
-    } else if (g->trans_b && g->k % 64 == 0 && (g->lda % 8) == 0 && ((uintptr_t)g->a & 15) == 0) {
+    } else if (ring.bm > 0) {
         // blocks along K: the ring kernel (A by DMA, B decoded in registers)
-        const unsigned tiles = (unsigned)(((g->m + 127) / 128) * ((g->n + 255) / 256));
-        // 8 waves (2 per SIMD), each 128 x 32: one wave's decode and stalls
-        // overlap the other's matrix-core work, and no B row is decoded twice
         if (k.out_f16) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<true, 4, 1, 8>), dim3(tiles), dim3(512), 0, s, k);
+            launch_q41_ring<QOUT_F16>(k, ring, s);
         } else {
-            NNOPS_LAUNCH((gemm_q4_1_ring<false, 4, 1, 8>), dim3(tiles), dim3(512), 0, s, k);
+            launch_q41_ring<QOUT_F32>(k, ring, s);
         }
     } else if (kn_ring_ok(*g)) {
         // blocks along N: the same ring, B rows staged raw and decoded per lane
@@ -3451,6 +3633,43 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
             NNOPS_LAUNCH((gemm_q4_1_mfma<128, 128, 2, 2, false>), dim3(tiles), dim3(256), 0, s, k);
         }
     }
+    return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
+}
+
+int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace,
+                                    size_t ws_bytes, hipStream_t stream)
+{
+    const TimingDisarm disarm;
+    if (!ring_splits(g) || g.n <= 0 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX ||
+        g.a == nullptr || g.b == nullptr || g.lda < g.k || g.ldb_bytes < g.k / 32 * 20 || (g.ldb_bytes & 3) ||
+        ((uintptr_t)g.b & 3) || workspace == nullptr || ((uintptr_t)workspace & 15) != 0 || pass.src == nullptr) {
+        return NNOPS_UNSUPPORTED;
+    }
+    const Q41RingPlan r = plan_q41_ring(g, 16);
+    if ((r.splits == 1 && !pass.gated) || q41_ring_bytes(g, r) > ws_bytes) {
+        return NNOPS_UNSUPPORTED;
+    }
+    // the gated form's fused tiles (128 rows x 2 x 128 weight rows, one
+    // workgroup per CU, the combine some 10 us) where they are the faster
+    if (pass.gated) {
+        const int64_t tiles = ((g.m + 127) / 128) * ((pass.n + 127) / 128);
+        const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
+        if ((float)((tiles + 255) / 256) * (float)(g.k / 64) * 1.17f + 10.0f <= r.us + staged) {
+            return NNOPS_UNSUPPORTED;
+        }
+    }
+    FpOut fo;
+    if (const int rc = make_fp_out(&pass, fo); rc != NNOPS_OK) {
+        return rc;
+    }
+    if (pass.rows != g.m || pass.n * (pass.gated ? 2 : 1) != g.n) {
+        return NNOPS_INVALID_ARGUMENT;
+    }
+    if ((pass.n + 1023) / 1024 * pass.rows > INT32_MAX) {
+        return NNOPS_UNSUPPORTED;
+    }
+    // an unsplit product (gated) goes where the caller's pass reads it
+    run_q41_split(g, r, fo, r.splits > 1 ? workspace : const_cast<float*>(pass.src), stream);
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }
 
@@ -3520,7 +3739,7 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
     }
     const int64_t tiles_m = (g->m + 127) / 128;
     const unsigned tiles = (unsigned)(tiles_m * ((pass->n + 127) / 128));
-    NNOPS_LAUNCH((gemm_q4_1_ring<false, 4, 1, 8, true>), dim3(tiles), dim3(512), 0, s, k);
+    NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true>), dim3(tiles), dim3(512), 0, s, k);
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }
 

@@ -1,0 +1,103 @@
+"""The blocks-along-K Q4_1 ring at the sizes where its plan changes: every
+tile shape with ragged edges, K splits whose last one is longer, row counts
+just past the skinny kernel, the output pass over the splits' partials (plain
+and gated), and calls without a workspace.
+
+Bar: the Q4_1 tolerance (2e-3, normalized), against the oracle with weights
+decoded to f16 (the decode's rounding, 2^-12 of a weight, is in both; an f32
+sum of K <= 14336 terms in any order adds 2^-24 sqrt(K) of the rms and an f16
+destination one rounding, 2^-11 of the value)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+import datagen as dg
+import nnops_amd as na
+from nnops_amd import ops
+from gpu_util import dev, host, announce, norm_err, oracle_rows
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-3
+
+# (M, K, N): the tile and split that the plan takes
+SHAPES = [
+    (3, 320, 100),          # fewer rows than a tile, K % 256 != 0
+    (17, 256, 130),         # 32 x 128, unsplit (4 stages of k)
+    (31, 4160, 1025),       # 32 x 128, 65 stages over the splits
+    (33, 4096, 260),        # 64 x 128, split
+    (77, 4096, 1024),       # 96 x 128, split
+    (97, 1088, 516),        # 17 stages, two tiles of rows
+    (128, 14336, 256),
+    (130, 512, 8192),       # 64 x 256
+    (300, 4096, 300),
+    (260, 256, 28700),      # 128 x 256
+]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("out_f16", [True, False])
+def test_q4_1_ring_tiles(M, K, N, out_f16):
+    import torch
+    announce(f"q4_1 ring {M}x{K}x{N} f16={out_f16}")
+    x = dg.normal(M + K, (M, K)).astype(np.float16)
+    blk = dg.q4_1_blocks(N + K, N, K)
+    c = torch.full((M, N + 8), 7.0, dtype=torch.float16 if out_f16 else torch.float32, device="cuda")
+    na.gemm_q4_1(dev(x), dev(blk), c[:, :N], n=N, trans_b=True)
+    got = host(c).astype(np.float32)
+    assert (got[:, N:] == 7.0).all()
+    want = oracle_rows(lambda r0, r1: oracle.gemm_q4_1(x, blk, N, trans_b=True, rows=(r0, r1),
+                                                       w_round_f16=True)[r0:r1], M, band=4)
+    assert norm_err(got[:, :N], want) <= TOL
+
+
+@pytest.mark.parametrize("M,K,N2", [(17, 4096, 520), (40, 4096, 2050), (128, 2048, 1032), (200, 4096, 516)])
+@pytest.mark.parametrize("kw", [dict(gated=True), dict(gated=True, add_to=True), dict(act=na.EP_RELU),
+                                dict(add_to=True, residual_pre_activation=True)])
+@pytest.mark.parametrize("f16", [True, False])
+def test_q4_1_ring_split_pass(M, K, N2, kw, f16):
+    """Linear with a bias: the splits' partials through the output pass (an
+    f32 X takes its own route to the same pass)."""
+    import torch
+    announce(f"q4_1 split pass {M}x{K}x{N2} {kw} f16={f16}")
+    dt = np.float16 if f16 else np.float32
+    gated = kw.get("gated", False)
+    n = N2 // 2 if gated else N2
+    x = dg.normal(M, (M, K)).astype(dt)
+    blk = dg.q4_1_blocks(N2 + 3, N2, K)
+    bias = (0.1 * dg.normal(N2, (N2,))).astype(dt)
+    old = dg.normal(4, (M, n)).astype(dt)
+    y = dev(old)
+    op = na.Linear(gate_activation=na.EP_SILU, output_dtype=na.DT_F16 if f16 else na.DT_F32, **kw)
+    rc = op.compute([na.tensor(y)], [na.tensor(dev(x)), na.tensor(dev(blk), dtype=na.DT_Q4_1, shape=[N2, K]),
+                                     na.tensor(dev(bias))])
+    assert rc == na.OK
+    torch.cuda.synchronize()
+    want = oracle_rows(lambda r0, r1: oracle.q4_1_linear(
+        x, blk, N2, rows=(r0, r1), w_round_f16=f16 or M > 48, gated=gated, out_f16=f16, bias=bias,
+        out=old if kw.get("add_to") else None, gate_act=oracle.ACT_SILU,
+        act=oracle.ACT_RELU if kw.get("act") else oracle.ACT_NONE, add_to=kw.get("add_to", False),
+        residual_pre=kw.get("residual_pre_activation", False)), M, band=4).astype(np.float32)
+    assert norm_err(host(y).astype(np.float32), want) <= TOL
+
+
+@pytest.mark.parametrize("M", [3, 24, 100])
+def test_q4_1_ring_without_workspace(M):
+    """No workspace (none was needed before K was split): the unsplit kernels."""
+    import torch
+    announce(f"q4_1 no workspace M={M}")
+    K, N = 4096, 384
+    x = dg.normal(M, (M, K)).astype(np.float16)
+    blk = dg.q4_1_blocks(11, N, K)
+    dx, db = dev(x), dev(blk)
+    c = torch.zeros((M, N), dtype=torch.float16, device="cuda")
+    g = na.GemmQ41Args()
+    g.a, g.b, g.c, g.m, g.n, g.k = dx.data_ptr(), db.data_ptr(), c.data_ptr(), M, N, K
+    g.lda, g.ldc, g.ldb_bytes, g.trans_b, g.a_f16, g.out_kind = K, N, db.stride(0), 1, 1, na.OUT_F16
+    assert na.lib().nnops_hip_gemm_q4_1(C.byref(g), None, 0, ops._stream_ptr(None)) == na.OK
+    want = oracle.gemm_q4_1(x, blk, N, trans_b=True, w_round_f16=True)
+    assert norm_err(host(c).astype(np.float32), want) <= TOL
