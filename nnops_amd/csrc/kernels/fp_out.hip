@@ -11,6 +11,8 @@
 //                 bytes, twice the source columns when gated).
 #include "fp_out.hpp"
 
+#include <cmath>
+
 namespace nnops_amd {
 namespace {
 
@@ -105,9 +107,15 @@ __global__ __launch_bounds__(256) void fp_out_pass(FpOut p, int cblocks)
         }
     }
     float y[4];
+    if (p.silu) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            y[e] = fp_out_silu(p, a[e], v[e], bg[e], bu[e]);
+        }
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        if (e < cn) {
+        if (e < cn && !p.silu) {
             y[e] = fp_out_value(p, a[e], v[e], old[e], bg[e], bu[e]);
         }
     }
@@ -174,6 +182,8 @@ int make_fp_out(const NnopsFpOutArgs* a, FpOut& p)
     p.mm = a->matmul_order != 0;
     p.alpha = a->alpha;
     p.beta = a->beta;
+    p.silu = p.gated && p.gate_act == NNOPS_ACT_SILU && std::isinf(p.gate_limit) && p.ep.act == NNOPS_ACT_NONE &&
+             p.ep.min_clip == -INFINITY && p.ep.max_clip == INFINITY && !p.add_to;
     return NNOPS_OK;
 }
 

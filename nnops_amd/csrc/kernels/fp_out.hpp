@@ -24,6 +24,7 @@ struct FpOut {
     float gate_alpha, gate_beta, gate_limit;
     int mm;                     // MatMul's order: alpha P + T(beta old + bias)
     float alpha, beta;
+    int silu;                   // gated, plain SwiGLU: Silu gate, no limit, activation, clip or residual
     int splits;                 // K splits to sum: src + s * slab, s = 0 .. splits - 1
     int64_t slab;
 };
@@ -130,6 +131,16 @@ __device__ __forceinline__ float fp_out_value(const FpOut& p, float a, float v, 
         }
     }
     return y;
+}
+
+// fp_out_value of a plain SwiGLU (p.silu): its operations, without its branches.
+__device__ __forceinline__ float fp_out_silu(const FpOut& p, float a, float v, float bg, float bu)
+{
+    const bool f16 = p.out_f16 != 0;
+    const float g = round_out(f16, __fadd_rn(a, bg));
+    const float u = round_out(f16, __fadd_rn(v, bu));
+    const float s = __fdiv_rn(g, __fadd_rn(1.0f, expf(__fmul_rn(-p.gate_alpha, g))));
+    return __fmul_rn(s, __fadd_rn(u, p.gate_beta));
 }
 
 __device__ __forceinline__ void fp_out_store(const FpOut& p, char* orow, int c, float y)

@@ -2432,12 +2432,13 @@ __global__ __launch_bounds__(256) void split_a_f32(const float* a, int64_t lda, 
 
 // ---------------------------------------------------------------------------
 // MFMA GEMM, f16 A, B blocks along K ([N][K/32], 2 blocks = 40 bytes per row
-// per 64-k stage), K % 64 == 0. 128 x 256 tiles, WM x WN waves (the launch
-// uses 1 x 8: each wave 128 x 32, two per SIMD) of 32x32 fragments
+// per 64-k stage), K % 64 == 0. BM x BN tiles, WM x WN waves (128 x 256 tiles:
+// 1 x 8, each wave 128 x 32, two per SIMD; 256 x 256: 2 x 4 of 128 x 64; tiles
+// of 128 columns: 1 x 4) of 32x32 fragments
 // (v_mfma_f32_32x32x16_f16), an NS-stage LDS ring filled only by
 // buffer_load ... lds (so every wait below is an explicit vmcnt):
-//   A     128 rows x 128 bytes; 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7)
-//   Braw  256 rows x 64 bytes (the row's 40 stage bytes + 24 not used); chunk
+//   A     BM rows x 128 bytes; 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7)
+//   Braw  BN rows x 64 bytes (the row's 40 stage bytes + 24 not used); chunk
 //         c of row r in slot c ^ ((r >> 2) & 3)
 // Both swizzles make the 16- and 4-byte fragment reads of 32 consecutive rows
 // conflict-free (A) or at most 2-way (Braw). Each lane decodes its own B
@@ -2465,19 +2466,22 @@ __device__ __forceinline__ v8h decode8_f16(uint32_t lo0, uint32_t lo1, v2h d2, v
     return __builtin_bit_cast(v8h, v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]});
 }
 
+// OUT: what is written (QOUT_PART: this K split's f32 partials, whole 128-byte
+// lines per half wave; launch_q41_ring's plan says when).
 // GATED: Linear's gated form with its output pass p.fo fused: the tile covers
 // output columns 128 tn .. + 127 and stages the weight's gate rows there and
-// its value rows (N / 2 further) in its second half, so waves 0-3 hold the
-// gate products and waves 4-7 the value products of the same columns, which
-// meet through LDS for the combine. (Fusing the plain pass -- bias, residual,
-// activation -- measured slower than the separate pass: 108 against 98 us at
-// 512 x 14336 x 4096, the pass's arithmetic then running with the matrix
-// cores idle; the gated form saves the larger staging: 196 -> 184 us.)
+// its value rows (N / 2 further) in its second half, so the lower half of the
+// waves holds the gate products and the upper half the value products of the
+// same columns, which meet through LDS for the combine. (Fusing the plain
+// pass -- bias, residual, activation -- measured slower than the separate
+// pass: 108 against 98 us at 512 x 14336 x 4096, the pass's arithmetic then
+// running with the matrix cores idle; the gated form saves the larger
+// staging.) 512 x 2 x 14336 x 4096: 173 us on 128-row tiles with a branching
+// combine, 161 with the straight-line one, 139 on 256-row tiles.
 template <int OUT, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
 {
-    static_assert(!GATED || (WM == 1 && WN == 8 && BM == 128 && BN == 256),
-                  "gated: one wave per 32 columns, halves 4 waves apart");
+    static_assert(!GATED || (BN == 256 && WN % 2 == 0), "gated: 128 gate and 128 value rows of the weight per tile");
     static_assert(!SPLIT || (!GATED && WM == 1), "split A: one wave row");
     constexpr int W = WM * WN;                      // waves: WM along M x WN along N
     constexpr int AP = SPLIT ? 2 : 1;               // planes of A (SPLIT: hi and lo f16 parts)
@@ -2663,42 +2667,71 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
     }
 
     // C[m][n]: lane holds column n = (lane & 31) of fragment j, rows 8 (r / 4) + 4 (lane >> 5) + r % 4
-    // The gated combine. The pass is too large to inline once per register
-    // (a call would put its parameters on the stack), so the products go
-    // through the ring (free once every wave is past it) and a loop of a few
-    // rows per step applies it: xs[wave][i * 16 + r][lane] is product row
-    // 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4 of the wave's column lane % 32.
-    // Gate wave w (0-3) and value wave w + 4 hold the two products of the
-    // same outputs; the gate wave combines rows 0-63, the value wave 64-127.
+    // The gated combine. The products go through the ring (free once every
+    // wave is past it), one 32-column fragment of the wave tiles at a time:
+    // xs[wave][i * 16 + r][lane] is product row 32 i + 8 (r / 4) + 4 (lane /
+    // 32) + r % 4 of the wave's column lane % 32. A gate wave and the value
+    // wave of the same columns, WN / 2 further, hold the two products of the
+    // same outputs; the gate wave combines the upper half of their rows, the
+    // value wave the lower. The general pass is too large to inline once per
+    // register (a call would put its parameters on the stack): a loop of a
+    // few rows per step applies it. The plain SwiGLU (host-known: fo.silu)
+    // is straight-line code, 8 rows at a time so that their LDS reads and
+    // exponentials overlap; the same operations, so the same bits.
     if constexpr (GATED) {
-        static_assert(W * FM * 16 * 64 * 4 <= NS * kStage, "the products fit the ring");
+        static_assert(W * FM * 16 * 64 * 4 <= NS * kStage, "the products of one column fragment fit the ring");
         const FpOut fo = p.fo;
-        __syncthreads();
         float* xs = reinterpret_cast<float*>(ring);
+        constexpr int WH = WN / 2;
+        const int wni = wave % WN;
+        const int gw = wave - (wni >= WH ? WH : 0);             // the pair's gate wave
+        const float* xg = xs + (gw * FM) * 1024 + lane;
+        const float* xv = xs + ((gw + WH) * FM) * 1024 + lane;
+        const int first = wni >= WH ? FM * 8 : 0;
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
+        for (int j = 0; j < FN; ++j) {
+            __syncthreads();
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                xs[((wave * FM + i) * 16 + r) * 64 + lane] = acc[i][0][r];
+            for (int i = 0; i < FM; ++i) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    xs[((wave * FM + i) * 16 + r) * 64 + lane] = acc[i][j][r];
+                }
             }
-        }
-        __syncthreads();
-        const int gw = wave & 3;
-        const int n = n0 + gw * 32 + (lane & 31);
-        if (n >= fo.n) {
-            return;
-        }
-        const float bg = bias_at(fo, n), bu = bias_at(fo, fo.n + n);
-        const int first = wave >= 4 ? FM * 8 : 0;
+            const int n = n0 + (wni % WH) * TN + j * 32 + (lane & 31);
+            const bool live = n < fo.n;
+            const float bg = live ? bias_at(fo, n) : 0.0f, bu = live ? bias_at(fo, fo.n + n) : 0.0f;
+            __syncthreads();
+            if (fo.silu) {
+#pragma unroll 1
+                for (int q = 0; q < FM * 8; q += 8) {
+                    float y[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int ir = first + q + e;
+                        y[e] = fp_out_silu(fo, xg[ir * 64], xv[ir * 64], bg, bu);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int ir = first + q + e, i = ir >> 4, r = ir & 15;
+                        const int m = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                        if (live && m < p.m) {
+                            fp_out_store(fo, static_cast<char*>(fo.out) + (int64_t)m * fo.ld_out * (fo.out_f16 ? 2 : 4),
+                                         n, y[e]);
+                        }
+                    }
+                }
+            } else {
 #pragma unroll 4
-        for (int q = 0; q < FM * 8; ++q) {
-            const int ir = first + q, i = ir >> 4, r = ir & 15;
-            const int m = m0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (m < p.m) {
-                char* orow = static_cast<char*>(fo.out) + (int64_t)m * fo.ld_out * (fo.out_f16 ? 2 : 4);
-                const float g = xs[((gw * FM) * 16 + ir) * 64 + lane];
-                const float v = xs[(((gw + 4) * FM) * 16 + ir) * 64 + lane];
-                fp_out_store(fo, orow, n, fp_out_value(fo, g, v, fp_out_old(fo, orow, n), bg, bu));
+                for (int q = 0; q < FM * 8; ++q) {
+                    const int ir = first + q, i = ir >> 4, r = ir & 15;
+                    const int m = m0 + wm0 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    if (live && m < p.m) {
+                        char* orow = static_cast<char*>(fo.out) + (int64_t)m * fo.ld_out * (fo.out_f16 ? 2 : 4);
+                        fp_out_store(fo, orow, n,
+                                     fp_out_value(fo, xg[ir * 64], xv[ir * 64], fp_out_old(fo, orow, n), bg, bu));
+                    }
+                }
             }
         }
         return;
@@ -3181,7 +3214,9 @@ inline bool ring_ok(const NnopsGemmQ41Args& g)
 }
 
 // The ring's tile shapes and the time of one 64-k step of one workgroup with
-// one workgroup per CU. The 128-column tiles have 4 waves and leave room for
+// one workgroup per CU. (256 x 256: each decoded weight fragment feeds 128 rows
+// as in the 128-row tiles, but each row of A is read from LDS by 4 waves in
+// place of 8: 1024 x 4096 x 14336 154 -> 129 us.) The 128-column tiles have 4 waves and leave room for
 // two workgroups on a CU, which then take 1.55 times one's time together.
 struct Q41RingTile {
     int bm, bn;
@@ -3189,6 +3224,7 @@ struct Q41RingTile {
 };
 constexpr Q41RingTile kQ41RingTiles[] = {
     {32, 128, 0.39f}, {64, 128, 0.51f}, {96, 128, 0.62f}, {128, 128, 0.83f}, {64, 256, 0.82f}, {128, 256, 1.17f},
+    {256, 256, 1.95f},
 };
 
 // The tile and K split of a call and what it is estimated to take.
@@ -3236,6 +3272,22 @@ inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
     return r;
 }
 
+// The fused gated tiles' time: 128 or 256 rows x 128 outputs, one workgroup per
+// CU, and the combine. At 2 x 14336 x 4096 the tall tiles take 512 rows in one
+// round (139 us, 161 in the 128-row tiles' two), 256 rows or fewer the low
+// ones (85 against 113 us).
+inline float gated_us(const NnopsGemmQ41Args& g, int bm)
+{
+    const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n / 2 + 127) / 128);
+    const float steps = (float)(g.k / 64);
+    return (float)((tiles + 255) / 256) * (bm == 256 ? steps * 1.95f + 14.0f : steps * 1.17f + 6.0f);
+}
+
+inline bool gated_tall(const NnopsGemmQ41Args& g)
+{
+    return gated_us(g, 256) < gated_us(g, 128);
+}
+
 // bytes of a plan's partials
 inline size_t q41_ring_bytes(const NnopsGemmQ41Args& g, const Q41RingPlan& r)
 {
@@ -3259,6 +3311,8 @@ void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
         }
     } else if (r.bm == 64) {
         NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8, false, false, 64, 256>), grid, dim3(512), 0, s, k);
+    } else if (r.bm == 256) {
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 2, 4, false, false, 256, 256>), grid, dim3(512), 0, s, k);
     } else {
         // 8 waves (2 per SIMD), each 128 x 32: one wave's decode and stalls
         // overlap the other's matrix-core work, and no B row is decoded twice
@@ -3649,12 +3703,10 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
     if ((r.splits == 1 && !pass.gated) || q41_ring_bytes(g, r) > ws_bytes) {
         return NNOPS_UNSUPPORTED;
     }
-    // the gated form's fused tiles (128 rows x 2 x 128 weight rows, one
-    // workgroup per CU, the combine some 10 us) where they are the faster
+    // the gated form's fused tiles where they are the faster
     if (pass.gated) {
-        const int64_t tiles = ((g.m + 127) / 128) * ((pass.n + 127) / 128);
         const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
-        if ((float)((tiles + 255) / 256) * (float)(g.k / 64) * 1.17f + 10.0f <= r.us + staged) {
+        if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
             return NNOPS_UNSUPPORTED;
         }
     }
@@ -3737,9 +3789,13 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
         }
         return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
     }
-    const int64_t tiles_m = (g->m + 127) / 128;
-    const unsigned tiles = (unsigned)(tiles_m * ((pass->n + 127) / 128));
-    NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true>), dim3(tiles), dim3(512), 0, s, k);
+    if (gated_tall(*g)) {
+        const unsigned tiles = (unsigned)(((g->m + 255) / 256) * ((pass->n + 127) / 128));
+        NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 3, 2, 4, true, false, 256, 256>), dim3(tiles), dim3(512), 0, s, k);
+    } else {
+        const unsigned tiles = (unsigned)(((g->m + 127) / 128) * ((pass->n + 127) / 128));
+        NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true>), dim3(tiles), dim3(512), 0, s, k);
+    }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }
 

@@ -101,3 +101,39 @@ def test_q4_1_ring_without_workspace(M):
     assert na.lib().nnops_hip_gemm_q4_1(C.byref(g), None, 0, ops._stream_ptr(None)) == na.OK
     want = oracle.gemm_q4_1(x, blk, N, trans_b=True, w_round_f16=True)
     assert norm_err(host(c).astype(np.float32), want) <= TOL
+
+
+@pytest.mark.parametrize("M,K,n", [(300, 256, 14336), (512, 64, 16200)])
+@pytest.mark.parametrize("kw", [dict(), dict(gate_limit=1.5), dict(add_to=True)])
+@pytest.mark.parametrize("f16", [True, False])
+def test_q4_1_gated_tall_tiles(M, K, n, kw, f16):
+    """The fused gated form on its 256-row tiles (ragged rows and columns, the
+    plain SwiGLU and the general combine), bit for bit the product and then
+    the pass."""
+    import torch
+    announce(f"q4_1 gated tall {M}x{K}x{n} {kw} f16={f16}")
+    x, blk = dev(dg.normal(M, (M, K)).astype(np.float16)), dev(dg.q4_1_blocks(n, 2 * n, K))
+    tdt = torch.float16 if f16 else torch.float32
+    bias = (0.1 * torch.randn(2 * n, device="cuda")).to(tdt)
+    old = torch.randn((M, n), device="cuda").to(tdt)
+    prod = torch.zeros((M, 2 * n), dtype=torch.float32, device="cuda")
+    lib, st = na.lib(), ops._stream_ptr(None)
+    g = na.GemmQ41Args()
+    g.a, g.b, g.c, g.m, g.n, g.k = x.data_ptr(), blk.data_ptr(), prod.data_ptr(), M, 2 * n, K
+    g.lda, g.ldc, g.ldb_bytes, g.trans_b, g.a_f16, g.out_kind = K, 2 * n, blk.stride(0), 1, 1, na.OUT_F32
+    outs = []
+    for fused in (True, False):
+        y = old.clone()
+        p = na._lib.FpOutArgs()
+        p.src, p.ld_src, p.out, p.ld_out, p.rows, p.n = prod.data_ptr(), 2 * n, y.data_ptr(), n, M, n
+        p.out_f16, p.bias, p.gated, p.gate_act, p.gate_alpha = int(f16), bias.data_ptr(), 1, na.ACT_SILU, 1.0
+        p.min_clip, p.max_clip, p.act_beta = -np.inf, np.inf, 1.0
+        p.gate_limit, p.add_to = kw.get("gate_limit", np.inf), int(kw.get("add_to", False))
+        if fused:
+            assert lib.nnops_hip_gemm_q4_1_fused(C.byref(g), C.byref(p), st) == na.OK
+        else:
+            # unsplit (no workspace): the fused tiles sum K in the same order
+            assert lib.nnops_hip_gemm_q4_1(C.byref(g), None, 0, st) == na.OK
+            assert lib.nnops_hip_fp_output_pass(C.byref(p), st) == na.OK
+        outs.append(host(y))
+    assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))
