@@ -63,7 +63,8 @@ struct Q41Kern {
     FpOut fo;            // the fused gated combine (gemm_q4_1_ring with GATED)
     const float* row_scale;  // SPLIT ring: [M] power-of-two factor of each row of A
     int64_t plane;           // SPLIT ring: bytes from the hi plane of A to the lo plane
-    int kt_per;              // QOUT_PART ring: 64-k stages per K split (the last takes the rest)
+    int kt_per;              // K splits of the ring (64-k stages) and the skinny kernel (stages per part) each;
+                             // the last takes the rest
 };
 
 // What the blocks-along-K ring writes: C in f32 or f16, or the f32 partials of
@@ -876,6 +877,160 @@ __global__ __launch_bounds__(256) void gemv_q4_1_pipe(Q41Kern p)
                     store_out(p, m, n0 + r, acc[r][m]);
                 }
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// GEMV, blocks along K, K > 4096 (129 to 512 blocks, a multiple of 4), M <= 2:
+// the pipelined form with a row's K split over the KW waves of a group. A wave
+// takes P = ceil(blocks / KW) blocks (a multiple of 4: 16-byte chunks) of R
+// rows: it DMAs them into LDS rows of 2560 bytes (two blocks per lane) and
+// decodes each (row, block half) as soon as its pieces land; the KW waves' sums
+// meet in LDS in K order. Every wave of the launch is resident at once (K =
+// 14336, N = 4096: 1024 workgroups of 40 KiB, four per CU). Bound: HBM and the
+// decode, as the K = 4096 form. The register form it replaces there
+// (gemv_q4_1_rows) loops over K with two loads in flight per row. K = 14336,
+// N = 4096: M = 1 16.1 -> 11.6 us, M = 2 21.9 -> 14.2; K = 11008: 15.8 -> 11.3.
+// ---------------------------------------------------------------------------
+template <int MT, int KW>
+__global__ __launch_bounds__(256) void gemv_q4_1_parts(Q41Kern p)
+{
+    constexpr int R = 4, kRow = 128 * 20, C = R * kRow / 1024;
+    static_assert(4 % KW == 0, "whole groups per workgroup");
+    __shared__ __attribute__((aligned(16))) uint8_t stage[4 * C * 1024 + 4 * R * MT * 4];
+    float* const red = reinterpret_cast<float*>(stage + 4 * C * 1024);      // [wave][R * MT]
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % KW;
+    const int n0 = (blockIdx.x * (4 / KW) + wave / KW) * R;
+    const int nb = p.k / 32;                                  // host-checked: K % 128 == 0
+    const int per = ((nb + KW - 1) / KW + 3) / 4 * 4;
+    const int b0 = part * per;
+    const int mine = max(0, min(per, nb - b0));               // this wave's blocks of a row
+    // A first: its loads retire before the DMA pieces queued behind them
+    const uint32_t* A = static_cast<const uint32_t*>(p.a);    // f16 pairs
+    uint32_t ah[2][MT][16];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const bool live = lane + 64 * u < mine;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const v4i* src = reinterpret_cast<const v4i*>(A + (int64_t)min(m, p.m - 1) * (p.lda / 2) +
+                                                          (live ? b0 + lane + 64 * u : 0) * 16);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v4i x = src[q];
+                ah[u][m][4 * q + 0] = (uint32_t)x.x;
+                ah[u][m][4 * q + 1] = (uint32_t)x.y;
+                ah[u][m][4 * q + 2] = (uint32_t)x.z;
+                ah[u][m][4 * q + 3] = (uint32_t)x.w;
+            }
+        }
+    }
+    // every lane issues every piece (rows past N re-read row N - 1, chunks past
+    // the part its first chunk), so the piece count and the waits are static
+    uint8_t* const mystage = stage + wave * C * 1024;
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+        const int off = q * 1024 + lane * 16, r = off / kRow, c = off % kRow;
+        const uint8_t* src = p.b + (int64_t)min(n0 + r, p.n - 1) * p.ldb + (c < mine * 20 ? b0 * 20 + c : 0);
+        __builtin_amdgcn_global_load_lds(NNOPS_GPTR(src), NNOPS_LPTR(mystage + q * 1024), 16, 0, 2);
+    }
+    const v2h one = __builtin_bit_cast(v2h, 0x3c003c00u);
+    float asum[2][MT];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            float t = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                t = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, ah[u][m][j]), one, t, false);
+            }
+            asum[u][m] = t;
+        }
+    }
+    float acc[R][MT];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            acc[r][m] = 0.0f;
+        }
+    }
+    auto phase = [&]<int RR, int U>() {
+        // last byte this (row, half) needs, and the piece holding it
+        constexpr int last = RR * kRow + (64 * U + 63) * 20 + 19;
+        wait_vmcnt<C - 1 - last / 1024>();
+        asm volatile("" ::: "memory");
+        const uint32_t* bp = reinterpret_cast<const uint32_t*>(mystage + RR * kRow + (lane + 64 * U) * 20);
+        uint32_t raw[5];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            raw[i] = bp[i];
+        }
+        const float d = h2f(raw[0] & 0xffffu);
+        const float mn = h2f(raw[0] >> 16);
+        uint32_t h[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t lo = raw[1 + i] & 0x0f0f0f0fu;
+            const uint32_t hi = (raw[1 + i] >> 4) & 0x0f0f0f0fu;
+            h[2 * i] = nib_pair(lo, 0x04010400u);
+            h[2 * i + 1] = nib_pair(lo, 0x04030402u);
+            h[8 + 2 * i] = nib_pair(hi, 0x04010400u);
+            h[8 + 2 * i + 1] = nib_pair(hi, 0x04030402u);
+        }
+        const bool live = lane + 64 * U < mine;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            float sq = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                sq = __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, ah[U][m][j]), __builtin_bit_cast(v2h, h[j]), sq,
+                                            false);
+            }
+            const float qsum = 16.0f * (sq - 64.0f * asum[U][m]);
+            const float next = fmaf(d, qsum, fmaf(mn, asum[U][m], acc[RR][m]));
+            acc[RR][m] = live ? next : acc[RR][m];             // a block past the part: nothing
+        }
+    };
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (phase.template operator()<I / 2, I % 2>(), ...);
+    }(std::make_integer_sequence<int, 2 * R>{});
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            float v = acc[r][m];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                v += __shfl_xor(v, off, 64);
+            }
+            acc[r][m] = v;
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                red[wave * R * MT + r * MT + m] = acc[r][m];
+            }
+        }
+    }
+    __syncthreads();
+    // the group's first wave: lane r * MT + m sums the parts of output (m, n0 + r)
+    if (part == 0 && lane < R * MT) {
+        float v = red[wave * R * MT + lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) {
+            v += red[(wave + w) * R * MT + lane];
+        }
+        const int n = n0 + lane / MT, m = lane % MT;
+        if (n < p.n && m < p.m) {
+            store_out(p, m, n, v);
         }
     }
 }
@@ -1742,7 +1897,9 @@ __global__ __launch_bounds__(256) void gemv_q4_1_bcm_mfma(Q41Kern p)
 // and v_pk_fma_f16 rounds d * q + m once; the 16 x 32 weight tile and A's
 // 32 x 16 tile (lane l: row l % 16, the same 8 k) meet in one
 // v_mfma_f32_16x16x32_f16. The K parts meet in LDS at the end, in part
-// order. Bound: the decode at a few waves per SIMD, then HBM.
+// order. KSPLIT: blockIdx.y is a K split, whose f32 sums go to p.partial (a
+// long K over few columns, skinny_split). Bound: the decode at a few waves
+// per SIMD, then HBM.
 // ---------------------------------------------------------------------------
 constexpr int kSkRows = 32;                          // per workgroup (16 per wave)
 constexpr int kSkWChunks = 11;                       // per weight row: 10 + pad
@@ -1751,7 +1908,7 @@ constexpr int kSkAChunks = 33;                       // per row of A: 32 + pad
 constexpr int kSkAPieces = 10;                       // 16 x 33 = 528 chunks, in 2 x 5 pieces
 constexpr int kSkL = kSkWPieces + kSkAPieces / 2;    // DMA instructions per wave and stage
 
-template <int NS, int KH>
+template <int NS, int KH, bool KSPLIT>
 __global__ __launch_bounds__(128 * KH) void gemv_q4_1_skinny(Q41Kern p)
 {
     static_assert(NS >= 2 && (NS - 2) * kSkL < 64, "vmcnt range");
@@ -1763,8 +1920,11 @@ __global__ __launch_bounds__(128 * KH) void gemv_q4_1_skinny(Q41Kern p)
     const int grp = wave & 1, part = wave >> 1;
     const int n0 = blockIdx.x * kSkRows + 16 * grp;
     const int rows = max(1, min(16, p.n - n0));      // a group past N re-reads row N - 1 (never stored)
-    const int stages = p.k / 256 / KH;               // per part (host-checked: K % (256 KH) == 0)
-    const int s0 = part * stages;                    // the part's first stage of K
+    // stages per part of this K split (host-checked: K % (256 KH) == 0; the
+    // last split takes the rest), and the part's first stage of K
+    const int sp = KSPLIT ? blockIdx.y : 0;
+    const int stages = KSPLIT && sp < p.splits - 1 ? p.kt_per : p.k / 256 / KH - (KSPLIT ? sp * p.kt_per : 0);
+    const int s0 = (KSPLIT ? sp * p.kt_per * KH : 0) + part * stages;
     const QBufRsrc rw = q_buffer_rsrc(p.b + (int64_t)min(n0, p.n - 1) * p.ldb, (uint32_t)((int64_t)rows * p.ldb));
     const QBufRsrc ra = q_buffer_rsrc(p.a, 0x7fffffffu);
     int w_off[kSkWPieces], a_off[kSkAPieces / 2];
@@ -1863,7 +2023,11 @@ __global__ __launch_bounds__(128 * KH) void gemv_q4_1_skinny(Q41Kern p)
     for (int r = 0; r < 4; ++r) {
         const int n = n0 + 4 * qk + r;
         if (r16 < p.m && n < p.n) {
-            store_out(p, r16, n, acc[r]);
+            if constexpr (KSPLIT) {
+                p.partial[((int64_t)sp * p.m + r16) * p.n + n] = acc[r];
+            } else {
+                store_out(p, r16, n, acc[r]);
+            }
         }
     }
 }
@@ -3294,6 +3458,44 @@ inline size_t q41_ring_bytes(const NnopsGemmQ41Args& g, const Q41RingPlan& r)
     return r.splits > 1 ? align_up((size_t)r.splits * (size_t)g.m * (size_t)g.n * sizeof(float)) : 0;
 }
 
+// K splits of the skinny kernel (one launch of up to 16 rows): where its
+// workgroups, 32 columns each, leave room for two per CU and K is long. K =
+// 14336, N = 4096, 8 rows: 28.4 us unsplit, 16.8 in four; K = 11008 36.2 -> 18.7.
+inline int skinny_split(const NnopsGemmQ41Args& g)
+{
+    if (!g.a_f16 || g.m > 16 || !skinny_ok(g)) {
+        return 1;
+    }
+    const int64_t wgs = (g.n + kSkRows - 1) / kSkRows, units = g.k / (g.k % 512 == 0 ? 512 : 256);
+    const int64_t sp = std::min<int64_t>({16, 512 / std::max<int64_t>(wgs, 1), units / 6});
+    return (int)std::max<int64_t>(sp, 1);
+}
+
+inline size_t skinny_bytes(const NnopsGemmQ41Args& g)
+{
+    const int sp = skinny_split(g);
+    return sp > 1 ? align_up((size_t)sp * (size_t)g.m * (size_t)g.n * sizeof(float)) : 0;
+}
+
+inline void launch_skinny(const Q41Kern& k, bool a_f16, hipStream_t s)
+{
+    const dim3 grid((unsigned)((k.n + kSkRows - 1) / kSkRows), (unsigned)std::max(1, k.splits));
+    if (!a_f16) {
+        NNOPS_LAUNCH(gemv_q4_1_skinny_f32<3>, grid, dim3(128), 0, s, k);
+    } else if (k.k % 512 == 0) {
+        // two K halves per workgroup: four waves, two stages in flight
+        if (k.splits > 1) {
+            NNOPS_LAUNCH((gemv_q4_1_skinny<2, 2, true>), grid, dim3(256), 0, s, k);
+        } else {
+            NNOPS_LAUNCH((gemv_q4_1_skinny<2, 2, false>), grid, dim3(256), 0, s, k);
+        }
+    } else if (k.splits > 1) {
+        NNOPS_LAUNCH((gemv_q4_1_skinny<4, 1, true>), grid, dim3(128), 0, s, k);
+    } else {
+        NNOPS_LAUNCH((gemv_q4_1_skinny<4, 1, false>), grid, dim3(128), 0, s, k);
+    }
+}
+
 template <int OUT>
 void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
 {
@@ -3363,6 +3565,21 @@ inline void run_q41_split(const NnopsGemmQ41Args& g, const Q41RingPlan& r, FpOut
     launch_fp_out_pass(fo, s);
 }
 
+// The same for the skinny kernel's splits.
+inline void run_skinny_split(const NnopsGemmQ41Args& g, FpOut& fo, void* ws, hipStream_t s)
+{
+    Q41Kern k = q41_kern(g);
+    k.partial = static_cast<float*>(ws);
+    k.splits = skinny_split(g);
+    k.kt_per = k.k / (k.k % 512 == 0 ? 512 : 256) / k.splits;
+    launch_skinny(k, true, s);
+    fo.src = k.partial;
+    fo.ld_src = k.n;
+    fo.splits = k.splits;
+    fo.slab = (int64_t)k.m * k.n;
+    launch_fp_out_pass(fo, s);
+}
+
 // the pass that only sums and stores
 inline FpOut q41_store_pass(const NnopsGemmQ41Args& g)
 {
@@ -3414,6 +3631,9 @@ extern "C" size_t nnops_hip_gemm_q4_1_workspace_size(const NnopsGemmQ41Args* g)
     }
     if (ring_splits(*g) && g->n > 0 && g->m <= INT32_MAX && g->n <= INT32_MAX && g->k <= INT32_MAX) {
         return q41_ring_bytes(*g, plan_q41_ring(*g, 16));
+    }
+    if (const size_t skinny = skinny_bytes(*g); skinny > 0) {
+        return skinny;
     }
     return least_workspace(*g);
 }
@@ -3472,6 +3692,9 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
     if (ring.splits > 1) {
         FpOut fo = q41_store_pass(*g);
         run_q41_split(*g, ring, fo, workspace, s);
+    } else if (const size_t skinny = skinny_bytes(*g); skinny > 0 && skinny <= ws_bytes) {
+        FpOut fo = q41_store_pass(*g);
+        run_skinny_split(*g, fo, workspace, s);
     } else if (skinny_ok(*g) && starved) {
         // a few rows of A: the weight streams once per 16 rows
         for (int m0 = 0; m0 < k.m; m0 += 16) {
@@ -3479,15 +3702,7 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
             kk.m = std::min(16, k.m - m0);
             kk.a = static_cast<const char*>(g->a) + (int64_t)m0 * g->lda * (g->a_f16 ? 2 : 4);
             kk.c = static_cast<char*>(g->c) + (int64_t)m0 * g->ldc * (k.out_f16 ? 2 : 4);
-            const dim3 grid((unsigned)((g->n + kSkRows - 1) / kSkRows));
-            if (!g->a_f16) {
-                NNOPS_LAUNCH(gemv_q4_1_skinny_f32<3>, grid, dim3(128), 0, s, kk);
-            } else if (g->k % 512 == 0) {
-                // two K halves per workgroup: four waves, two stages in flight
-                NNOPS_LAUNCH((gemv_q4_1_skinny<2, 2>), grid, dim3(256), 0, s, kk);
-            } else {
-                NNOPS_LAUNCH((gemv_q4_1_skinny<4, 1>), grid, dim3(128), 0, s, kk);
-            }
+            launch_skinny(kk, g->a_f16 != 0, s);
         }
     } else if (use_gemv(*g)) {
         // rows of A handled per pass: 2 (f16 pairs), 1 for f32 A
@@ -3506,6 +3721,9 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
                     // LDS-staged rows: whole 16-byte chunks per row, <= 128 blocks
                     const bool staged = nbk <= 128 && (nbk % 4) == 0 && (g->ldb_bytes % 16) == 0 &&
                                         ((uintptr_t)g->b & 15) == 0;
+                    // longer rows, aligned A: K split over a group's waves
+                    const bool parts = nbk > 128 && nbk <= 512 && g->k % 128 == 0 && (g->ldb_bytes % 16) == 0 &&
+                                       ((uintptr_t)g->b & 15) == 0 && (g->lda % 8) == 0 && ((uintptr_t)kk.a & 15) == 0;
                     // K = 4096 rows stored back to back, aligned A: the pipelined form
                     const bool pipe = g->k == 128 * 32 && g->ldb_bytes == 128 * 20 && ((uintptr_t)g->b & 15) == 0 &&
                                       (g->lda % 8) == 0 && ((uintptr_t)kk.a & 15) == 0;
@@ -3516,6 +3734,20 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
                             NNOPS_LAUNCH((gemv_q4_1_pipe<1, 4>), dim3(rb4), dim3(256), 0, s, kk);
                         } else {
                             NNOPS_LAUNCH((gemv_q4_1_pipe<2, 4>), dim3(rb4), dim3(256), 0, s, kk);
+                        }
+                    } else if (parts && nbk <= 256) {
+                        const unsigned pb = (unsigned)((g->n + 7) / 8);
+                        if (kk.m == 1) {
+                            NNOPS_LAUNCH((gemv_q4_1_parts<1, 2>), dim3(pb), dim3(256), 0, s, kk);
+                        } else {
+                            NNOPS_LAUNCH((gemv_q4_1_parts<2, 2>), dim3(pb), dim3(256), 0, s, kk);
+                        }
+                    } else if (parts) {
+                        const unsigned pb = (unsigned)((g->n + 3) / 4);
+                        if (kk.m == 1) {
+                            NNOPS_LAUNCH((gemv_q4_1_parts<1, 4>), dim3(pb), dim3(256), 0, s, kk);
+                        } else {
+                            NNOPS_LAUNCH((gemv_q4_1_parts<2, 4>), dim3(pb), dim3(256), 0, s, kk);
                         }
                     } else if (staged) {
                         if (kk.m == 1) {
@@ -3694,21 +3926,31 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
                                     size_t ws_bytes, hipStream_t stream)
 {
     const TimingDisarm disarm;
-    if (!ring_splits(g) || g.n <= 0 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX ||
-        g.a == nullptr || g.b == nullptr || g.lda < g.k || g.ldb_bytes < g.k / 32 * 20 || (g.ldb_bytes & 3) ||
+    if (!g.trans_b || g.m <= 2 || g.n <= 0 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX ||
+        g.a == nullptr || g.b == nullptr || g.lda < g.k || g.ldb_bytes < (g.k + 31) / 32 * 20 || (g.ldb_bytes & 3) ||
         ((uintptr_t)g.b & 3) || workspace == nullptr || ((uintptr_t)workspace & 15) != 0 || pass.src == nullptr) {
         return NNOPS_UNSUPPORTED;
     }
-    const Q41RingPlan r = plan_q41_ring(g, 16);
-    if ((r.splits == 1 && !pass.gated) || q41_ring_bytes(g, r) > ws_bytes) {
-        return NNOPS_UNSUPPORTED;
-    }
-    // the gated form's fused tiles where they are the faster
-    if (pass.gated) {
-        const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
-        if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
+    const size_t skinny = skinny_bytes(g);
+    Q41RingPlan r;
+    if (skinny == 0) {
+        if (!ring_splits(g)) {
             return NNOPS_UNSUPPORTED;
         }
+        r = plan_q41_ring(g, 16);
+        if (r.splits == 1 && !pass.gated) {
+            return NNOPS_UNSUPPORTED;
+        }
+        // the gated form's fused tiles where they are the faster
+        if (pass.gated) {
+            const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
+            if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
+                return NNOPS_UNSUPPORTED;
+            }
+        }
+    }
+    if (std::max(skinny, q41_ring_bytes(g, r)) > ws_bytes) {
+        return NNOPS_UNSUPPORTED;
     }
     FpOut fo;
     if (const int rc = make_fp_out(&pass, fo); rc != NNOPS_OK) {
@@ -3720,8 +3962,12 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
     if ((pass.n + 1023) / 1024 * pass.rows > INT32_MAX) {
         return NNOPS_UNSUPPORTED;
     }
-    // an unsplit product (gated) goes where the caller's pass reads it
-    run_q41_split(g, r, fo, r.splits > 1 ? workspace : const_cast<float*>(pass.src), stream);
+    if (skinny > 0) {
+        run_skinny_split(g, fo, workspace, stream);
+    } else {
+        // an unsplit product (gated) goes where the caller's pass reads it
+        run_q41_split(g, r, fo, r.splits > 1 ? workspace : const_cast<float*>(pass.src), stream);
+    }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }
 

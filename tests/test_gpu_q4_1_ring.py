@@ -137,3 +137,39 @@ def test_q4_1_gated_tall_tiles(M, K, n, kw, f16):
             assert lib.nnops_hip_fp_output_pass(C.byref(p), st) == na.OK
         outs.append(host(y))
     assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))
+
+
+@pytest.mark.parametrize("K", [4224, 8192, 8320, 11008, 16384])
+@pytest.mark.parametrize("M,N", [(1, 37), (2, 130)])
+@pytest.mark.parametrize("out_f16", [True, False])
+def test_q4_1_gemv_long_rows(K, M, N, out_f16):
+    """GEMV rows past 128 blocks, K over two or four waves: the shortest and
+    longest rows of each, the last part shorter, ragged N. The pitch is wider
+    than the row; the weights of the padding would show up as huge values."""
+    import torch
+    announce(f"q4_1 gemv parts {M}x{K}x{N} f16={out_f16}")
+    x = dg.normal(M + K, (M, K)).astype(np.float16)
+    blk = dg.q4_1_blocks(N + K, N, K)
+    wide = np.full((N, blk.shape[1] + 48), 0x7b, np.uint8)
+    wide[:, :blk.shape[1]] = blk
+    c = torch.zeros((M, N), dtype=torch.float16 if out_f16 else torch.float32, device="cuda")
+    na.gemm_q4_1(dev(x), dev(wide), c, n=N, trans_b=True)
+    want = oracle.gemm_q4_1(x, blk, N, trans_b=True)
+    assert norm_err(host(c).astype(np.float32), want) <= TOL
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 14336, 100), (16, 11008, 516), (7, 6144, 1000), (5, 3072, 32)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_q4_1_skinny_splits(M, K, N, bias):
+    """Up to 16 rows over a long K: the skinny kernel's K splits (one longer
+    than the others), summed by the store pass or the bias pass."""
+    import torch
+    announce(f"q4_1 skinny split {M}x{K}x{N} bias={bias}")
+    x = dg.normal(M + K, (M, K)).astype(np.float16)
+    blk = dg.q4_1_blocks(N + K, N, K)
+    b = dg.normal(1, (N,)).astype(np.float16)
+    y = torch.zeros((M, N), dtype=torch.float16, device="cuda")
+    ins = [na.tensor(dev(x)), na.tensor(dev(blk), dtype=na.DT_Q4_1, shape=[N, K])] + ([na.tensor(dev(b))] if bias else [])
+    assert na.Linear(output_dtype=na.DT_F16).compute([na.tensor(y)], ins) == na.OK
+    want = oracle.q4_1_linear(x, blk, N, w_round_f16=True, out_f16=True, bias=b if bias else None).astype(np.float32)
+    assert norm_err(host(y).astype(np.float32), want) <= TOL
