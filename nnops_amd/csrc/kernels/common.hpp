@@ -90,8 +90,8 @@ inline uint64_t next_launch_epoch()
 // ---------------------------------------------------------------------------
 // Epilogue parameters, resolved once on the host (device pointers only).
 // ---------------------------------------------------------------------------
-// The least workspace nnops_hip_gemm_i8 runs a call with (its plan without K
-// splits; nnops_hip_gemm_i8_workspace_size is what the full plan takes).
+// The workspace nnops_hip_gemm_i8 asks of a call: that of its plan, or where
+// the ring is optional (gemm_i8.hip) that of the plan without it.
 size_t gemm_i8_least_workspace(const NnopsGemmI8Args& g);
 
 // The Q4_1 GEMM as K splits whose partials, in the workspace, the output pass

@@ -33,7 +33,7 @@ namespace nnops_amd {
 
 // gemm_f16.hip: the ring GEMM over f16 operands (C = alpha A B, f32 or f16 C),
 // or NNOPS_UNSUPPORTED, nothing launched, where the shape, the alignment or
-// (below 64 rows) the workspace does not fit it.
+// (shapes with another kernel) the workspace does not fit it.
 int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s);
 size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g);
 

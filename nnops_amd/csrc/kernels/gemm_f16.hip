@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void transpose_b16(const uint16_t* src, int64_
 }
 
 // C = alpha * (the f16 ring's f32 partials summed in split order): 4 columns
-// per thread (N % 4 == 0), grid.y walking the rows; a group's splits are loaded
+// per thread (the last past N cut), grid.y walking the rows; a group's splits are loaded
 // four at a time ahead of their sum. Bound: HBM / MALL.
 __global__ __launch_bounds__(256) void ring_f16_reduce(GemmI8Kern p, RingSplit sk)
 {
@@ -41,9 +41,10 @@ __global__ __launch_bounds__(256) void ring_f16_reduce(GemmI8Kern p, RingSplit s
         return;
     }
     const bool f16 = p.ep.out_kind == NNOPS_OUT_F16;
-    const int64_t slab = (int64_t)p.m * p.n;
+    const int64_t slab = (int64_t)p.m * sk.ldp;
+    const int cn = min(4, p.n - nb);
     for (int m = (int)blockIdx.y; m < p.m; m += (int)gridDim.y) {
-        const float* src = reinterpret_cast<const float*>(sk.part) + (int64_t)m * p.n + nb;
+        const float* src = reinterpret_cast<const float*>(sk.part) + (int64_t)m * sk.ldp + nb;
         v4f v = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         int sp = 0;
         for (; sp + 3 < sk.splits; sp += 4) {
@@ -59,6 +60,9 @@ __global__ __launch_bounds__(256) void ring_f16_reduce(GemmI8Kern p, RingSplit s
         char* crow = static_cast<char*>(p.c) + (int64_t)m * p.ldc_bytes;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+            if (e >= cn) {
+                break;
+            }
             const float y = __fmul_rn(v[e], p.ep.s_a_scalar);
             if (f16) {
                 reinterpret_cast<_Float16*>(crow)[nb + e] = (_Float16)y;
@@ -118,7 +122,7 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
     }
     if (f.ring.mode == RING_PART) {
         f.part_off = off;
-        off += align_up((size_t)f.ring.splits * (size_t)g.m * (size_t)g.n * 4);
+        off += align_up((size_t)f.ring.splits * (size_t)g.m * (size_t)((g.n + 3) / 4) * 16);
     }
     f.total = off;
     return f;
@@ -138,7 +142,9 @@ size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g)
 
 int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s)
 {
-    if (workspace == nullptr || (g.m < 64 && (uintptr_t)workspace % 16 != 0)) {
+    // shapes that the GEMV and the tile kernel take without a workspace
+    const bool optional = g.m < 64 || g.k % 32 != 0 || g.n % 4 != 0;
+    if (workspace == nullptr || (optional && (uintptr_t)workspace % 16 != 0)) {
         ws_bytes = 0;
     }
     F16Plan f = plan_f16(g);
@@ -149,10 +155,9 @@ int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hi
         return NNOPS_UNSUPPORTED;
     }
     if (ws_bytes < f.total) {
-        // below 64 rows the caller has kernels that need none
-        return g.m < 64 ? NNOPS_UNSUPPORTED : NNOPS_NOT_INITIALIZED;
+        return optional ? NNOPS_UNSUPPORTED : NNOPS_NOT_INITIALIZED;
     }
-    if (g.m >= 64 && (uintptr_t)workspace % 16 != 0) {
+    if (!optional && (uintptr_t)workspace % 16 != 0) {
         return NNOPS_INVALID_ARGUMENT;   // staged operands and partials are 16-byte vectors
     }
     char* ws = static_cast<char*>(workspace);
@@ -185,7 +190,7 @@ int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hi
     const RingSplit sk = ring_split(k, f.ring, reinterpret_cast<int32_t*>(ws + f.part_off));
     launch_ring_tiles<true, false>(k, f.ring, sk, s);
     if (f.ring.mode == RING_PART) {
-        const dim3 grid((unsigned)((k.n / 4 + 255) / 256), (unsigned)std::min(k.m, 65535));
+        const dim3 grid((unsigned)((sk.ldp / 4 + 255) / 256), (unsigned)std::min(k.m, 65535));
         NNOPS_LAUNCH(ring_f16_reduce, grid, dim3(256), 0, s, k, sk);
     }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;

@@ -538,6 +538,7 @@ struct Out4 {
     uint32_t oldw;
     char* crow;
     int8_t* c8;
+    int cn;            // columns within N
     bool word8;
 };
 
@@ -547,11 +548,12 @@ __device__ __forceinline__ Out4 out4_prepare(const GemmI8Kern& p, int m, int nb)
     Out4 o{};
     o.crow = static_cast<char*>(p.c) + (int64_t)m * p.ldc_bytes;
     o.c8 = reinterpret_cast<int8_t*>(o.crow) + nb;
-    o.word8 = !epi_is_fp(ep) && ep.out_kind != NNOPS_OUT_S32 && ((uintptr_t)o.c8 & 3) == 0;
+    o.cn = min(4, p.n - nb);
+    o.word8 = !epi_is_fp(ep) && ep.out_kind != NNOPS_OUT_S32 && o.cn == 4 && ((uintptr_t)o.c8 & 3) == 0;
     o.row = epi_row(ep, m);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        o.cols[e] = epi_col(ep, nb + e);
+        o.cols[e] = epi_col(ep, min(nb + e, p.n - 1));
     }
     if (o.word8 && ep.add_to) {
         o.oldw = *reinterpret_cast<const uint32_t*>(o.c8);
@@ -566,7 +568,9 @@ __device__ __forceinline__ void out4_store(const GemmI8Kern& p, const Out4& o, i
     if (epi_is_fp(ep)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            epi_store(ep, o.row, o.cols[e], raw[e], o.crow, nb + e);
+            if (e < o.cn) {
+                epi_store(ep, o.row, o.cols[e], raw[e], o.crow, nb + e);
+            }
         }
         return;
     }
@@ -574,7 +578,9 @@ __device__ __forceinline__ void out4_store(const GemmI8Kern& p, const Out4& o, i
         int32_t* c32 = reinterpret_cast<int32_t*>(o.crow) + nb;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            c32[e] = epi_value(ep, o.row, o.cols[e], raw[e], 0);
+            if (e < o.cn) {
+                c32[e] = epi_value(ep, o.row, o.cols[e], raw[e], 0);
+            }
         }
         return;
     }
@@ -592,6 +598,9 @@ __device__ __forceinline__ void out4_store(const GemmI8Kern& p, const Out4& o, i
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
+        if (e >= o.cn) {
+            break;
+        }
         const int32_t old = ep.add_to ? (u8 ? (int32_t)((const uint8_t*)o.c8)[e] : (int32_t)o.c8[e]) : 0;
         o.c8[e] = (int8_t)epi_value(ep, o.row, o.cols[e], raw[e], old);
     }
@@ -599,7 +608,7 @@ __device__ __forceinline__ void out4_store(const GemmI8Kern& p, const Out4& o, i
 
 // Sum of the K-split partial accumulators and the full output pass
 // (compensation, bias, Relu, requant or the float epilogue, add_to). TPG
-// threads share a group of 4 consecutive columns of a row (N % 4 == 0), each
+// threads share a group of 4 consecutive columns of a row (the last past N is cut), each
 // summing every TPG-th split with its loads in flight together, then combine
 // with lane shuffles; the first of them runs the output pass. TPG = 16 suits
 // many splits of a small output (each thread's loads in one round trip), TPG =
@@ -607,14 +616,14 @@ __device__ __forceinline__ void out4_store(const GemmI8Kern& p, const Out4& o, i
 template <int TPG>
 __global__ __launch_bounds__(256) void gemm_i8_reduce(GemmI8Kern p, RingSplit sk)
 {
-    const int groups = p.n / 4;
+    const int groups = sk.ldp / 4;
     const int64_t gid = ((int64_t)blockIdx.x * 256 + threadIdx.x) / TPG;
     const int j = threadIdx.x % TPG;
     const bool in = gid < (int64_t)p.m * groups;
     const int m = in ? (int)(gid / groups) : 0;
     const int nb = in ? (int)(gid - (int64_t)m * groups) * 4 : 0;
-    const int64_t slab = (int64_t)p.m * p.n;
-    const int32_t* src = sk.part + (int64_t)m * p.n + nb;
+    const int64_t slab = (int64_t)p.m * sk.ldp;
+    const int32_t* src = sk.part + (int64_t)m * sk.ldp + nb;
     // the output pass's constants and the residual word, loaded with the
     // partials rather than after them
     Out4 o{};
@@ -675,7 +684,7 @@ __global__ __launch_bounds__(256) void gemm_i8_reduce_q(GemmI8Kern p, RingSplit 
     const float row_k = sk.row_k;
     const float inv_out = sk.inv_out;
     const bool clip = !(ep.min_clip == -__builtin_inff() && ep.max_clip == __builtin_inff());
-    const int64_t slab = (int64_t)p.m * p.n;
+    const int64_t slab = (int64_t)p.m * p.n;              // N % 4 == 0: the partials' pitch is N
     for (int m = (int)blockIdx.y; m < p.m; m += (int)gridDim.y) {
         const int32_t* src = sk.part + (int64_t)m * p.n + nb;
         v4i raw = v4i{0, 0, 0, 0};
@@ -1653,8 +1662,12 @@ KnPlan plan_kn(const NnopsGemmI8Args& g)
 }
 
 
+// Shapes that gemm_i8_mfma, which writes no partials, also takes at a tolerable
+// rate: they run without the ring where the workspace has no room for it.
+inline bool ring_optional(const NnopsGemmI8Args& g) { return g.m < 64 || g.k % 64 != 0 || g.n % 4 != 0; }
+
 // lean: the plan for a workspace too small for the full one: no K split, and
-// below 64 rows no ring (gemm_i8_mfma writes no partials).
+// no ring where it is optional.
 WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
 {
     WsPlan w;
@@ -1685,7 +1698,7 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
     const bool need_rb = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0;
     // (from 17 rows: 24 x 11008 x 4096 s8 15.8 us on 64 x 64 tiles in four
     // splits, 52 us on gemm_i8_mfma's 64 workgroups of the whole K)
-    const bool ring = g.m > 16 && !(lean && g.m < 64);
+    const bool ring = g.m > 16 && !(lean && ring_optional(g));
     const int max_splits = lean ? 1 : 16;
     if (!g.trans_b && !need_rb && ring) {
         w.ring = plan_ring(g, a, lda, b, ldb, true, max_splits);
@@ -1698,8 +1711,15 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
     if (!w.ring.trb && ring) {
         w.ring = plan_ring(g, a, lda, b, ldb, false, max_splits);
     }
+    // few rows that need the general output pass, over a short k: one launch of
+    // gemm_i8_mfma (0.3 us per 64 bytes of k) before the ring and its reduce
+    // (34 x 1024 x 677: 11.3 against 12.2 us)
+    if (w.ring.mode == RING_PART && !w.ring.trb && w.ring.splits == 1 && g.m < 64 &&
+        0.3f * (float)(g.k / 64) < w.ring.us) {
+        w.ring = RingPlan{};
+    }
     if (w.ring.mode == RING_PART) {
-        w.part = off; off += align_up((size_t)w.ring.splits * (size_t)g.m * (size_t)g.n * 4);
+        w.part = off; off += align_up((size_t)w.ring.splits * (size_t)g.m * (size_t)((g.n + 3) / 4) * 16);
     }
     w.total = off;
     return w;
@@ -1753,7 +1773,7 @@ bool reduce_q_ok(const GemmI8Kern& k)
 {
     const EpiParams& e = k.ep;
     return (e.out_kind == NNOPS_OUT_S8 || e.out_kind == NNOPS_OUT_U8) && !e.compensate && e.s_a == nullptr &&
-           e.s_out_rows == nullptr && e.zp_out_rows == nullptr && ((uintptr_t)e.s_b % 16) == 0 &&
+           e.s_out_rows == nullptr && e.zp_out_rows == nullptr && k.n % 4 == 0 && ((uintptr_t)e.s_b % 16) == 0 &&
            ((uintptr_t)e.bias % 16) == 0 && ((uintptr_t)k.c % 4) == 0 && (k.ldc_bytes % 4) == 0 &&
            (e.act == NNOPS_ACT_NONE || e.act == NNOPS_ACT_RELU || (e.act == NNOPS_ACT_GELU && e.float_ep));
 }
@@ -1777,7 +1797,7 @@ void launch_reduce_q_act(const GemmI8Kern& k, const RingSplit& sk, const dim3& g
 
 void launch_reduce(const GemmI8Kern& k, const RingSplit& sk, hipStream_t s)
 {
-    const int64_t groups = (int64_t)k.m * (k.n / 4);
+    const int64_t groups = (int64_t)k.m * (sk.ldp / 4);
     if (sk.splits <= 8 && reduce_q_ok(k)) {
         const dim3 grid((unsigned)((k.n / 4 + 255) / 256), (unsigned)std::min<int64_t>(k.m, 65535));
         RingSplit q = sk;
@@ -1805,6 +1825,7 @@ void launch_kn(const GemmI8Kern& k, const KnPlan& r, int32_t* part, uint64_t* fl
     sk.splits = r.splits;
     sk.kt_per = 0;
     sk.part = part;
+    sk.ldp = k.n;
     if (r.tr) {
         sk.flag = flag;
         sk.epoch = next_launch_epoch();
@@ -1915,7 +1936,7 @@ extern "C" size_t nnops_hip_gemm_i8_workspace_size(const NnopsGemmI8Args* g)
 
 size_t nnops_amd::gemm_i8_least_workspace(const NnopsGemmI8Args& g)
 {
-    return plan_workspace(g, true).total;
+    return plan_workspace(g, ring_optional(g)).total;
 }
 
 extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, void* stream)

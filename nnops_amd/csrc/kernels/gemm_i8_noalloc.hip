@@ -63,9 +63,7 @@ extern "C" int nnops_hip_gemm_i8_noalloc(const NnopsGemmI8Args* args, void* stre
     if (args == nullptr) {
         return NNOPS_INVALID_ARGUMENT;
     }
-    // (below 64 rows a plan without partials takes over where they do not fit)
-    const size_t need = args->m < 64 ? nnops_amd::gemm_i8_least_workspace(*args)
-                                     : nnops_hip_gemm_i8_workspace_size(args);
+    const size_t need = nnops_amd::gemm_i8_least_workspace(*args);
     if (need > kScratchBytes) {
         return NNOPS_OUT_OF_MEMORY;   // the plan needs more than the fixed array holds
     }

@@ -27,7 +27,8 @@ enum { RING_S8 = 0, RING_S32 = 1, RING_PART = 2, RING_FP = 3 };
 struct RingSplit {
     int splits;        // K ranges per output tile
     int kt_per;        // staged k steps per split (the last split takes the rest)
-    int32_t* part;     // RING_PART: [splits][M][N] raw accumulators
+    int32_t* part;     // RING_PART: [splits][M][ldp] raw accumulators
+    int ldp;           // the partials' row pitch: N rounded up to 4
     float row_k;       // gemm_i8_reduce_q: RN(s_a / s_out) and RN(1 / s_out), the
     float inv_out;     // host's correctly rounded f32 quotients (the device's bits)
     uint64_t* flag;    // gemv_i8_kn_tr: [column groups][splits] split-completion flags
@@ -37,10 +38,10 @@ struct RingSplit {
 // Which ring-kernel configuration a call takes (all zero: another kernel).
 struct RingPlan {
     int bm = 0, bn = 0;     // block tile
-    int bk = 64;            // k bytes per staged row (128 when K allows)
     int splits = 0;         // K splits (1: no split)
     int mode = -1;          // RING_S8 / RING_S32 / RING_PART
     bool trb = false;       // B is [K,N] row-major, read in place (TRB)
+    float us = 0.0f;        // the estimate it won by
 };
 
 // The ring plan of an int8 call (ring_plan.hip); an f16 call asks with its K and
@@ -70,7 +71,7 @@ __device__ __forceinline__ int32_t med3_i32(int32_t x, int32_t lo, int32_t hi)
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile kernel with an asynchronous LDS ring (K % 64 == 0, 16-byte-aligned
+// Large-tile kernel with an asynchronous LDS ring (K % 32 == 0, 16-byte-aligned
 // operands). Stages are filled by buffer_load_dwordx4 ... lds: each wave
 // instruction writes 1 KiB of LDS contiguously (lane l -> bytes 16l..16l+15),
 // i.e. 16 tile rows of 64 bytes, so the 16-byte chunk a lane fetches from HBM
@@ -313,13 +314,20 @@ __device__ __forceinline__ void ring_coords(int tiles_m, int tiles_n, int& tm, i
 // stage holds BK k rows of BN bytes, 16-byte chunk c of row r in slot
 // c ^ swzb(r), and the B fragments are built by lds_read_tr8 (two per
 // fragment: k rows +0..7 and +8..15 of the lane's 16). No transposed copy.
-template <int BM, int BN, int WM, int WN, int BK, int NS, int MODE, bool FLIP, bool F16 = false, bool TRB = false>
+//
+// TAIL: K % 128 != 0 (a multiple of 32): the last stage holds fewer than four
+// 32-byte slices of k. Its staging reads past a row's k (into the next row's,
+// or past the operand's end, where the descriptors make it 0); only the slices
+// of k run on the matrix cores.
+template <int BM, int BN, int WM, int WN, int NS, int MODE, bool FLIP, bool F16 = false, bool TRB = false,
+          bool TAIL = false>
 __global__ __launch_bounds__(WM * WN * 64)
 __attribute__((amdgpu_waves_per_eu((WM * WN + 3) / 4, BM + BN <= 192 ? 4 : (WM * WN + 3) / 4)))
 void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
 {
     static_assert(!F16 || MODE == RING_FP || MODE == RING_PART, "f16 operands: fp or partial outputs");
     static_assert(!TRB || !F16, "row-major B: int8 operands");
+    constexpr int BK = 128;                       // k bytes per stage and row
     constexpr int W = WM * WN;
     constexpr int TM = BM / WM, TN = BN / WN;
     constexpr int FM = TM / 32, FN = TN / 32;
@@ -337,7 +345,6 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
     constexpr int S = BK / 32;                    // 32-k MFMA slices per stage
     constexpr int kStage = (BM + BN) * BK;
     constexpr int kPitch8 = TN + 16;              // staged byte row pitch: 2-way bank conflicts at most
-    static_assert(BK == 64 || BK == 128, "stage depth");
     static_assert(QA * W * RPI == BM && QB * W * RPI == BN, "rows per stage");
     // TRB staging: 1024 / BN k rows per load instruction, CPRB chunks per row
     constexpr int RPIB = TRB ? 1024 / BN : 1;
@@ -372,13 +379,15 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm0 = (wave / WN) * TM, wn0 = (wave % WN) * TN;
     const int kt0 = sp * sk.kt_per;
-    const int kt = (sp == sk.splits - 1) ? p.k / BK - kt0 : sk.kt_per;
+    const int kt = (sp == sk.splits - 1) ? (p.k + BK - 1) / BK - kt0 : sk.kt_per;
+    // the stages of whole slices, and the slices of a last, shorter one
+    const int tail = TAIL && sp == sk.splits - 1 ? (p.k % BK) / 32 : 0;
+    const int kf = tail != 0 ? kt - 1 : kt;
 
     // Staged rows are BK bytes; chunk c of row r sits in slot c ^ swz(r), so
     // the 16 rows a fragment read serves per LDS cycle hit 16 distinct 16-byte
-    // bank groups (BK = 64: 4 rows per 256 bytes, swz = (r >> 2) & 3;
-    // BK = 128: 2 rows per 256 bytes, swz = (r >> 1) & 7).
-    auto swz = [](int r) { return BK == 64 ? ((r >> 2) & 3) : ((r >> 1) & 7); };
+    // bank groups (2 rows per 256 bytes).
+    auto swz = [](int r) { return (r >> 1) & 7; };
     // TRB: a transposed read serves 8 k rows x two 16-byte chunks per 32
     // lanes; rows sharing a 256-byte bank row (256 / BN of them) keep their
     // slots, and the bank rows' 8 slot pairs differ in slot bits 1.., so the
@@ -387,12 +396,15 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
 
     // Descriptors over this tile's row panels from this split's first k; rows
     // past M/N are clamped to the last row (computed, never stored).
-    const BufRsrc rsa = buffer_rsrc(p.a + (int64_t)m0 * p.lda + (int64_t)kt0 * BK);
+    // They end at the last row's last k.
+    const int a_end = (min(BM, p.m - m0) - 1) * (int)p.lda + p.k - kt0 * BK;
+    const BufRsrc rsa = buffer_rsrc(p.a + (int64_t)m0 * p.lda + (int64_t)kt0 * BK, a_end);
     // TRB: the descriptor ends at B's last byte, so chunks past column N of
     // the last k row read 0 (earlier rows' read the next row: never stored)
     const BufRsrc rsb = TRB ? buffer_rsrc(p.b + (int64_t)kt0 * BK * p.ldb + n0,
                                           (int)((int64_t)(p.k - kt0 * BK - 1) * p.ldb + (p.n - n0)))
-                            : buffer_rsrc(p.b + (int64_t)n0 * p.ldb + (int64_t)kt0 * BK);
+                            : buffer_rsrc(p.b + (int64_t)n0 * p.ldb + (int64_t)kt0 * BK,
+                                          (min(BN, p.n - n0) - 1) * (int)p.ldb + p.k - kt0 * BK);
     int a_off[QA], b_off[QB];
 #pragma unroll
     for (int q = 0; q < QA; ++q) {
@@ -686,13 +698,32 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
     // own gets a full vmcnt(0) before it)
     int t0 = 0;
     if constexpr (kTrAsm) {
-        if (kt > 0) {
+        if (kf > 0) {
             step(0);
         }
         t0 = 1;
     }
-    for (int t = t0; t < kt; ++t) {
+    for (int t = t0; t < kf; ++t) {
         step(t);
+    }
+    if constexpr (TAIL) {
+        // slice 0 of the last stage is read already
+        const int8_t* st = ring + ((kt - 1) % NS) * kStage;
+        auto tail_slice = [&](int ks, v4i (&fa)[FM], v4i (&fb)[FN]) {
+            if (ks < tail) {
+                if (ks > 0) {
+                    read_frags(st, ks, fa, fb);
+                }
+                if constexpr (kTrAsm) {
+                    lds_tr8_ready_frags(fb);
+                }
+                mfma_all(fa, fb);
+            }
+        };
+        // (an even stage ends with slice 0 of the next in f0a / f0b)
+        tail_slice(0, f0a, f0b);
+        tail_slice(1, f1a, f1b);
+        tail_slice(2, f0a, f0b);
     }
     // The output pass's per-column scales: from the LDS copy staged at the
     // start, or else a lane's 8 loads issued together with one wait. They are
@@ -1058,7 +1089,8 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
             }
         }
     } else {
-        // int32 groups (host-checked: N % 4 == 0, 16-byte-aligned rows),
+        // int32 groups (16-byte-aligned rows: host-checked for C, N % 4 == 0;
+        // a last group past N stays within the partials' pitch),
         // staged through the ring so every store is a 16-byte piece of a
         // whole tile row: 32 lanes write one row's BN * 4 bytes. Straight
         // from the accumulator layout a store instruction would touch 32 rows
@@ -1073,8 +1105,8 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
             cbase = static_cast<char*>(p.c);
             ld = p.ldc_bytes;
         } else {
-            cbase = reinterpret_cast<char*>(sk.part + (int64_t)sp * p.m * p.n);
-            ld = (int64_t)p.n * 4;
+            cbase = reinterpret_cast<char*>(sk.part + (int64_t)sp * p.m * sk.ldp);
+            ld = (int64_t)sk.ldp * 4;
         }
         constexpr int kRowB = BN * 4 + 16;            // staged row pitch: rows 16 bytes apart in the banks
         constexpr int PI = (WM * FM * 32 * kRowB <= NS * kStage) ? FM
@@ -1135,8 +1167,8 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
     }
 }
 
-template <int BM, int BN, int WM, int WN, int BK, int NS, bool F16, bool TRB>
-void launch_ring_bk(const GemmI8Kern& k, const RingSplit& sk, int mode, bool flip, hipStream_t s)
+template <int BM, int BN, int WM, int WN, int NS, bool F16, bool TRB, bool TAIL>
+void launch_ring_mode(const GemmI8Kern& k, const RingSplit& sk, int mode, bool flip, hipStream_t s)
 {
     const unsigned blocks = (unsigned)(((k.m + BM - 1) / BM) * ((k.n + BN - 1) / BN) * sk.splits);
     const dim3 block(WM * WN * 64);
@@ -1144,62 +1176,54 @@ void launch_ring_bk(const GemmI8Kern& k, const RingSplit& sk, int mode, bool fli
         // [K,N] B in place; plain A (no u8 flip: its column sums need the copy)
         (void)flip;
         if (mode == RING_S8) {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_S8, false, false, true>), dim3(blocks), block, 0, s,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_S8, false, false, true, TAIL>), dim3(blocks), block, 0, s,
                          k, sk);
         } else if (mode == RING_S32) {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_S32, false, false, true>), dim3(blocks), block, 0,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_S32, false, false, true, TAIL>), dim3(blocks), block, 0,
                          s, k, sk);
         } else if (mode == RING_FP) {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_FP, false, false, true>), dim3(blocks), block, 0, s,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_FP, false, false, true, TAIL>), dim3(blocks), block, 0, s,
                          k, sk);
         } else {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_PART, false, false, true>), dim3(blocks), block, 0,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_PART, false, false, true, TAIL>), dim3(blocks), block, 0,
                          s, k, sk);
         }
     } else if constexpr (F16) {
         (void)flip;
         if (mode == RING_FP) {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_FP, false, true>), dim3(blocks), block, 0,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_FP, false, true, false, TAIL>), dim3(blocks), block, 0,
                                s, k, sk);
         } else {
-            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_PART, false, true>), dim3(blocks), block,
+            NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_PART, false, true, false, TAIL>), dim3(blocks), block,
                                0, s, k, sk);
         }
     } else if (flip) {
-        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_PART, true>), dim3(blocks), block, 0, s, k, sk);
+        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_PART, true, false, false, TAIL>), dim3(blocks), block, 0, s, k, sk);
     } else if (mode == RING_S8) {
-        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_S8, false>), dim3(blocks), block, 0, s, k, sk);
+        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_S8, false, false, false, TAIL>), dim3(blocks), block, 0, s, k, sk);
     } else if (mode == RING_S32) {
-        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_S32, false>), dim3(blocks), block, 0, s, k, sk);
+        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_S32, false, false, false, TAIL>), dim3(blocks), block, 0, s, k, sk);
     } else if (mode == RING_FP) {
-        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_FP, false>), dim3(blocks), block, 0, s, k, sk);
+        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_FP, false, false, false, TAIL>), dim3(blocks), block, 0, s, k, sk);
     } else {
-        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, BK, NS, RING_PART, false>), dim3(blocks), block, 0, s, k, sk);
+        NNOPS_LAUNCH((gemm_i8_ring<BM, BN, WM, WN, NS, RING_PART, false, false, false, TAIL>), dim3(blocks), block, 0, s, k, sk);
     }
 }
 
 // 128-byte staged rows (whole cache lines: twice the bytes per L2 request of
-// 64-byte rows, which is what limits a CU's load rate) in 2 slots when K
-// allows, else 64-byte rows in 4 slots.
+// 64-byte rows, which is what limits a CU's load rate). Three stage slots
+// where the LDS holds them (192x128 tiles: 33.7 -> 32.9 us against two), two
+// for the 256x256 tile, four for the tiles of 128 columns and rows or fewer;
+// the 64 x 64 tiles of small grids keep 8 stages in flight (their latency is
+// the call's).
 template <int BM, int BN, int WM, int WN, bool F16, bool TRB>
-void launch_ring_cfg(const GemmI8Kern& k, const RingSplit& sk, int bk, int mode, bool flip, hipStream_t s)
+void launch_ring_cfg(const GemmI8Kern& k, const RingSplit& sk, int mode, bool flip, hipStream_t s)
 {
-    if (bk == 128) {
-        // three stage slots where the LDS holds them (config 5's 192x128 tiles:
-        // 33.7 -> 32.9 us), two for the 256x256 tile, four for the tiles of
-        // 128 columns and rows or fewer; the 64 x 64 tiles of small grids keep
-        // 8 stages in flight (their latency is the call's)
-        if constexpr (BM + BN <= 128) {
-            launch_ring_bk<BM, BN, WM, WN, 128, 8, F16, TRB>(k, sk, mode, flip, s);
-        } else if constexpr (BM + BN <= 256) {
-            launch_ring_bk<BM, BN, WM, WN, 128, 4, F16, TRB>(k, sk, mode, flip, s);
-        } else if constexpr ((BM + BN) * 128 * 3 <= 160 * 1024 && BM + BN < 512) {
-            launch_ring_bk<BM, BN, WM, WN, 128, 3, F16, TRB>(k, sk, mode, flip, s);
-        } else {
-            launch_ring_bk<BM, BN, WM, WN, 128, 2, F16, TRB>(k, sk, mode, flip, s);
-        }
-    } else if constexpr (BM % (16 * WM * WN) == 0 && BN % (16 * WM * WN) == 0) {
-        launch_ring_bk<BM, BN, WM, WN, 64, 4, F16, TRB>(k, sk, mode, flip, s);
+    constexpr int NS = BM + BN <= 128 ? 8 : BM + BN <= 256 ? 4 : BM + BN < 512 ? 3 : 2;
+    if (k.k % 128 == 0) {
+        launch_ring_mode<BM, BN, WM, WN, NS, F16, TRB, false>(k, sk, mode, flip, s);
+    } else {
+        launch_ring_mode<BM, BN, WM, WN, NS, F16, TRB, true>(k, sk, mode, flip, s);
     }
 }
 
@@ -1210,19 +1234,19 @@ void launch_ring_tiles(const GemmI8Kern& k, const RingPlan& r, const RingSplit& 
     const bool flip = k.a_xor != 0u;
     auto is = [&](int bm, int bn) { return r.bm == bm && r.bn == bn; };
     if (is(64, 64)) {
-        launch_ring_cfg<64, 64, 2, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<64, 64, 2, 2, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(128, 64)) {
-        launch_ring_cfg<128, 64, 2, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<128, 64, 2, 2, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(128, 128)) {
-        launch_ring_cfg<128, 128, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<128, 128, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(192, 128)) {
-        launch_ring_cfg<192, 128, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<192, 128, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(256, 128)) {
-        launch_ring_cfg<256, 128, 4, 2, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<256, 128, 4, 2, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(128, 256)) {
-        launch_ring_cfg<128, 256, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<128, 256, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
     } else {
-        launch_ring_cfg<256, 256, 2, 4, F16, TRB>(k, sk, r.bk, r.mode, flip, s);
+        launch_ring_cfg<256, 256, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
     }
 }
 
@@ -1230,8 +1254,9 @@ inline RingSplit ring_split(const GemmI8Kern& k, const RingPlan& r, int32_t* par
 {
     RingSplit sk{};
     sk.splits = r.splits;
-    sk.kt_per = (k.k / r.bk) / r.splits;
+    sk.kt_per = ((k.k + 127) / 128) / r.splits;
     sk.part = part;
+    sk.ldp = (k.n + 3) / 4 * 4;
     return sk;
 }
 

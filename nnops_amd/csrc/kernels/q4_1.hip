@@ -2596,7 +2596,7 @@ __global__ __launch_bounds__(256) void split_a_f32(const float* a, int64_t lda, 
 
 // ---------------------------------------------------------------------------
 // MFMA GEMM, f16 A, B blocks along K ([N][K/32], 2 blocks = 40 bytes per row
-// per 64-k stage), K % 64 == 0. BM x BN tiles, WM x WN waves (128 x 256 tiles:
+// per 64-k stage), K % 32 == 0. BM x BN tiles, WM x WN waves (128 x 256 tiles:
 // 1 x 8, each wave 128 x 32, two per SIMD; 256 x 256: 2 x 4 of 128 x 64; tiles
 // of 128 columns: 1 x 4) of 32x32 fragments
 // (v_mfma_f32_32x32x16_f16), an NS-stage LDS ring filled only by
@@ -2679,10 +2679,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
     const int wm0 = (wave / WN) * TM;
     // this split's stages of 64 k
     const int kt0 = OUT == QOUT_PART ? sp * p.kt_per : 0;
-    const int kt = OUT == QOUT_PART && sp < p.splits - 1 ? p.kt_per : p.k / 64 - kt0;
+    const int kt = OUT == QOUT_PART && sp < p.splits - 1 ? p.kt_per : (p.k + 63) / 64 - kt0;
+    // K % 64 == 32: the last stage holds one block of k (its staging reads on
+    // into the next row, or 0 past the operand's end; unused)
+    const bool half = p.k % 64 != 0 && kt0 + kt == (p.k + 63) / 64;
+    const int kf = half ? kt - 1 : kt;
 
     // A: rows 8 * (4 * wave + i) + lane / 8; B raw: rows 16 * (4 * wave + i) + lane / 4
-    const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda + (int64_t)kt0 * 64, 0x7fffffffu);
+    const int64_t a_bytes = SPLIT ? 0x7fffffff
+                                  : ((int64_t)(min(BM, p.m - m0) - 1) * p.lda + p.k - (int64_t)kt0 * 64) * 2;
+    const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda + (int64_t)kt0 * 64,
+                                       (uint32_t)std::min<int64_t>(a_bytes, 0x7fffffff));
     const int64_t b_bytes = (int64_t)(p.n - (GATED ? 0 : n0)) * p.ldb;
     const QBufRsrc rsb = q_buffer_rsrc(p.b + (GATED ? 0 : (int64_t)n0 * p.ldb) + (int64_t)kt0 * 40,
                                        (uint32_t)std::min<int64_t>(b_bytes - (int64_t)kt0 * 40, 0x7fffffff));
@@ -2800,7 +2807,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
             }
         }
     };
-    for (int t = 0; t < kt; ++t) {
+    for (int t = 0; t < kf; ++t) {
         const uint8_t* st = ring + (t % NS) * kStage;
         // stage t+NS-1 into the slot read in step t-1
         const bool more = t + NS - 1 < kt;
@@ -2828,6 +2835,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
         __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+    }
+
+    if (half) {
+        const uint8_t* st = ring + (kf % NS) * kStage;
+        load_b(st, 0, fb0, fb1);
+        load_a(st, 0, fa0);
+        load_a(st, 1, fa1);
+        mfma_slice(fa0, fb0);
+        mfma_slice(fa1, fb1);
     }
 
     // C[m][n]: lane holds column n = (lane & 31) of fragment j, rows 8 (r / 4) + 4 (lane >> 5) + r % 4
@@ -3373,7 +3389,7 @@ inline size_t split_ws_bytes(const NnopsGemmQ41Args& g)
 // The blocks-along-K ring's conditions (f16 A; any M).
 inline bool ring_ok(const NnopsGemmQ41Args& g)
 {
-    return g.trans_b && !g.b_soa && g.a_f16 && g.k >= 64 && g.k % 64 == 0 && (g.lda % 8) == 0 &&
+    return g.trans_b && !g.b_soa && g.a_f16 && g.k >= 32 && g.k % 32 == 0 && (g.lda % 8) == 0 &&
            ((uintptr_t)g.a & 15) == 0;
 }
 
@@ -3407,7 +3423,7 @@ struct Q41RingPlan {
 inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
 {
     Q41RingPlan r;
-    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)(g.k / 64);
+    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)((g.k + 63) / 64);
     const float out_bytes = 4.0f * (float)m * (float)n;
     const uint32_t most = std::min({(uint32_t)max_splits, kt / 4, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)});
     for (const Q41RingTile& t : kQ41RingTiles) {
@@ -3443,7 +3459,7 @@ inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
 inline float gated_us(const NnopsGemmQ41Args& g, int bm)
 {
     const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n / 2 + 127) / 128);
-    const float steps = (float)(g.k / 64);
+    const float steps = (float)((g.k + 63) / 64);
     return (float)((tiles + 255) / 256) * (bm == 256 ? steps * 1.95f + 14.0f : steps * 1.17f + 6.0f);
 }
 
@@ -3556,7 +3572,7 @@ inline void run_q41_split(const NnopsGemmQ41Args& g, const Q41RingPlan& r, FpOut
     Q41Kern k = q41_kern(g);
     k.partial = static_cast<float*>(ws);
     k.splits = r.splits;
-    k.kt_per = (k.k / 64) / r.splits;
+    k.kt_per = ((k.k + 63) / 64) / r.splits;
     launch_q41_ring<QOUT_PART>(k, r, s);
     fo.src = k.partial;
     fo.ld_src = k.n;
@@ -3987,7 +4003,7 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
     }
     const bool pipe_gemv = g->m <= 2 && g->k == 128 * 32 && g->ldb_bytes == 128 * 20 && ((uintptr_t)g->b & 15) == 0 &&
                            (g->lda % 8) == 0 && ((uintptr_t)g->a & 15) == 0 && pass->gated && g->n % 2 == 0;
-    if (!pipe_gemv && (use_gemv(*g) || skinny_ok(*g) || g->k % 64 != 0 || (g->lda % 8) != 0 ||
+    if (!pipe_gemv && (use_gemv(*g) || skinny_ok(*g) || g->k % 32 != 0 || (g->lda % 8) != 0 ||
                        ((uintptr_t)g->a & 15) != 0)) {
         return NNOPS_UNSUPPORTED;
     }

@@ -11,17 +11,17 @@ namespace {
 struct RingTile {
     int bm, bn;
     float step_us;
-    bool narrow;        // has a form with 64-byte k steps (K % 128 != 0)
 };
 constexpr RingTile kRingTiles[] = {
-    {64, 64, 0.38f, true},    {128, 64, 0.48f, true},   {128, 128, 0.68f, true},  {192, 128, 0.82f, false},
-    {256, 128, 1.08f, true},  {128, 256, 1.08f, true},  {256, 256, 1.80f, true},
+    {64, 64, 0.38f},    {128, 64, 0.48f},   {128, 128, 0.68f},  {192, 128, 0.82f},
+    {256, 128, 1.08f},  {128, 256, 1.08f},  {256, 256, 1.80f},
 };
 
 }  // namespace
 
-// The ring kernel needs 64-byte k steps, 16-byte-aligned k-contiguous rows,
-// N % 4 == 0 (int32 groups), and 32-bit buffer offsets within a row panel.
+// The ring kernel needs K % 32 == 0 (bytes of k: whole matrix-core slices),
+// 16-byte-aligned k-contiguous rows and 32-bit buffer offsets within a row
+// panel.
 // The tile and the K split are the cheapest by
 //   rounds of 256 workgroups x k steps x the tile's step time
 //   + (partials: 3 us, and their bytes written and read at 3.5 TB/s),
@@ -38,7 +38,7 @@ constexpr RingTile kRingTiles[] = {
 // so the workspace) by those of one tile per CU. max_splits 1: no split, for
 // a workspace too small for the partials.
 // The fused output modes need row-uniform parameters, no zero-point terms,
-// half-away rounding, 16-byte-aligned tables and destination, and no split;
+// half-away rounding, N % 4 == 0, 16-byte-aligned tables and destination, and no split;
 // everything else writes raw partials and runs gemm_i8_reduce.
 // trb: B is the caller's [K,N] (row pitch ldb), read in place (its whole
 // span within 32-bit buffer offsets).
@@ -46,7 +46,7 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
                    int max_splits)
 {
     RingPlan r;
-    if (g.m < 1 || g.n < 4 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX || g.k < 64 || g.k % 64 != 0 || g.n % 4 != 0 || !aligned16(a, lda) || !aligned16(b, ldb)) {
+    if (g.m < 1 || g.n < 1 || g.m > INT32_MAX || g.n > INT32_MAX - 3 || g.k > INT32_MAX - 127 || g.k < 32 || g.k % 32 != 0 || !aligned16(a, lda) || !aligned16(b, ldb)) {
         return r;
     }
     if (trb && (g.k * ldb + g.n >= (int64_t)INT32_MAX || ldb < g.n)) {
@@ -60,7 +60,9 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
                        !g.round_even && !fp_out && tables16 && ((uintptr_t)g.c % 16 == 0);
     const size_t ebytes = g.out_kind == NNOPS_OUT_F16 ? 2 : 4;
     int fused = RING_PART;
-    if (fp_out && !compensate && (g.act == NNOPS_ACT_NONE || g.act == NNOPS_ACT_RELU) &&
+    if (g.n % 4 != 0) {
+        // raw partials
+    } else if (fp_out && !compensate && (g.act == NNOPS_ACT_NONE || g.act == NNOPS_ACT_RELU) &&
         (uintptr_t)g.c % 16 == 0 && (g.ldc * ebytes) % 16 == 0 &&
         ((uintptr_t)g.s_b % 16) == 0 && (g.bias_fp == nullptr || (uintptr_t)g.bias_fp % (4 * ebytes) == 0)) {
         fused = RING_FP;       // dequantizing output pass fused
@@ -71,24 +73,21 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
             fused = RING_S8;
         }
     }
-    const int bk = (g.k % 128 == 0) ? 128 : 64;
-    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)(g.k / bk);
+    const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)((g.k + 127) / 128);
     const float out_bytes = 4.0f * (float)m * (float)n;
-    const float step_scale = (float)bk / 128.0f;
-    const uint32_t most = std::min(16u, std::min(kt * (uint32_t)bk / 512u, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)));
+    const uint32_t most = std::min(16u, std::min(kt / 4u, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)));
     const int split_area = m <= 256 ? 256 * 128 : m <= 384 ? 192 * 128 : 256 * 256;
     float best = 0.0f;
     for (const RingTile& t : kRingTiles) {
-        if ((bk == 64 && !t.narrow) || t.bm * lda >= (int64_t)INT32_MAX ||
+        if (t.bm * lda >= (int64_t)INT32_MAX ||
             (!trb && t.bn * ldb >= (int64_t)INT32_MAX)) {
             continue;
         }
         const uint64_t tiles = (uint64_t)((m + t.bm - 1) / (uint32_t)t.bm) * ((n + t.bn - 1) / (uint32_t)t.bn);
-        const float step = t.step_us * step_scale;
         auto consider = [&](uint32_t sp, uint64_t rounds) {
             const uint32_t steps = kt - (sp - 1) * (kt / sp);       // the last split's, the longest
             const bool part = sp > 1 || fused == RING_PART;
-            const float us = (float)rounds * (float)steps * step +
+            const float us = (float)rounds * (float)steps * t.step_us +
                              (part ? 3.0f + 2.0f * (float)sp * out_bytes / 3.5e6f : 0.0f);
             if (r.bm == 0 || us < best) {
                 best = us;
@@ -111,7 +110,7 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
         }
     }
     if (r.bm != 0) {
-        r.bk = bk;
+        r.us = best;
         r.trb = trb;
     }
     return r;

@@ -27,6 +27,10 @@ TOL = 2e-3
 # (M, K, N): the tile and split that the plan takes
 SHAPES = [
     (3, 320, 100),          # fewer rows than a tile, K % 256 != 0
+    (5, 32, 40),            # one block of k in all
+    (48, 1696, 1000),       # half a stage last
+    (300, 4128, 260),       # the same, split
+    (1000, 96, 14080),      # 256 x 256
     (17, 256, 130),         # 32 x 128, unsplit (4 stages of k)
     (31, 4160, 1025),       # 32 x 128, 65 stages over the splits
     (33, 4096, 260),        # 64 x 128, split
@@ -103,7 +107,7 @@ def test_q4_1_ring_without_workspace(M):
     assert norm_err(host(c).astype(np.float32), want) <= TOL
 
 
-@pytest.mark.parametrize("M,K,n", [(300, 256, 14336), (512, 64, 16200)])
+@pytest.mark.parametrize("M,K,n", [(300, 256, 14336), (512, 96, 16200)])
 @pytest.mark.parametrize("kw", [dict(), dict(gate_limit=1.5), dict(add_to=True)])
 @pytest.mark.parametrize("f16", [True, False])
 def test_q4_1_gated_tall_tiles(M, K, n, kw, f16):

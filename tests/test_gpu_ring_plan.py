@@ -22,11 +22,17 @@ pytestmark = pytest.mark.gpu
 
 # (M, K, N): the tile that the shape's plan takes
 SHAPES = [
-    (17, 704, 68),          # 64 x 64, 64-byte k steps
+    (17, 704, 68),          # 64 x 64, half a stage last
     (63, 8192, 132),        # 64 x 64, K split
     (65, 4096, 260),        # 64 x 64 split, one row past a tile
     (500, 256, 4000),       # 128 x 64
-    (130, 4160, 1028),      # 64-byte k steps, split
+    (130, 4160, 1028),      # split, the last stage half as deep
+    (20, 32, 36),           # one slice of k in all
+    (65, 4128, 260),        # 32 k in the last stage, split
+    (333, 1120, 1024),      # 96 k in the last stage
+    (40, 8160, 257),        # split, N % 4 == 1
+    (200, 288, 4003),       # N % 4 == 3
+    (1000, 96, 16130),      # N % 4 == 2, 256 x 256
     (500, 256, 4100),       # 128 x 128, last tile 4 columns wide
     (300, 2048, 1024),      # split over several tiles of rows
     (384, 256, 16000),      # 192 x 128
@@ -68,7 +74,25 @@ def test_i8_tiles(M, K, N, trans_b, out):
         assert np.array_equal(got[r:r + 1].view(np.uint8), rows(r, r + 1).view(np.uint8)), r
 
 
-@pytest.mark.parametrize("M,K,N", [(3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
+@pytest.mark.parametrize("M,K,N", [(18, 224, 69), (70, 4128, 132), (300, 160, 1030)])
+@pytest.mark.parametrize("trans_b", [True, False])
+def test_u8_zero_points_short_stage(M, K, N, trans_b):
+    """u8 A (flipped in registers, not in the padding) and zero points over a
+    short last stage."""
+    announce(f"ring u8 {M}x{K}x{N} tb={trans_b}")
+    a = dg.ints(M, (M, K), 0, 255, np.uint8)
+    w = dg.ints(N, (N, K), -127, 127)
+    sb = dg.uniform(3, (N,), 0.001, 0.01)
+    zb = dg.ints(4, (N,), -3, 3, np.int32)
+    c = dev(np.zeros((M, N), np.int8))
+    na.gemm_i8(dev(a), dev(w if trans_b else np.ascontiguousarray(w.T)), c, trans_b=trans_b, out_kind=na.OUT_S8,
+               s_a=0.02, zp_a=117, s_b=dev(sb), zp_b=dev(zb), s_out=0.4, zp_out=3)
+    want = oracle.gemm_i8(a, w, trans_b=True, out_kind=oracle.OUT_S8, s_a=0.02, zp_a=117, s_b=sb, zp_b=zb, s_out=0.4,
+                          zp_out=3)
+    assert np.array_equal(host(c), want)
+
+
+@pytest.mark.parametrize("M,K,N", [(20, 48, 33), (130, 1040, 1001), (40, 8208, 78), (3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
                                    (500, 128, 4000), (500, 128, 4100), (384, 128, 16000)])
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("out_f16", [True, False])
