@@ -659,6 +659,28 @@ __global__ __launch_bounds__(256) void gemm_i8_reduce(GemmI8Kern p, RingSplit sk
     out4_store(p, o, nb, raw);
 }
 
+// round(gelu_tanh(x) / s_out), clamped, where a cheap evaluation settles it:
+// gelu(x) = x / (1 + 2^(-2 log2(e) c (x + 0.044715 x^3))) on the hardware's
+// exponential and reciprocal. With T = 1 + tanh its error against gelu_tanh's
+// T is below 5e-7 + 5e-7 T: the exponent's rounding moves T by at most 8e-8
+// (2 |a| e / (1 + e)^2 2^-23 over all e = 2^a), the exponential, the sum and the
+// reciprocal by 4e-7 T, and gelu_tanh's own tanh and sum are within 2.4e-7; the
+// products and the quotient add 3e-7 of the value. `sure` is set where the
+// quotient is further from the next rounding boundary (a half-integer, in
+// either rounding) than twice all of that, |x / s_out| (5e-7 + 8e-7 T); NaN and
+// overflow compare as not sure. A third of gelu_tanh's instructions.
+__device__ __forceinline__ float gelu_quotient(float x, float inv_out, bool& sure)
+{
+    const float x3 = __fmul_rn(__fmul_rn(__fmul_rn(0.044715f, x), x), x);
+    const float e = __builtin_amdgcn_exp2f((x + x3) * (-2.0f * 1.44269504f * 0.7978845608f));
+    const float r = __builtin_amdgcn_rcpf(1.0f + e);          // T / 2
+    const float z = x * inv_out;
+    const float y = z * r;
+    const float off = __builtin_fabsf(__builtin_amdgcn_fractf(__builtin_fabsf(y)) - 0.5f);
+    sure = off > __builtin_fabsf(z) * __builtin_fmaf(r, 16e-7f, 5e-7f);
+    return y;
+}
+
 // The same sum and output pass for s8 / u8 destinations with row-uniform
 // parameters (per-tensor s_a, s_out and zp_out, no zero-point terms, 16-byte
 // aligned tables, 4-byte aligned destination rows), with the activation,
@@ -705,6 +727,27 @@ __global__ __launch_bounds__(256) void gemm_i8_reduce_q(GemmI8Kern p, RingSplit 
             oldw = *reinterpret_cast<const uint32_t*>(c8);
         }
         uint32_t outw = 0;
+        if constexpr (FEP && ACT == NNOPS_ACT_GELU && !ADD) {
+            // the cheap evaluation, where it settles all four roundings
+            bool sure = true;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float f = __fmul_rn((float)(raw[e] + bias[e]), __fmul_rn(ep.s_a_scalar, sb[e]));
+                if (clip) {
+                    f = f < ep.min_clip ? ep.min_clip : f;
+                    f = ep.max_clip < f ? ep.max_clip : f;
+                }
+                bool s1;
+                const int32_t q = requant_clamped(gelu_quotient(f, inv_out, s1), ep.zp_out, u8, even);
+                outw |= ((uint32_t)q & 0xffu) << (8 * e);
+                sure = sure && s1;
+            }
+            if (sure) {
+                *reinterpret_cast<uint32_t*>(c8) = outw;
+                continue;
+            }
+            outw = 0;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             int32_t v = raw[e] + bias[e];

@@ -148,3 +148,25 @@ def test_i8_least_workspace():
     ws = torch.empty(least, dtype=torch.uint8, device="cuda")
     assert na.lib().nnops_hip_gemm_i8(C.byref(g), ws.data_ptr(), least, ops._stream_ptr(None)) == na.OK
     assert np.array_equal(host(c), oracle.gemm_i8(a, w, trans_b=True))
+
+
+@pytest.mark.parametrize("s_out", [0.031, 0.0007, 1.3])
+@pytest.mark.parametrize("even", [False, True])
+@pytest.mark.parametrize("clip", [False, True])
+def test_gelu_requant_dense(s_out, even, clip):
+    """GELU on an s8 destination over a dense range of accumulators (a bias per
+    column, 70 rows of different sums): bit for bit the oracle's, so every
+    value near a rounding boundary took the exact evaluation."""
+    announce(f"gelu dense s_out={s_out} even={even} clip={clip}")
+    M, K, N = 70, 128, 40000
+    a = np.zeros((M, K), np.int8)
+    a[:, 0] = np.arange(M)
+    w = dg.ints(1, (N, K), -127, 127)
+    bias = (np.arange(N, dtype=np.int32) - N // 2) * 7
+    sb = dg.uniform(2, (N,), 0.9, 1.1).astype(np.float32)
+    kw = dict(s_a=4.0e-5 * max(1.0, s_out * 10), s_out=s_out, zp_out=-3, float_ep=True, round_even=even,
+              min_clip=-1.5 if clip else -np.inf, max_clip=2.0 if clip else np.inf)
+    c = dev(np.zeros((M, N), np.int8))
+    na.gemm_i8(dev(a), dev(w), c, trans_b=True, out_kind=na.OUT_S8, bias=dev(bias), s_b=dev(sb), act=na.ACT_GELU, **kw)
+    want = oracle.gemm_i8(a, w, trans_b=True, out_kind=oracle.OUT_S8, bias=bias, s_b=sb, act=oracle.ACT_GELU, **kw)
+    assert np.array_equal(host(c), want)
