@@ -766,7 +766,7 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
         // so the stores are whole rows of the tile (BN bytes: whole 128-byte
         // lines) rather than each wave's TN-byte segments
         constexpr int kWholeP = BN + 16;
-        constexpr bool kWhole = BM * kWholeP <= NS * kStage && (BN % 128) == 0 && (BM * BN / 16) % (W * 64) == 0;
+        constexpr bool kWhole = BM * kWholeP <= NS * kStage && (BN % 64) == 0 && (BM * BN / 16) % (W * 64) == 0;
         constexpr int kSP = kWhole ? kWholeP : kPitch8;
         int8_t* stage8 = kWhole ? ring + wm0 * kSP + wn0 : ring + wave * (TM * kPitch8);
         // Two instructions per element are dropped where the parameters
@@ -975,7 +975,8 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
             int8_t* tile = ring + wave * (TM * 128);
             auto slab = [&](auto esz_c, auto clip_c, auto form_c) {
                 constexpr int ESZ = decltype(esz_c)::value;          // output element bytes
-                constexpr int SC = (TN < 128 / ESZ) ? TN : 128 / ESZ; // columns per slab
+                // columns per slab: 128 bytes of a row where they divide the wave tile
+                constexpr int SC = TN < 128 / ESZ ? TN : TN % (128 / ESZ) == 0 ? 128 / ESZ : 32;
                 constexpr int GPS = SC / 4;                          // 4-column entries per slab row
                 constexpr int E = 4 * ESZ;                           // entry bytes
                 constexpr int RB = GPS * E;                          // slab row bytes
@@ -1213,13 +1214,13 @@ void launch_ring_mode(const GemmI8Kern& k, const RingSplit& sk, int mode, bool f
 // 128-byte staged rows (whole cache lines: twice the bytes per L2 request of
 // 64-byte rows, which is what limits a CU's load rate). Three stage slots
 // where the LDS holds them (192x128 tiles: 33.7 -> 32.9 us against two), two
-// for the 256x256 tile, four for the tiles of 128 columns and rows or fewer;
+// for the 256x256 and 256x192 tiles, four for the tiles of 128 columns and rows or fewer;
 // the 64 x 64 tiles of small grids keep 8 stages in flight (their latency is
 // the call's).
 template <int BM, int BN, int WM, int WN, bool F16, bool TRB>
 void launch_ring_cfg(const GemmI8Kern& k, const RingSplit& sk, int mode, bool flip, hipStream_t s)
 {
-    constexpr int NS = BM + BN <= 128 ? 8 : BM + BN <= 256 ? 4 : BM + BN < 512 ? 3 : 2;
+    constexpr int NS = BM + BN <= 128 ? 8 : BM + BN <= 256 ? 4 : BM + BN <= 384 ? 3 : 2;
     if (k.k % 128 == 0) {
         launch_ring_mode<BM, BN, WM, WN, NS, F16, TRB, false>(k, sk, mode, flip, s);
     } else {
@@ -1241,6 +1242,14 @@ void launch_ring_tiles(const GemmI8Kern& k, const RingPlan& r, const RingSplit& 
         launch_ring_cfg<128, 128, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(192, 128)) {
         launch_ring_cfg<192, 128, 2, 4, F16, TRB>(k, sk, r.mode, flip, s);
+    } else if (is(128, 192) && !TRB) {
+        if constexpr (!TRB) {          // (a TRB stage row is a power of two)
+            launch_ring_cfg<128, 192, 4, 2, F16, TRB>(k, sk, r.mode, flip, s);
+        }
+    } else if (is(256, 192) && !TRB) {
+        if constexpr (!TRB) {
+            launch_ring_cfg<256, 192, 4, 2, F16, TRB>(k, sk, r.mode, flip, s);
+        }
     } else if (is(256, 128)) {
         launch_ring_cfg<256, 128, 4, 2, F16, TRB>(k, sk, r.mode, flip, s);
     } else if (is(128, 256)) {

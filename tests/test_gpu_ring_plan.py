@@ -38,6 +38,8 @@ SHAPES = [
     (384, 256, 16000),      # 192 x 128
     (500, 128, 16100),      # 256 x 128
     (640, 128, 11776),      # 128 x 256
+    (500, 128, 11004),      # 128 x 192
+    (1000, 96, 11008),      # 256 x 192
     (1000, 128, 16132),     # 256 x 256
 ]
 
@@ -93,7 +95,8 @@ def test_u8_zero_points_short_stage(M, K, N, trans_b):
 
 
 @pytest.mark.parametrize("M,K,N", [(20, 48, 33), (130, 1040, 1001), (40, 8208, 78), (3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
-                                   (500, 128, 4000), (500, 128, 4100), (384, 128, 16000)])
+                                   (500, 128, 4000), (500, 128, 4100), (384, 128, 16000), (500, 64, 11004),
+                                   (1000, 48, 11000)])
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("out_f16", [True, False])
 def test_f16_tiles(M, K, N, trans_b, out_f16):
