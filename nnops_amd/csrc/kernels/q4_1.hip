@@ -2642,8 +2642,11 @@ __device__ __forceinline__ v8h decode8_f16(uint32_t lo0, uint32_t lo1, v2h d2, v
 // running with the matrix cores idle; the gated form saves the larger
 // staging.) 512 x 2 x 14336 x 4096: 173 us on 128-row tiles with a branching
 // combine, 161 with the straight-line one, 139 on 256-row tiles.
-template <int OUT, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
+// TAIL: K % 64 == 32. (A form of its own: with the last stage's code in every
+// kernel the K loop's schedule lost 2 %, 495 x 11008 x 11008 171 -> 174.5 us.)
+template <int OUT, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256,
+          bool TAIL = false>
+__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
 {
     static_assert(!GATED || (BN == 256 && WN % 2 == 0), "gated: 128 gate and 128 value rows of the weight per tile");
     static_assert(!SPLIT || (!GATED && WM == 1), "split A: one wave row");
@@ -2679,14 +2682,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
     const int wm0 = (wave / WN) * TM;
     // this split's stages of 64 k
     const int kt0 = OUT == QOUT_PART ? sp * p.kt_per : 0;
-    const int kt = OUT == QOUT_PART && sp < p.splits - 1 ? p.kt_per : (p.k + 63) / 64 - kt0;
-    // K % 64 == 32: the last stage holds one block of k (its staging reads on
+    const int kt = OUT == QOUT_PART && sp < p.splits - 1 ? p.kt_per : (p.k + (TAIL ? 63 : 0)) / 64 - kt0;
+    // TAIL: the last stage holds one block of k (its staging reads on
     // into the next row, or 0 past the operand's end; unused)
-    const bool half = p.k % 64 != 0 && kt0 + kt == (p.k + 63) / 64;
+    const bool half = TAIL && kt0 + kt == (p.k + 63) / 64;
     const int kf = half ? kt - 1 : kt;
 
     // A: rows 8 * (4 * wave + i) + lane / 8; B raw: rows 16 * (4 * wave + i) + lane / 4
-    const int64_t a_bytes = SPLIT ? 0x7fffffff
+    const int64_t a_bytes = !TAIL ? 0x7fffffff
                                   : ((int64_t)(min(BM, p.m - m0) - 1) * p.lda + p.k - (int64_t)kt0 * 64) * 2;
     const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda + (int64_t)kt0 * 64,
                                        (uint32_t)std::min<int64_t>(a_bytes, 0x7fffffff));
@@ -2837,7 +2840,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_q4_1_ring(Q41Kern p)
         asm volatile("" ::: "memory");
     }
 
-    if (half) {
+    if (TAIL && half) {
         const uint8_t* st = ring + (kf % NS) * kStage;
         load_b(st, 0, fb0, fb1);
         load_a(st, 0, fa0);
@@ -3512,29 +3515,39 @@ inline void launch_skinny(const Q41Kern& k, bool a_f16, hipStream_t s)
     }
 }
 
-template <int OUT>
-void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
+template <int OUT, bool TAIL>
+void launch_q41_tiles(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
 {
     const int64_t tiles = (int64_t)((k.m + r.bm - 1) / r.bm) * ((k.n + r.bn - 1) / r.bn);
     const dim3 grid((unsigned)(tiles * r.splits));
     if (r.bn == 128) {
         if (r.bm == 32) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 32, 128>), grid, dim3(256), 0, s, k);
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 32, 128, TAIL>), grid, dim3(256), 0, s, k);
         } else if (r.bm == 64) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 64, 128>), grid, dim3(256), 0, s, k);
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 64, 128, TAIL>), grid, dim3(256), 0, s, k);
         } else if (r.bm == 96) {
-            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 96, 128>), grid, dim3(256), 0, s, k);
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 4, false, false, 96, 128, TAIL>), grid, dim3(256), 0, s, k);
         } else {
-            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 1, 4, false, false, 128, 128>), grid, dim3(256), 0, s, k);
+            NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 1, 4, false, false, 128, 128, TAIL>), grid, dim3(256), 0, s, k);
         }
     } else if (r.bm == 64) {
-        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8, false, false, 64, 256>), grid, dim3(512), 0, s, k);
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8, false, false, 64, 256, TAIL>), grid, dim3(512), 0, s, k);
     } else if (r.bm == 256) {
-        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 2, 4, false, false, 256, 256>), grid, dim3(512), 0, s, k);
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 3, 2, 4, false, false, 256, 256, TAIL>), grid, dim3(512), 0, s, k);
     } else {
         // 8 waves (2 per SIMD), each 128 x 32: one wave's decode and stalls
         // overlap the other's matrix-core work, and no B row is decoded twice
-        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8>), grid, dim3(512), 0, s, k);
+        NNOPS_LAUNCH((gemm_q4_1_ring<OUT, 4, 1, 8, false, false, 128, 256, TAIL>), grid, dim3(512), 0, s, k);
+    }
+}
+
+template <int OUT>
+void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
+{
+    if (k.k % 64 == 0) {
+        launch_q41_tiles<OUT, false>(k, r, s);
+    } else {
+        launch_q41_tiles<OUT, true>(k, r, s);
     }
 }
 
@@ -4051,12 +4064,21 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
         }
         return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
     }
+    const bool tail = g->k % 64 != 0;
     if (gated_tall(*g)) {
-        const unsigned tiles = (unsigned)(((g->m + 255) / 256) * ((pass->n + 127) / 128));
-        NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 3, 2, 4, true, false, 256, 256>), dim3(tiles), dim3(512), 0, s, k);
+        const dim3 grid((unsigned)(((g->m + 255) / 256) * ((pass->n + 127) / 128)));
+        if (tail) {
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 3, 2, 4, true, false, 256, 256, true>), grid, dim3(512), 0, s, k);
+        } else {
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 3, 2, 4, true, false, 256, 256>), grid, dim3(512), 0, s, k);
+        }
     } else {
-        const unsigned tiles = (unsigned)(((g->m + 127) / 128) * ((pass->n + 127) / 128));
-        NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true>), dim3(tiles), dim3(512), 0, s, k);
+        const dim3 grid((unsigned)(((g->m + 127) / 128) * ((pass->n + 127) / 128)));
+        if (tail) {
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true, false, 128, 256, true>), grid, dim3(512), 0, s, k);
+        } else {
+            NNOPS_LAUNCH((gemm_q4_1_ring<QOUT_F32, 4, 1, 8, true>), grid, dim3(512), 0, s, k);
+        }
     }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
 }
