@@ -211,7 +211,7 @@ def run_cfg2(args, torch, dg, na, stream):
         "roofline": {"bound": "mfma", "achieved": k_tops, "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
                      "frac": k_tops / PEAK_INT8_TOPS, "traffic": measured_traffic("gemm_i8_ring_cfg2"),
                      "launch_us": t["launch_ms"] * 1e3,
-                     "kernel": "gemm_i8_ring<256,256,2,4,BK=128,NS=2,RING_S8>", "algorithmic_ops_per_launch": ops,
+                     "kernel": "gemm_i8_ring<256,256,2,4,NS=2,RING_S8>", "algorithmic_ops_per_launch": ops,
                      "algorithmic_bytes_per_launch": float(M * K + N * K + M * N + N * 8)},
         "dtype": "int8 (s32 accumulate)",
     }

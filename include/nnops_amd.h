@@ -226,6 +226,8 @@ typedef struct NnopsGemmQ41Args {
     int64_t ldb_dm;
 } NnopsGemmQ41Args;
 
+/* The workspace of a call. Where it is room for K splits only (f16 A, blocks
+ * along K), a call given less runs unsplit. */
 size_t nnops_hip_gemm_q4_1_workspace_size(const NnopsGemmQ41Args* args);
 int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* args, void* workspace, size_t workspace_bytes,
                         void* stream);
@@ -239,8 +241,9 @@ int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* args, void* workspace, size_t wo
  * bias, beta, residual and epilogue are the output pass below.
  * A [M][lda], B [N][ldb] (trans_b) or [K][ldb], C [M][ldc]; pitches in
  * elements. The workspace holds K-split partials (small M, [K][N] B), a
- * transposed [K][N] f16 B and the ring GEMM's split partials (large f16
- * shapes): nnops_hip_gemm_fp_workspace_size bytes, 16-byte aligned. */
+ * transposed [K][N] f16 B and the ring GEMM's split partials (f16):
+ * nnops_hip_gemm_fp_workspace_size bytes, 16-byte aligned; given less, a call
+ * whose product needs no K split or copy runs without. */
 typedef struct NnopsGemmFpArgs {
     const void* a;
     const void* b;
@@ -311,7 +314,7 @@ int nnops_hip_fp_output_pass(const NnopsFpOutArgs* args, void* stream);
  * with the same operations and rounding as nnops_hip_gemm_q4_1 into f32
  * followed by nnops_hip_fp_output_pass (nnops' Linear write-back,
  * src/backend/cpu/matmul/linear.cpp:74-170,233-282). Taken by the gated
- * form on the blocks-along-K ring route (trans_b, f16 A, K % 64 == 0,
+ * form on the blocks-along-K ring route (trans_b, f16 A, K % 32 == 0,
  * 16-byte A rows, M past the GEMV and skinny shapes), where it saves the
  * f32 staging of both halves; NNOPS_UNSUPPORTED otherwise (the plain pass
  * included: in the write-back it costs more than its staging), with nothing

@@ -3331,9 +3331,9 @@ inline bool use_gemv(const NnopsGemmQ41Args& g)
 // The blocks-along-N ring: f16 A with 16-byte rows, K % 64 == 0, 16-byte B
 // rows, and every stage offset within a buffer resource's 31-bit range
 // The skinny MFMA GEMM (gemv_q4_1_skinny): blocks along K, f16 A with 16-byte
-// rows, 3 <= M <= 48 (launches of 16 rows), K % 256 == 0, 16-byte weight rows,
-// 32-bit offsets. At K = 4096, N = 14336 a launch takes 16 us, the ring 58-62
-// us for any M <= 128: past three launches the ring is the faster.
+// rows, 3 <= M <= 48 (launches of 16 rows; with f16 A past 16 rows only where
+// the ring's K splits have no workspace), K % 256 == 0, 16-byte weight rows,
+// 32-bit offsets. At K = 4096, N = 14336 a launch takes 13 us.
 constexpr int64_t kSkinnyMaxM = 48;
 
 inline bool skinny_ok(const NnopsGemmQ41Args& g)
