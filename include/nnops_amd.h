@@ -357,6 +357,25 @@ typedef struct NnopsQdqArgs {
 int nnops_hip_quantize_linear(const NnopsQdqArgs* args, void* stream);
 int nnops_hip_dequantize_linear(const NnopsQdqArgs* args, void* stream);
 
+/* What the kernel selection of a call comes to (no counterpart in nnops; for
+ * tests and for callers that tune shapes). Host code: the arguments' pointers
+ * are looked at for their alignment only, and nothing is launched. */
+typedef struct NnopsGemmPlan {
+    int32_t tile_m, tile_n;     /* output tile of the LDS-ring GEMM; 0: another kernel takes the call */
+    int32_t splits;             /* K splits (0: the other kernel's own) */
+    int32_t fused;              /* the GEMM writes the destination itself (else partials and a pass) */
+    int32_t short_stage;        /* K ends in a stage shorter than the ring's */
+    int32_t in_place;           /* int8: a [K,N] B read where it lies */
+} NnopsGemmPlan;
+
+/* pass: the product alone, or a product whose output pass follows (Linear:
+ * plain or gated). */
+#define NNOPS_PLAN_NO_PASS 0
+#define NNOPS_PLAN_PASS 1
+#define NNOPS_PLAN_GATED_PASS 2
+int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* args, int32_t pass, size_t workspace_bytes,
+                             NnopsGemmPlan* plan);
+
 /* Library version and build target, for the caller's diagnostics. */
 const char* nnops_hip_build_info(void);
 

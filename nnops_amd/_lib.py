@@ -125,6 +125,14 @@ class FpOutArgs(C.Structure):
     ]
 
 
+class GemmPlan(C.Structure):
+    _fields_ = [("tile_m", C.c_int32), ("tile_n", C.c_int32), ("splits", C.c_int32), ("fused", C.c_int32),
+                ("short_stage", C.c_int32), ("in_place", C.c_int32)]
+
+
+PLAN_NO_PASS, PLAN_PASS, PLAN_GATED_PASS = range(3)
+
+
 # Every symbol the two headers declare, with its ctypes signature.
 SIGNATURES = {
     "nnops_hip_gemm_i8_workspace_size": (C.c_size_t, [C.POINTER(GemmI8Args)]),
@@ -132,6 +140,7 @@ SIGNATURES = {
     "nnops_hip_gemm_i8_noalloc": (C.c_int, [C.POINTER(GemmI8Args), C.c_void_p]),
     "nnops_hip_gemm_q4_1_workspace_size": (C.c_size_t, [C.POINTER(GemmQ41Args)]),
     "nnops_hip_gemm_q4_1": (C.c_int, [C.POINTER(GemmQ41Args), C.c_void_p, C.c_size_t, C.c_void_p]),
+    "nnops_hip_gemm_q4_1_plan": (C.c_int, [C.POINTER(GemmQ41Args), C.c_int32, C.c_size_t, C.POINTER(GemmPlan)]),
     "nnops_hip_gemm_fp_workspace_size": (C.c_size_t, [C.POINTER(GemmFpArgs)]),
     "nnops_hip_gemm_fp": (C.c_int, [C.POINTER(GemmFpArgs), C.c_void_p, C.c_size_t, C.c_void_p]),
     "nnops_hip_fp_output_pass": (C.c_int, [C.POINTER(FpOutArgs), C.c_void_p]),

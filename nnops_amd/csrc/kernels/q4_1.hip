@@ -41,6 +41,7 @@
 
 
 #include <atomic>
+#include <cmath>
 #include <utility>
 
 namespace nnops_amd {
@@ -3410,7 +3411,18 @@ constexpr Q41RingTile kQ41RingTiles[] = {
     {256, 256, 1.95f},
 };
 
-// The tile and K split of a call and what it is estimated to take.
+// Whether every staging offset of a tile of bm rows of A and bn rows of B stays
+// below 2^31: the kernel forms them in 32 bits, and its descriptors end there,
+// so that rows further on would read 0.
+inline bool q41_tile_fits(const NnopsGemmQ41Args& g, int64_t bm, int64_t bn)
+{
+    const int64_t stages = (g.k + 63) / 64;
+    return (std::min(bm, g.m) - 1) * g.lda * 2 + stages * 128 < INT32_MAX &&
+           (std::min(bn, g.n) - 1) * g.ldb_bytes + stages * 40 + 24 < INT32_MAX;
+}
+
+// The tile and K split of a call and what it is estimated to take (bm 0: no
+// tile of the ring takes the call's row pitches).
 struct Q41RingPlan {
     int bm = 0, bn = 0, splits = 1;
     float us = 0.0f;
@@ -3430,6 +3442,9 @@ inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
     const float out_bytes = 4.0f * (float)m * (float)n;
     const uint32_t most = std::min({(uint32_t)max_splits, kt / 4, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)});
     for (const Q41RingTile& t : kQ41RingTiles) {
+        if (!q41_tile_fits(g, t.bm, t.bn)) {
+            continue;
+        }
         const uint64_t tiles = (uint64_t)((m + t.bm - 1) / (uint32_t)t.bm) * ((n + t.bn - 1) / (uint32_t)t.bn);
         const bool pairs = t.bn == 128;
         auto consider = [&](uint32_t sp) {
@@ -3458,9 +3473,13 @@ inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
 // The fused gated tiles' time: 128 or 256 rows x 128 outputs, one workgroup per
 // CU, and the combine. At 2 x 14336 x 4096 the tall tiles take 512 rows in one
 // round (139 us, 161 in the 128-row tiles' two), 256 rows or fewer the low
-// ones (85 against 113 us).
+// ones (85 against 113 us). Infinite where the tile's offsets do not fit (its
+// weight rows, N / 2 apart, are the fused entry's own check).
 inline float gated_us(const NnopsGemmQ41Args& g, int bm)
 {
+    if (!q41_tile_fits(g, bm, 1)) {
+        return INFINITY;
+    }
     const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n / 2 + 127) / 128);
     const float steps = (float)((g.k + 63) / 64);
     return (float)((tiles + 255) / 256) * (bm == 256 ? steps * 1.95f + 14.0f : steps * 1.17f + 6.0f);
@@ -3558,6 +3577,58 @@ void launch_q41_ring(const Q41Kern& k, const Q41RingPlan& r, hipStream_t s)
 inline bool ring_splits(const NnopsGemmQ41Args& g)
 {
     return ring_ok(g) && (g.m > 16 || (g.m > 2 && g.k % 256 != 0));
+}
+
+// The ring's plan of a call with ws_bytes of workspace: its K splits, or
+// without room for them no split. starved: few rows go to the skinny kernel
+// where it takes them, since the ring may not split or fits no tile.
+inline Q41RingPlan choose_q41_ring(const NnopsGemmQ41Args& g, size_t ws_bytes, bool& starved)
+{
+    Q41RingPlan r;
+    starved = !ring_splits(g);
+    if (ring_ok(g) && g.m > 2) {
+        r = plan_q41_ring(g, starved ? 1 : 16);
+        if (q41_ring_bytes(g, r) > ws_bytes) {
+            r = plan_q41_ring(g, 1);
+            starved = true;
+        }
+        starved = starved || r.bm == 0;
+    }
+    return r;
+}
+
+// How the output pass's call runs: the skinny kernel's or the ring's partials
+// (r) summed by the pass, or neither (the fused gated tiles, or the product
+// and then the pass).
+enum class Q41PassRoute { none, skinny, ring };
+inline Q41PassRoute q41_pass_route(const NnopsGemmQ41Args& g, bool gated, size_t ws_bytes, Q41RingPlan& r)
+{
+    if (const size_t skinny = skinny_bytes(g); skinny > 0) {
+        return skinny <= ws_bytes ? Q41PassRoute::skinny : Q41PassRoute::none;
+    }
+    if (!ring_splits(g)) {
+        return Q41PassRoute::none;
+    }
+    r = plan_q41_ring(g, 16);
+    if (r.bm == 0 || (r.splits == 1 && !gated) || q41_ring_bytes(g, r) > ws_bytes) {
+        return Q41PassRoute::none;
+    }
+    if (gated) {
+        // the gated form's fused tiles where they are the faster
+        const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
+        if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
+            return Q41PassRoute::none;
+        }
+    }
+    return Q41PassRoute::ring;
+}
+
+// Whether the fused gated tiles take a call (what nnops_hip_gemm_q4_1_fused
+// checks of the product).
+inline bool gated_ring_ok(const NnopsGemmQ41Args& g)
+{
+    return ring_ok(g) && !use_gemv(g) && !skinny_ok(g) && g.n * g.ldb_bytes < INT32_MAX &&
+           std::isfinite(gated_us(g, 128));
 }
 
 // The kernel arguments of a checked call.
@@ -3705,16 +3776,8 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
     if (workspace == nullptr || ((uintptr_t)workspace & 15) != 0) {
         ws_bytes = 0;            // (below: room for the ring's partials, 16-byte vectors)
     }
-    // the ring's plan: its K splits, or without room for them no split
-    Q41RingPlan ring;
-    bool starved = !ring_splits(*g);
-    if (ring_ok(*g) && g->m > 2) {
-        ring = plan_q41_ring(*g, starved ? 1 : 16);
-        if (q41_ring_bytes(*g, ring) > ws_bytes) {
-            ring = plan_q41_ring(*g, 1);
-            starved = true;
-        }
-    }
+    bool starved;
+    const Q41RingPlan ring = choose_q41_ring(*g, ws_bytes, starved);
     const Q41Kern k = q41_kern(*g);
     const bool soa = g->b_soa != 0;
 
@@ -3960,25 +4023,9 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
         ((uintptr_t)g.b & 3) || workspace == nullptr || ((uintptr_t)workspace & 15) != 0 || pass.src == nullptr) {
         return NNOPS_UNSUPPORTED;
     }
-    const size_t skinny = skinny_bytes(g);
     Q41RingPlan r;
-    if (skinny == 0) {
-        if (!ring_splits(g)) {
-            return NNOPS_UNSUPPORTED;
-        }
-        r = plan_q41_ring(g, 16);
-        if (r.splits == 1 && !pass.gated) {
-            return NNOPS_UNSUPPORTED;
-        }
-        // the gated form's fused tiles where they are the faster
-        if (pass.gated) {
-            const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
-            if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
-                return NNOPS_UNSUPPORTED;
-            }
-        }
-    }
-    if (std::max(skinny, q41_ring_bytes(g, r)) > ws_bytes) {
+    const Q41PassRoute route = q41_pass_route(g, pass.gated != 0, ws_bytes, r);
+    if (route == Q41PassRoute::none) {
         return NNOPS_UNSUPPORTED;
     }
     FpOut fo;
@@ -3991,13 +4038,53 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
     if ((pass.n + 1023) / 1024 * pass.rows > INT32_MAX) {
         return NNOPS_UNSUPPORTED;
     }
-    if (skinny > 0) {
+    if (route == Q41PassRoute::skinny) {
         run_skinny_split(g, fo, workspace, stream);
     } else {
         // an unsplit product (gated) goes where the caller's pass reads it
         run_q41_split(g, r, fo, r.splits > 1 ? workspace : const_cast<float*>(pass.src), stream);
     }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
+}
+
+extern "C" int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* g, int32_t pass, size_t ws_bytes, NnopsGemmPlan* out)
+{
+    if (g == nullptr || out == nullptr || g->m <= 0 || g->n <= 0 || g->k <= 0 || g->m > INT32_MAX ||
+        g->n > INT32_MAX || g->k > INT32_MAX) {
+        return NNOPS_INVALID_ARGUMENT;
+    }
+    *out = NnopsGemmPlan{};
+    bool starved;
+    Q41RingPlan r;
+    if (pass != NNOPS_PLAN_NO_PASS && g->trans_b && g->m > 2) {
+        const Q41PassRoute route = q41_pass_route(*g, pass == NNOPS_PLAN_GATED_PASS, ws_bytes, r);
+        if (route == Q41PassRoute::skinny) {
+            out->splits = skinny_split(*g);
+            return NNOPS_OK;
+        }
+        if (route == Q41PassRoute::none) {
+            r = Q41RingPlan{};
+            if (pass == NNOPS_PLAN_GATED_PASS && g->n % 2 == 0 && gated_ring_ok(*g)) {
+                r.bm = gated_tall(*g) ? 256 : 128;
+                r.bn = 256;
+                out->fused = 1;
+            }
+        }
+    }
+    if (r.bm == 0) {
+        r = choose_q41_ring(*g, ws_bytes, starved);
+        const size_t skinny = skinny_bytes(*g);
+        if (r.splits == 1 && ((skinny > 0 && skinny <= ws_bytes) || (skinny_ok(*g) && starved))) {
+            out->splits = skinny > 0 && skinny <= ws_bytes ? skinny_split(*g) : 1;
+            return NNOPS_OK;
+        }
+        out->fused = r.bm > 0 && r.splits == 1;
+    }
+    out->tile_m = r.bm;
+    out->tile_n = r.bn;
+    out->splits = r.splits;
+    out->short_stage = r.bm > 0 && g->k % 64 != 0;
+    return NNOPS_OK;
 }
 
 extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsFpOutArgs* pass, void* stream)
@@ -4016,8 +4103,7 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
     }
     const bool pipe_gemv = g->m <= 2 && g->k == 128 * 32 && g->ldb_bytes == 128 * 20 && ((uintptr_t)g->b & 15) == 0 &&
                            (g->lda % 8) == 0 && ((uintptr_t)g->a & 15) == 0 && pass->gated && g->n % 2 == 0;
-    if (!pipe_gemv && (use_gemv(*g) || skinny_ok(*g) || g->k % 32 != 0 || (g->lda % 8) != 0 ||
-                       ((uintptr_t)g->a & 15) != 0)) {
+    if (!pipe_gemv && (use_gemv(*g) || skinny_ok(*g) || !ring_ok(*g))) {
         return NNOPS_UNSUPPORTED;
     }
     FpOut fo;
@@ -4032,8 +4118,9 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
     if (!pass->gated) {
         return NNOPS_UNSUPPORTED;
     }
-    // the gated tile addresses both halves of the weight from its start
-    if (pass->gated && g->n * g->ldb_bytes >= INT32_MAX) {
+    // the gated tile addresses both halves of the weight from its start, and
+    // its rows of A from the first of them
+    if (g->n * g->ldb_bytes >= INT32_MAX || (!pipe_gemv && !gated_ring_ok(*g))) {
         return NNOPS_UNSUPPORTED;
     }
     Q41Kern k{};

@@ -177,3 +177,25 @@ def test_q4_1_skinny_splits(M, K, N, bias):
     assert na.Linear(output_dtype=na.DT_F16).compute([na.tensor(y)], ins) == na.OK
     want = oracle.q4_1_linear(x, blk, N, w_round_f16=True, out_f16=True, bias=b if bias else None).astype(np.float32)
     assert norm_err(host(y).astype(np.float32), want) <= TOL
+
+
+@pytest.mark.parametrize("lda", [8388608, 16777216])
+@pytest.mark.parametrize("gated", [True, False])
+def test_q4_1_wide_row_pitch(lda, gated):
+    """Rows of A millions of elements apart (the last token of many sequences,
+    as a slice): the same bits as from packed rows, which the same sums over K
+    give on any unsplit tile. 256-row tiles would pass 2^31 here."""
+    import torch
+    M, K, N = 300, 512, 28672
+    announce(f"q4_1 row pitch {lda} gated={gated}")
+    x, blk = dev(dg.normal(M, (M, K)).astype(np.float16)), dev(dg.q4_1_blocks(N, N, K))
+    wide = torch.empty(M * lda, dtype=torch.float16, device="cuda").view(M, lda)[:, :K]
+    wide.copy_(x)
+    outs = []
+    for a in (x, wide):
+        y = torch.zeros((M, N // 2 if gated else N), dtype=torch.float16, device="cuda")
+        op = na.Linear(output_dtype=na.DT_F16, gated=gated, gate_activation=na.EP_SILU if gated else na.EP_NONE)
+        assert op.compute([na.tensor(y)], [na.tensor(a), na.tensor(blk, dtype=na.DT_Q4_1, shape=[N, K])]) == na.OK
+        outs.append(host(y))
+    assert np.abs(outs[0][-1].astype(np.float32)).max() > 0
+    assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))

@@ -1,0 +1,50 @@
+"""The kernel selection of the ring GEMMs (nnops_hip_gemm_*_plan), on the host:
+no call here reaches a kernel launch."""
+from __future__ import annotations
+
+import ctypes as C
+
+import pytest
+
+import nnops_amd as na
+from nnops_amd import _lib as L
+
+ALL = 1 << 62       # a workspace with room for any plan
+
+
+def q41_plan(M, K, N, pass_=L.PLAN_NO_PASS, ws=ALL, lda=None, ldb=None, a=0):
+    g = na.GemmQ41Args()
+    g.a, g.m, g.n, g.k = a, M, N, K
+    g.lda, g.ldc, g.ldb_bytes = lda or K, N, ldb or (K + 31) // 32 * 20
+    g.trans_b, g.a_f16, g.out_kind = 1, 1, na.OUT_F16
+    p = L.GemmPlan()
+    assert na.lib().nnops_hip_gemm_q4_1_plan(C.byref(g), pass_, ws, C.byref(p)) == na.OK
+    return p
+
+
+# pitches of the last token of M sequences, 4096 wide: up to 4096 tokens each
+@pytest.mark.parametrize("lda", [4096, 4194304, 4227136, 8388608, 8454144, 16777216, 33554432, 134217728])
+@pytest.mark.parametrize("M", [17, 130, 300, 512])
+@pytest.mark.parametrize("N,pass_", [(4096, L.PLAN_NO_PASS), (28672, L.PLAN_PASS), (28672, L.PLAN_GATED_PASS)])
+def test_q4_1_row_pitch(lda, M, N, pass_):
+    """Every offset of the planned tile's rows of A stays below 2^31 (the
+    kernel forms them in 32 bits): a wide pitch takes lower tiles, and past
+    the lowest one another kernel."""
+    p = q41_plan(M, 4096, N, pass_, lda=lda)
+    if p.tile_m:
+        assert (min(p.tile_m, M) - 1) * lda * 2 + 4096 * 2 < 2**31
+    assert p.tile_m or lda > 16777216
+
+
+def test_q4_1_row_pitch_keeps_the_tall_tile():
+    """512 rows of a gated product: the 256-row tiles where their offsets fit,
+    else the 128-row ones."""
+    tiles = [q41_plan(512, 4096, 28672, L.PLAN_GATED_PASS, lda=lda) for lda in (4096, 4194304, 8388608)]
+    assert [t.tile_m for t in tiles] == [256, 256, 128]
+    assert all(t.fused for t in tiles)
+
+
+@pytest.mark.parametrize("ldb", [2560, 8388608, 16777216, 134217728])
+def test_q4_1_weight_pitch(ldb):
+    p = q41_plan(300, 4096, 300, ldb=ldb)
+    assert p.tile_m == 0 or (min(p.tile_n, 300) - 1) * ldb + 2560 < 2**31
