@@ -368,11 +368,12 @@ typedef struct NnopsGemmPlan {
     int32_t in_place;           /* int8: a [K,N] B read where it lies */
 } NnopsGemmPlan;
 
-/* pass: the product alone, or a product whose output pass follows (Linear:
+/* Q4_1's pass: the product alone, or a product whose output pass follows (Linear:
  * plain or gated). */
 #define NNOPS_PLAN_NO_PASS 0
 #define NNOPS_PLAN_PASS 1
 #define NNOPS_PLAN_GATED_PASS 2
+int nnops_hip_gemm_i8_plan(const NnopsGemmI8Args* args, size_t workspace_bytes, NnopsGemmPlan* plan);
 int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* args, int32_t pass, size_t workspace_bytes,
                              NnopsGemmPlan* plan);
 

@@ -1768,6 +1768,16 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
     return w;
 }
 
+// The plan that a call with ws_bytes of workspace runs on.
+WsPlan choose_plan(const NnopsGemmI8Args& g, size_t ws_bytes)
+{
+    WsPlan w = plan_workspace(g);
+    if (ws_bytes < w.total) {
+        w = plan_workspace(g, true);
+    }
+    return w;
+}
+
 template <int BM, int BN, int WM, int WN, int WPE, bool FULLK, bool ALIGNED>
 void launch_gemm_epi(const GemmI8Kern& k, int epi, hipStream_t s)
 {
@@ -1977,6 +1987,25 @@ extern "C" size_t nnops_hip_gemm_i8_workspace_size(const NnopsGemmI8Args* g)
     return plan_workspace(*g).total;
 }
 
+extern "C" int nnops_hip_gemm_i8_plan(const NnopsGemmI8Args* g, size_t ws_bytes, NnopsGemmPlan* out)
+{
+    if (g == nullptr || out == nullptr || g->m <= 0 || g->n <= 0 || g->k <= 0 || g->k > 65535 || g->m > INT32_MAX ||
+        g->n > INT32_MAX) {
+        return NNOPS_INVALID_ARGUMENT;
+    }
+    *out = NnopsGemmPlan{};
+    const WsPlan w = choose_plan(*g, ws_bytes);
+    if (w.kn.cpl == 0 && w.ring.mode >= 0) {
+        out->tile_m = w.ring.bm;
+        out->tile_n = w.ring.bn;
+        out->splits = w.ring.splits;
+        out->fused = w.ring.mode != RING_PART;
+        out->short_stage = g->k % 128 != 0;
+        out->in_place = w.ring.trb;
+    }
+    return NNOPS_OK;
+}
+
 size_t nnops_amd::gemm_i8_least_workspace(const NnopsGemmI8Args& g)
 {
     return plan_workspace(g, ring_optional(g)).total;
@@ -2017,10 +2046,7 @@ extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size
     if (g->lda < min_lda || g->ldb < min_ldb || g->ldc < g->n) {
         return NNOPS_INVALID_ARGUMENT;
     }
-    WsPlan w = plan_workspace(*g);
-    if (ws_bytes < w.total) {
-        w = plan_workspace(*g, true);
-    }
+    const WsPlan w = choose_plan(*g, ws_bytes);
     if (w.total > 0 && (workspace == nullptr || ws_bytes < w.total)) {
         return NNOPS_NOT_INITIALIZED;
     }

@@ -399,10 +399,12 @@ void gemm_i8_ring(GemmI8Kern p, RingSplit sk)
     // They end at the last row's last k.
     const int a_end = (min(BM, p.m - m0) - 1) * (int)p.lda + p.k - kt0 * BK;
     const BufRsrc rsa = buffer_rsrc(p.a + (int64_t)m0 * p.lda + (int64_t)kt0 * BK, a_end);
-    // TRB: the descriptor ends at B's last byte, so chunks past column N of
-    // the last k row read 0 (earlier rows' read the next row: never stored)
+    // TRB: the descriptor ends with the dword of B's last byte, so chunks past
+    // column N of the last k row read 0 (earlier rows' read the next row: never
+    // stored). Whole dwords: the range check makes one that is only partly in
+    // range 0, N % 4 valid columns with it (ldb and B are multiples of 16).
     const BufRsrc rsb = TRB ? buffer_rsrc(p.b + (int64_t)kt0 * BK * p.ldb + n0,
-                                          (int)((int64_t)(p.k - kt0 * BK - 1) * p.ldb + (p.n - n0)))
+                                          (int)((int64_t)(p.k - kt0 * BK - 1) * p.ldb + ceil_div(p.n - n0, 4) * 4))
                             : buffer_rsrc(p.b + (int64_t)n0 * p.ldb + (int64_t)kt0 * BK,
                                           (min(BN, p.n - n0) - 1) * (int)p.ldb + p.k - kt0 * BK);
     int a_off[QA], b_off[QB];

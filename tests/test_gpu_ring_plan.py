@@ -16,7 +16,8 @@ import oracle
 import datagen as dg
 import nnops_amd as na
 from nnops_amd import ops
-from gpu_util import dev, host, announce, norm_err
+from gpu_util import dev, host, announce, norm_err, oracle_rows, pitched
+from test_plan import i8_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -74,6 +75,24 @@ def test_i8_tiles(M, K, N, trans_b, out):
     edges = sorted({r for e in (0, 64, 128, 192, 256, 384, 512, M) for r in range(e - 2, e + 2) if 0 <= r < M})
     for r in edges:
         assert np.array_equal(got[r:r + 1].view(np.uint8), rows(r, r + 1).view(np.uint8)), r
+
+
+# [K,N] weights of odd width at a 16-byte pitch: read in place, the last k
+# row's last columns in a dword that N ends inside
+@pytest.mark.parametrize("M,K,N,tile_m", [(17, 768, 257, 64), (40, 1120, 1001, 64), (333, 4096, 1002, 64),
+                                          (500, 1152, 5002, 128), (700, 1056, 8001, 192), (1000, 416, 16001, 256)])
+def test_i8_in_place_odd_columns(M, K, N, tile_m):
+    announce(f"ring i8 in place {M}x{K}x{N}")
+    plan = i8_plan(M, K, N, trans_b=False, ldb=(N + 15) // 16 * 16, ldc=N, out_kind=na.OUT_S32)
+    assert plan.in_place and plan.tile_m == tile_m, plan.tile_m
+    a = dg.act_s8(M, (M, K))
+    w = dg.ints(N, (N, K), -127, 127)
+    b = pitched(np.ascontiguousarray(w.T), (N + 15) // 16 * 16)
+    c = dev(np.zeros((M, N), np.int32))
+    na.gemm_i8(dev(a), b, c, trans_b=False)
+    got = host(c)
+    want = oracle_rows(lambda r0, r1: oracle.gemm_i8(a[r0:r1], w, trans_b=True), M)
+    assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("M,K,N", [(18, 224, 69), (70, 4128, 132), (300, 160, 1030)])

@@ -22,6 +22,19 @@ def q41_plan(M, K, N, pass_=L.PLAN_NO_PASS, ws=ALL, lda=None, ldb=None, a=0):
     return p
 
 
+def i8_plan(M, K, N, ws=ALL, trans_b=True, ldb=None, ldc=None, b=0, **fields):
+    g = na.GemmI8Args()
+    g.b, g.m, g.n, g.k = b, M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b = K, ldb or (K if trans_b else N), ldc or N, int(trans_b)
+    g.out_kind, g.s_a_scalar, g.s_b_scalar, g.s_out = na.OUT_S8, 1.0, 1.0, 1.0
+    g.min_clip, g.max_clip = -float("inf"), float("inf")
+    for k, v in fields.items():
+        setattr(g, k, v)
+    p = L.GemmPlan()
+    assert na.lib().nnops_hip_gemm_i8_plan(C.byref(g), ws, C.byref(p)) == na.OK
+    return p
+
+
 # pitches of the last token of M sequences, 4096 wide: up to 4096 tokens each
 @pytest.mark.parametrize("lda", [4096, 4194304, 4227136, 8388608, 8454144, 16777216, 33554432, 134217728])
 @pytest.mark.parametrize("M", [17, 130, 300, 512])
