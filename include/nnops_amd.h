@@ -132,10 +132,10 @@ int nnops_hip_gemm_i8(const NnopsGemmI8Args* args, void* workspace, size_t works
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): the same kernels and results, with the workspace taken from a
  * fixed device array of NNOPS_HIP_NOALLOC_SCRATCH_BYTES that the library
- * holds on each GPU it runs on until the process ends. A call whose plan needs
- * more (nnops_hip_gemm_i8_workspace_size > the limit, e.g. a raw [K,N] B of
- * 64 MiB that is staged transposed) returns NNOPS_OUT_OF_MEMORY and enqueues
- * nothing. Calls on one GPU share the array: calls that may overlap on one
+ * holds on each GPU it runs on until the process ends. A call that needs more
+ * even with its K split no further than its row count's tile asks for (e.g. a
+ * raw [K,N] B of 64 MiB that is staged transposed) returns NNOPS_OUT_OF_MEMORY
+ * and enqueues nothing; any other takes as many K splits as the array holds. Calls on one GPU share the array: calls that may overlap on one
  * GPU (two streams, two threads) race. `stream` must belong to the current
  * device. Nothing is allocated, no host sync. */
 #define NNOPS_HIP_NOALLOC_SCRATCH_BYTES (64u << 20)
@@ -366,6 +366,7 @@ typedef struct NnopsGemmPlan {
     int32_t fused;              /* the GEMM writes the destination itself (else partials and a pass) */
     int32_t short_stage;        /* K ends in a stage shorter than the ring's */
     int32_t in_place;           /* int8: a [K,N] B read where it lies */
+    size_t workspace_bytes;     /* what it uses of the workspace */
 } NnopsGemmPlan;
 
 /* Q4_1's pass: the product alone, or a product whose output pass follows (Linear:

@@ -127,7 +127,7 @@ class FpOutArgs(C.Structure):
 
 class GemmPlan(C.Structure):
     _fields_ = [("tile_m", C.c_int32), ("tile_n", C.c_int32), ("splits", C.c_int32), ("fused", C.c_int32),
-                ("short_stage", C.c_int32), ("in_place", C.c_int32)]
+                ("short_stage", C.c_int32), ("in_place", C.c_int32), ("workspace_bytes", C.c_size_t)]
 
 
 PLAN_NO_PASS, PLAN_PASS, PLAN_GATED_PASS = range(3)

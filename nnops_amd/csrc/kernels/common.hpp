@@ -90,8 +90,8 @@ inline uint64_t next_launch_epoch()
 // ---------------------------------------------------------------------------
 // Epilogue parameters, resolved once on the host (device pointers only).
 // ---------------------------------------------------------------------------
-// The workspace nnops_hip_gemm_i8 asks of a call: that of its plan, or where
-// the ring is optional (gemm_i8.hip) that of the plan without it.
+// The workspace that is enough for a call of nnops_hip_gemm_i8: its plan's, or
+// that of the plan by its rows alone, whichever is less.
 size_t gemm_i8_least_workspace(const NnopsGemmI8Args& g);
 
 // The Q4_1 GEMM as K splits whose partials, in the workspace, the output pass

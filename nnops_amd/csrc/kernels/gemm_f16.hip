@@ -114,7 +114,7 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
         b = nullptr;          // the staged copy: 256-byte aligned, 128-byte rows
         ldb = f.kp;
     }
-    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb, false, lean ? 1 : 16);
+    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb, false, lean ? 1 : kMostSplits);
     if (f.ring.mode != RING_FP && f.ring.mode != RING_PART) {
         f.ring = RingPlan{};
         f.stage_b = false;

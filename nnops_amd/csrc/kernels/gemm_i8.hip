@@ -1709,9 +1709,15 @@ KnPlan plan_kn(const NnopsGemmI8Args& g)
 // rate: they run without the ring where the workspace has no room for it.
 inline bool ring_optional(const NnopsGemmI8Args& g) { return g.m < 64 || g.k % 64 != 0 || g.n % 4 != 0; }
 
-// lean: the plan for a workspace too small for the full one: no K split, and
-// no ring where it is optional.
-WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
+// How a call is planned: with as many K splits as `room` bytes hold, or by its
+// rows alone (plan_ring_by_rows), or without the ring.
+struct PlanFor {
+    size_t room = SIZE_MAX;
+    bool by_rows = false;
+    bool ring = true;
+};
+
+WsPlan plan_workspace(const NnopsGemmI8Args& g, const PlanFor& f = PlanFor{})
 {
     WsPlan w;
     size_t off = 0;
@@ -1741,10 +1747,13 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
     const bool need_rb = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0;
     // (from 17 rows: 24 x 11008 x 4096 s8 15.8 us on 64 x 64 tiles in four
     // splits, 52 us on gemm_i8_mfma's 64 workgroups of the whole K)
-    const bool ring = g.m > 16 && !(lean && ring_optional(g));
-    const int max_splits = lean ? 1 : 16;
+    const bool ring = g.m > 16 && f.ring;
+    auto plan = [&](bool trb) {
+        return f.by_rows ? plan_ring_by_rows(g, a, lda, b, ldb, trb, true)
+                         : plan_ring(g, a, lda, b, ldb, trb, std::max(1, splits_in(f.room, off, g.m, g.n)));
+    };
     if (!g.trans_b && !need_rb && ring) {
-        w.ring = plan_ring(g, a, lda, b, ldb, true, max_splits);
+        w.ring = plan(true);
     }
     if (!g.trans_b && w.ring.mode < 0) {
         w.b_t = off; off += align_up((size_t)g.n * (size_t)w.kp);
@@ -1752,12 +1761,12 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, bool lean = false)
         ldb = w.kp;
     }
     if (!w.ring.trb && ring) {
-        w.ring = plan_ring(g, a, lda, b, ldb, false, max_splits);
+        w.ring = plan(false);
     }
     // few rows that need the general output pass, over a short k: one launch of
     // gemm_i8_mfma (0.3 us per 64 bytes of k) before the ring and its reduce
     // (34 x 1024 x 677: 11.3 against 12.2 us)
-    if (w.ring.mode == RING_PART && !w.ring.trb && w.ring.splits == 1 && g.m < 64 &&
+    if (!f.by_rows && w.ring.mode == RING_PART && !w.ring.trb && w.ring.splits == 1 && g.m < 64 &&
         0.3f * (float)(g.k / 64) < w.ring.us) {
         w.ring = RingPlan{};
     }
@@ -1773,7 +1782,10 @@ WsPlan choose_plan(const NnopsGemmI8Args& g, size_t ws_bytes)
 {
     WsPlan w = plan_workspace(g);
     if (ws_bytes < w.total) {
-        w = plan_workspace(g, true);
+        w = plan_workspace(g, {.room = ws_bytes});
+        if (ws_bytes < w.total && ring_optional(g)) {
+            w = plan_workspace(g, {.ring = false});
+        }
     }
     return w;
 }
@@ -1995,6 +2007,7 @@ extern "C" int nnops_hip_gemm_i8_plan(const NnopsGemmI8Args* g, size_t ws_bytes,
     }
     *out = NnopsGemmPlan{};
     const WsPlan w = choose_plan(*g, ws_bytes);
+    out->workspace_bytes = w.total;
     if (w.kn.cpl == 0 && w.ring.mode >= 0) {
         out->tile_m = w.ring.bm;
         out->tile_n = w.ring.bn;
@@ -2008,7 +2021,7 @@ extern "C" int nnops_hip_gemm_i8_plan(const NnopsGemmI8Args* g, size_t ws_bytes,
 
 size_t nnops_amd::gemm_i8_least_workspace(const NnopsGemmI8Args& g)
 {
-    return plan_workspace(g, ring_optional(g)).total;
+    return std::min(plan_workspace(g).total, plan_workspace(g, {.by_rows = true}).total);
 }
 
 extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, void* stream)

@@ -65,7 +65,7 @@ extern "C" int nnops_hip_gemm_i8_noalloc(const NnopsGemmI8Args* args, void* stre
     }
     const size_t need = nnops_amd::gemm_i8_least_workspace(*args);
     if (need > kScratchBytes) {
-        return NNOPS_OUT_OF_MEMORY;   // the plan needs more than the fixed array holds
+        return NNOPS_OUT_OF_MEMORY;   // more than the fixed array holds
     }
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {

@@ -44,10 +44,24 @@ struct RingPlan {
     float us = 0.0f;        // the estimate it won by
 };
 
-// The ring plan of an int8 call (ring_plan.hip); an f16 call asks with its K and
-// row pitches in bytes.
+constexpr int kMostSplits = 16;     // K splits at most
+
+// The ring plan of an int8 call (ring_plan.hip), and the one by its rows alone;
+// an f16 call asks with its K and row pitches in bytes.
 RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, bool trb,
                    int max_splits);
+RingPlan plan_ring_by_rows(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
+                           bool trb, bool small_tiles);
+
+// How many splits' partials of an M x N output `room` bytes hold past `off`.
+inline int splits_in(size_t room, size_t off, int64_t m, int64_t n)
+{
+    if (room == SIZE_MAX) {
+        return kMostSplits;
+    }
+    const size_t slab = (size_t)m * (size_t)((n + 3) / 4) * 16;
+    return room <= off ? 0 : (int)std::min<size_t>(kMostSplits, (room - off) / 256 * 256 / slab);
+}
 
 inline bool aligned16(const void* p, int64_t ld) { return ((uintptr_t)p % 16 == 0) && (ld % 16 == 0); }
 

@@ -4060,6 +4060,7 @@ extern "C" int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* g, int32_t pass,
         const Q41PassRoute route = q41_pass_route(*g, pass == NNOPS_PLAN_GATED_PASS, ws_bytes, r);
         if (route == Q41PassRoute::skinny) {
             out->splits = skinny_split(*g);
+            out->workspace_bytes = skinny_bytes(*g);
             return NNOPS_OK;
         }
         if (route == Q41PassRoute::none) {
@@ -4076,6 +4077,7 @@ extern "C" int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* g, int32_t pass,
         const size_t skinny = skinny_bytes(*g);
         if (r.splits == 1 && ((skinny > 0 && skinny <= ws_bytes) || (skinny_ok(*g) && starved))) {
             out->splits = skinny > 0 && skinny <= ws_bytes ? skinny_split(*g) : 1;
+            out->workspace_bytes = out->splits > 1 ? skinny : 0;
             return NNOPS_OK;
         }
         out->fused = r.bm > 0 && r.splits == 1;
@@ -4084,6 +4086,7 @@ extern "C" int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* g, int32_t pass,
     out->tile_n = r.bn;
     out->splits = r.splits;
     out->short_stage = r.bm > 0 && g->k % 64 != 0;
+    out->workspace_bytes = r.bm > 0 ? q41_ring_bytes(*g, r) : least_workspace(*g);
     return NNOPS_OK;
 }
 

@@ -61,3 +61,31 @@ def test_q4_1_row_pitch_keeps_the_tall_tile():
 def test_q4_1_weight_pitch(ldb):
     p = q41_plan(300, 4096, 300, ldb=ldb)
     assert p.tile_m == 0 or (min(p.tile_n, 300) - 1) * ldb + 2560 < 2**31
+
+
+NOALLOC = 64 << 20
+
+
+@pytest.mark.parametrize("M", [77, 104, 128])
+@pytest.mark.parametrize("fields", [dict(a_u8=1), dict(zp_a_scalar=3), dict(a_u8=1, out_kind=na.OUT_S32)])
+def test_i8_splits_within_the_fixed_scratch(M, fields):
+    """A transposed copy that nearly fills the library's own 64 MiB: K splits
+    as far as the rest holds, where the full plan's partials do not fit."""
+    full, p = (i8_plan(M, 14336, 4096, ws, trans_b=False, **fields) for ws in (ALL, NOALLOC))
+    assert full.workspace_bytes > NOALLOC
+    assert p.tile_m > 0 and p.splits >= 2 and p.workspace_bytes <= NOALLOC
+
+
+@pytest.mark.parametrize("M", [24, 64, 128, 300, 512])
+@pytest.mark.parametrize("out", [na.OUT_S8, na.OUT_S32])
+def test_i8_splits_grow_with_the_workspace(M, out):
+    """Plans for less and less room fit into it, down to an unsplit one."""
+    full = i8_plan(M, 14336, 1024, out_kind=out)
+    assert full.splits > 1
+    seen = set()
+    for slabs in range(full.splits, 0, -1):
+        room = full.workspace_bytes - (full.splits - slabs) * M * 1024 * 4
+        p = i8_plan(M, 14336, 1024, room, out_kind=out)
+        assert p.tile_m > 0 and p.workspace_bytes <= room and p.splits <= slabs
+        seen.add(p.splits)
+    assert full.splits in seen and 1 in seen

@@ -126,3 +126,19 @@ def test_noalloc_rejects_a_plan_beyond_the_scratch():
     torch.cuda.synchronize()
     assert rc == na.OUT_OF_MEMORY
     assert bool((c == 7).all())
+
+
+@pytest.mark.parametrize("M", [77, 104, 128])
+def test_noalloc_splits_as_far_as_the_scratch_holds(M):
+    """A u8 A over a raw [K,N] weight whose transposed copy takes 58.7 MB of the
+    64: the splits of the full plan do not fit beside it, fewer do."""
+    import torch
+    announce(f"noalloc {M}x14336x4096 u8 [K,N]")
+    K, N = 14336, 4096
+    assert _need(M, N, K, False, a_u8=1, out_kind=na.OUT_S8, lda=K, ldb=N, ldc=N) > LIMIT
+    a = dev(dg.ints(541, (M, K), 0, 255, np.uint8))
+    b = dev(dg.ints(542, (K, N), -127, 127))
+    c0 = torch.zeros((M, N), dtype=torch.int8, device="cuda")
+    got, want = _pair(a, b, c0, trans_b=False, out_kind=na.OUT_S8, s_a=0.03, zp_a=128, s_b=0.001, s_out=1.5)
+    np.testing.assert_array_equal(got, want)
+    assert np.unique(want).size > 50
