@@ -18,8 +18,9 @@
  *   - nothing is allocated and nothing synchronises the host: work is enqueued
  *     on `stream` and the call returns;
  *   - `workspace` must hold at least the matching *_workspace_size() bytes
- *     (NNOPS_NOT_INITIALIZED otherwise) and must not be shared by calls that
- *     may run concurrently; its contents on entry are irrelevant;
+ *     (NNOPS_NOT_INITIALIZED otherwise, but where an entry point says what
+ *     it does with less) and must not be shared by calls that may run
+ *     concurrently; its contents on entry are irrelevant;
  *   - a rejected call returns a non-zero status and enqueues nothing.
  */
 #ifndef NNOPS_AMD_H
@@ -124,6 +125,10 @@ typedef struct NnopsGemmI8Args {
                                    or a u8 A needs them */
 } NnopsGemmI8Args;
 
+/* The workspace of a call. With less, a call of fewer than 64 rows, of K % 64 !=
+ * 0 or of N % 4 != 0 splits K less or runs without its ring kernel, and others
+ * split K less as long as the buffer holds the splits that their rows' tile
+ * asks for; below that NNOPS_NOT_INITIALIZED. */
 size_t nnops_hip_gemm_i8_workspace_size(const NnopsGemmI8Args* args);
 int nnops_hip_gemm_i8(const NnopsGemmI8Args* args, void* workspace, size_t workspace_bytes,
                       void* stream);
@@ -242,8 +247,9 @@ int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* args, void* workspace, size_t wo
  * A [M][lda], B [N][ldb] (trans_b) or [K][ldb], C [M][ldc]; pitches in
  * elements. The workspace holds K-split partials (small M, [K][N] B), a
  * transposed [K][N] f16 B and the ring GEMM's split partials (f16):
- * nnops_hip_gemm_fp_workspace_size bytes, 16-byte aligned; given less, a call
- * whose product needs no K split or copy runs without. */
+ * nnops_hip_gemm_fp_workspace_size bytes, 16-byte aligned. With less, f16 calls
+ * do as the int8 ones above (fewer than 64 rows, K % 32 != 0 or N % 4 != 0: none
+ * is needed). */
 typedef struct NnopsGemmFpArgs {
     const void* a;
     const void* b;
@@ -375,6 +381,7 @@ typedef struct NnopsGemmPlan {
 #define NNOPS_PLAN_PASS 1
 #define NNOPS_PLAN_GATED_PASS 2
 int nnops_hip_gemm_i8_plan(const NnopsGemmI8Args* args, size_t workspace_bytes, NnopsGemmPlan* plan);
+int nnops_hip_gemm_fp_plan(const NnopsGemmFpArgs* args, size_t workspace_bytes, NnopsGemmPlan* plan);
 int nnops_hip_gemm_q4_1_plan(const NnopsGemmQ41Args* args, int32_t pass, size_t workspace_bytes,
                              NnopsGemmPlan* plan);
 

@@ -141,6 +141,7 @@ SIGNATURES = {
     "nnops_hip_gemm_q4_1_workspace_size": (C.c_size_t, [C.POINTER(GemmQ41Args)]),
     "nnops_hip_gemm_q4_1": (C.c_int, [C.POINTER(GemmQ41Args), C.c_void_p, C.c_size_t, C.c_void_p]),
     "nnops_hip_gemm_i8_plan": (C.c_int, [C.POINTER(GemmI8Args), C.c_size_t, C.POINTER(GemmPlan)]),
+    "nnops_hip_gemm_fp_plan": (C.c_int, [C.POINTER(GemmFpArgs), C.c_size_t, C.POINTER(GemmPlan)]),
     "nnops_hip_gemm_q4_1_plan": (C.c_int, [C.POINTER(GemmQ41Args), C.c_int32, C.c_size_t, C.POINTER(GemmPlan)]),
     "nnops_hip_gemm_fp_workspace_size": (C.c_size_t, [C.POINTER(GemmFpArgs)]),
     "nnops_hip_gemm_fp": (C.c_int, [C.POINTER(GemmFpArgs), C.c_void_p, C.c_size_t, C.c_void_p]),

@@ -12,18 +12,14 @@
 #include "nnops/ops/matmul.hpp"
 #include "nnops_amd.h"
 
+#include "../kernels/entry.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <array>
 #include <cstring>
 #include <limits>
-
-namespace nnops_amd {
-// q4_1.hip: the K splits of a Q4_1 product, summed by its output pass.
-int gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace, size_t ws_bytes,
-                         hipStream_t stream);
-}  // namespace nnops_amd
 
 namespace nnops {
 namespace {
@@ -558,7 +554,7 @@ Status run_i8(const QuantCall& q, const Geometry& g, TensorView& out, const Tens
             xb.s_a = x.s_a != nullptr ? x.s_a + row_base : nullptr;
             xb.zp_a = x.zp_a != nullptr ? x.zp_a + row_base : nullptr;
         }
-        const int rc = nnops_hip_gemm_i8(&xb, ws, ws_left, stream);
+        const int rc = nnops_amd::gemm_i8_in(xb, ws, ws_left, stream);
         if (rc != NNOPS_OK) {
             return from_code(rc);
         }

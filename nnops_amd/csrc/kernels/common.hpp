@@ -11,6 +11,7 @@
 
 #include <atomic>
 
+#include "entry.hpp"
 #include "nnops_amd.h"
 
 namespace nnops_amd {
@@ -90,16 +91,6 @@ inline uint64_t next_launch_epoch()
 // ---------------------------------------------------------------------------
 // Epilogue parameters, resolved once on the host (device pointers only).
 // ---------------------------------------------------------------------------
-// The workspace that is enough for a call of nnops_hip_gemm_i8: its plan's, or
-// that of the plan by its rows alone, whichever is less.
-size_t gemm_i8_least_workspace(const NnopsGemmI8Args& g);
-
-// The Q4_1 GEMM as K splits whose partials, in the workspace, the output pass
-// sums (one launch and one staging fewer than the product and then the pass);
-// NNOPS_UNSUPPORTED, nothing launched, where another route is the call's.
-int gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace, size_t ws_bytes,
-                         hipStream_t stream);
-
 struct EpiParams {
     const int32_t* bias;       // [N] int32 (integer outputs) or nullptr
     const int32_t* r_a;        // [M] sum_k A (true values), or nullptr

@@ -83,9 +83,9 @@ struct F16Plan {
 // From 3 rows over [N][K] rows of B (4096 x 4096: 3 rows 13.7 us against the
 // GEMV's 19.6, 16 rows 13.7 against 21.4; 2 rows stay with the GEMV, 9.7) and
 // from 17 over a [K][N] B, whose transposed copy the GEMV needs not (17 to 63
-// rows on gemm_fp_tile, in f32: 475 us). lean: the plan for a workspace too
-// small for the full one, without K splits.
-F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
+// rows on gemm_fp_tile, in f32: 475 us). room: the workspace that K splits may
+// use. by_rows: the plan by the call's rows alone, whose workspace is enough.
+F16Plan plan_f16(const NnopsGemmFpArgs& g, size_t room = SIZE_MAX, bool by_rows = false)
 {
     F16Plan f;
     if (!g.in_f16 || g.m < (g.trans_b ? 3 : 17) || 2 * g.k > INT32_MAX || g.m > INT32_MAX || g.n > INT32_MAX) {
@@ -114,7 +114,18 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
         b = nullptr;          // the staged copy: 256-byte aligned, 128-byte rows
         ldb = f.kp;
     }
-    f.ring = plan_ring(x, static_cast<const int8_t*>(g.a), x.lda, b, ldb, false, lean ? 1 : kMostSplits);
+    const int8_t* a = static_cast<const int8_t*>(g.a);
+    if (by_rows) {
+        f.ring = plan_ring_by_rows(x, a, x.lda, b, ldb, false, false);
+        // (128 x 256 tiles that nearly fill the CUs: no split)
+        if (f.ring.splits > 1 && g.m > 128 && ((g.m + 127) / 128) * ((g.n + 255) / 256) >= 192 &&
+            (uintptr_t)g.c % 16 == 0 && (g.ldc * (g.out_f16 ? 2 : 4)) % 16 == 0) {
+            f.ring.splits = 1;
+            f.ring.mode = RING_FP;
+        }
+    } else {
+        f.ring = plan_ring(x, a, x.lda, b, ldb, false, std::max(1, splits_in(room, off, g.m, g.n)));
+    }
     if (f.ring.mode != RING_FP && f.ring.mode != RING_PART) {
         f.ring = RingPlan{};
         f.stage_b = false;
@@ -128,34 +139,66 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, bool lean = false)
     return f;
 }
 
+// The plan that a call with ws_bytes of workspace runs on (if that holds it).
+F16Plan choose_f16(const NnopsGemmFpArgs& g, size_t ws_bytes)
+{
+    const F16Plan f = plan_f16(g);
+    return ws_bytes < f.total ? plan_f16(g, ws_bytes) : f;
+}
+
+// The plan's workspace. The destination's alignment (which a size query may not
+// see) picks between the fused output and the split partials: room for either.
+size_t f16_workspace(const NnopsGemmFpArgs& g, bool by_rows)
+{
+    NnopsGemmFpArgs x = g;
+    const size_t a = plan_f16(x, SIZE_MAX, by_rows).total;
+    x.c = reinterpret_cast<void*>(uintptr_t{2});
+    return std::max(a, plan_f16(x, SIZE_MAX, by_rows).total);
+}
+
+// Shapes that the GEMV and the tile kernel take without a workspace.
+inline bool ring_f16_optional(const NnopsGemmFpArgs& g) { return g.m < 64 || g.k % 32 != 0 || g.n % 4 != 0; }
+
 }  // namespace
 
 size_t ring_gemm_f16_workspace(const NnopsGemmFpArgs& g)
 {
-    // the destination's alignment (which a size query may not see) picks
-    // between the fused output and the split partials: room for either
-    NnopsGemmFpArgs x = g;
-    const size_t a = plan_f16(x).total;
-    x.c = reinterpret_cast<void*>(uintptr_t{2});
-    return std::max(a, plan_f16(x).total);
+    return f16_workspace(g, false);
+}
+
+extern "C" int nnops_hip_gemm_fp_plan(const NnopsGemmFpArgs* g, size_t ws_bytes, NnopsGemmPlan* out)
+{
+    if (g == nullptr || out == nullptr || g->m <= 0 || g->n <= 0 || g->k <= 0) {
+        return NNOPS_INVALID_ARGUMENT;
+    }
+    *out = NnopsGemmPlan{};
+    const F16Plan f = choose_f16(*g, ws_bytes);
+    if (f.ring.mode >= 0 && f.total <= ws_bytes) {
+        out->tile_m = f.ring.bm;
+        out->tile_n = f.ring.bn;
+        out->splits = f.ring.splits;
+        out->fused = f.ring.mode != RING_PART;
+        out->short_stage = 2 * g->k % 128 != 0;
+        out->workspace_bytes = f.total;
+    }
+    return NNOPS_OK;
 }
 
 int ring_gemm_f16(const NnopsGemmFpArgs& g, void* workspace, size_t ws_bytes, hipStream_t s)
 {
-    // shapes that the GEMV and the tile kernel take without a workspace
-    const bool optional = g.m < 64 || g.k % 32 != 0 || g.n % 4 != 0;
+    const bool optional = ring_f16_optional(g);
     if (workspace == nullptr || (optional && (uintptr_t)workspace % 16 != 0)) {
         ws_bytes = 0;
     }
-    F16Plan f = plan_f16(g);
-    if (ws_bytes < f.total) {
-        f = plan_f16(g, true);
-    }
+    const F16Plan f = choose_f16(g, ws_bytes);
     if (f.ring.mode < 0) {
         return NNOPS_UNSUPPORTED;
     }
     if (ws_bytes < f.total) {
         return optional ? NNOPS_UNSUPPORTED : NNOPS_NOT_INITIALIZED;
+    }
+    if (!optional && ws_bytes < f16_workspace(g, false) && ws_bytes < f16_workspace(g, true)) {
+        return NNOPS_NOT_INITIALIZED;       // less than the query's, and than is enough
     }
     if (!optional && (uintptr_t)workspace % 16 != 0) {
         return NNOPS_INVALID_ARGUMENT;   // staged operands and partials are 16-byte vectors

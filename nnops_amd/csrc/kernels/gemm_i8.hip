@@ -1641,6 +1641,7 @@ inline int kn_mt(int64_t m) { return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <=
 
 struct WsPlan {
     size_t r_a = 0, r_b = 0, a_t = 0, b_t = 0, part = 0, flag = 0, total = 0;
+    size_t full = 0;        // the total of the plan with all the room it would take (choose_plan)
     int64_t kp = 0;
     RingPlan ring;
     KnPlan kn;
@@ -1781,12 +1782,14 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, const PlanFor& f = PlanFor{})
 WsPlan choose_plan(const NnopsGemmI8Args& g, size_t ws_bytes)
 {
     WsPlan w = plan_workspace(g);
-    if (ws_bytes < w.total) {
+    const size_t full = w.total;
+    if (ws_bytes < full) {
         w = plan_workspace(g, {.room = ws_bytes});
         if (ws_bytes < w.total && ring_optional(g)) {
             w = plan_workspace(g, {.ring = false});
         }
     }
+    w.full = full;
     return w;
 }
 
@@ -2024,9 +2027,12 @@ size_t nnops_amd::gemm_i8_least_workspace(const NnopsGemmI8Args& g)
     return std::min(plan_workspace(g).total, plan_workspace(g, {.by_rows = true}).total);
 }
 
-extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, void* stream)
+namespace nnops_amd {
+namespace {
+
+// any_workspace: also with less than the least that the query's callers give.
+int run_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, hipStream_t s, bool any_workspace)
 {
-    const TimingDisarm disarm;
     if (g == nullptr || g->m < 0 || g->n < 0 || g->k < 0) {
         return NNOPS_INVALID_ARGUMENT;
     }
@@ -2060,13 +2066,15 @@ extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size
         return NNOPS_INVALID_ARGUMENT;
     }
     const WsPlan w = choose_plan(*g, ws_bytes);
+    if (!any_workspace && ws_bytes < w.full && ws_bytes < plan_workspace(*g, {.by_rows = true}).total) {
+        return NNOPS_NOT_INITIALIZED;
+    }
     if (w.total > 0 && (workspace == nullptr || ws_bytes < w.total)) {
         return NNOPS_NOT_INITIALIZED;
     }
     if ((uintptr_t)workspace % 16 != 0) {
         return NNOPS_INVALID_ARGUMENT;   // staged operands and partials are 16-byte vectors
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
     char* ws = static_cast<char*>(workspace);
 
     GemmI8Kern k{};
@@ -2193,4 +2201,20 @@ extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size
         launch_gemm<32, 64, 1, 2, 4>(k, aligned, fullk, epi, s);
     }
     return hipGetLastError() == hipSuccess ? NNOPS_OK : NNOPS_INTERNAL;
+}
+
+}  // namespace
+
+int gemm_i8_in(const NnopsGemmI8Args& g, void* workspace, size_t ws_bytes, hipStream_t stream)
+{
+    const TimingDisarm disarm;
+    return run_gemm_i8(&g, workspace, ws_bytes, stream, true);
+}
+
+}  // namespace nnops_amd
+
+extern "C" int nnops_hip_gemm_i8(const NnopsGemmI8Args* g, void* workspace, size_t ws_bytes, void* stream)
+{
+    const TimingDisarm disarm;
+    return run_gemm_i8(g, workspace, ws_bytes, static_cast<hipStream_t>(stream), false);
 }

@@ -89,3 +89,40 @@ def test_i8_splits_grow_with_the_workspace(M, out):
         assert p.tile_m > 0 and p.workspace_bytes <= room and p.splits <= slabs
         seen.add(p.splits)
     assert full.splits in seen and 1 in seen
+
+
+# A call whose workspace is too small is refused before any launch: the
+# pointers are never followed.
+FAR = 1 << 20
+
+
+def i8_call(ws, M, K, N, **fields):
+    g = na.GemmI8Args()
+    g.a, g.b, g.c, g.m, g.n, g.k = FAR, FAR, FAR, M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b, g.out_kind = K, K, N, 1, na.OUT_S8
+    g.s_a_scalar = g.s_b_scalar = g.s_out = 1.0
+    for k, v in fields.items():
+        setattr(g, k, v)
+    return g, na.lib().nnops_hip_gemm_i8(C.byref(g), FAR, ws, None)
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (128, 14336, 1024), (333, 14336, 4096), (512, 8192, 1024)])
+@pytest.mark.parametrize("fields", [dict(), dict(s_a=FAR), dict(trans_b=0, ldb=4096)])
+def test_i8_refuses_a_small_workspace(M, K, N, fields):
+    """Between the sums' room and what the splits of the rows' tile take."""
+    p = i8_plan(M, K, N, **fields)
+    assert p.splits > 1
+    sums = (M * 4 + 255) // 256 * 256 + (N * 4 + 255) // 256 * 256
+    for ws in (0, sums, sums + M * N * 4):
+        assert i8_call(ws, M, K, N, **fields)[1] == na.NOT_INITIALIZED
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 4096, 4096), (333, 8192, 4096), (512, 14336, 1024)])
+def test_f16_refuses_a_small_workspace(M, K, N):
+    g = na.GemmFpArgs()
+    g.a, g.b, g.c, g.m, g.n, g.k = FAR, FAR, FAR, M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b, g.in_f16, g.out_f16, g.alpha = K, K, N, 1, 1, 1, 1.0
+    need = na.lib().nnops_hip_gemm_fp_workspace_size(C.byref(g))
+    assert need >= M * N * 4
+    for ws in (0, M * N * 4 - 1):
+        assert na.lib().nnops_hip_gemm_fp(C.byref(g), FAR, ws, None) == na.NOT_INITIALIZED
