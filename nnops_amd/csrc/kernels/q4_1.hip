@@ -2694,7 +2694,9 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
                                   : ((int64_t)(min(BM, p.m - m0) - 1) * p.lda + p.k - (int64_t)kt0 * 64) * 2;
     const QBufRsrc rsa = q_buffer_rsrc(static_cast<const _Float16*>(p.a) + (int64_t)m0 * p.lda + (int64_t)kt0 * 64,
                                        (uint32_t)std::min<int64_t>(a_bytes, 0x7fffffff));
-    const int64_t b_bytes = (int64_t)(p.n - (GATED ? 0 : n0)) * p.ldb;
+    // ends with the last row's last block: a stage's 64 bytes of a row reach
+    // past its blocks, which at a wide pitch may be past the operand
+    const int64_t b_bytes = (int64_t)(p.n - 1 - (GATED ? 0 : n0)) * p.ldb + (int64_t)(p.k / 32) * 20;
     const QBufRsrc rsb = q_buffer_rsrc(p.b + (GATED ? 0 : (int64_t)n0 * p.ldb) + (int64_t)kt0 * 40,
                                        (uint32_t)std::min<int64_t>(b_bytes - (int64_t)kt0 * 40, 0x7fffffff));
     int a_off[QA], b_off[QB];

@@ -199,3 +199,24 @@ def test_q4_1_wide_row_pitch(lda, gated):
         outs.append(host(y))
     assert np.abs(outs[0][-1].astype(np.float32)).max() > 0
     assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))
+
+
+@pytest.mark.parametrize("M,K,N", [(20, 96, 40), (20, 320, 40), (130, 4128, 260), (300, 416, 1000)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_q4_1_weight_at_the_end_of_its_buffer(M, K, N, gated):
+    """A weight that is the right part of a wider buffer: its last row ends
+    where the allocation does, less than a stage's bytes past its last block.
+    The same bits as from the packed weight."""
+    import torch
+    announce(f"q4_1 end of buffer {M}x{K}x{N} gated={gated}")
+    x, blk = dev(dg.normal(M, (M, K)).astype(np.float16)), dev(dg.q4_1_blocks(N, N, K))
+    wide = torch.full((N, 48 + blk.shape[1]), 0x7b, dtype=torch.uint8, device="cuda")[:, 48:]
+    wide.copy_(blk)
+    outs = []
+    for w in (blk, wide):
+        y = torch.zeros((M, N // 2 if gated else N), dtype=torch.float16, device="cuda")
+        op = na.Linear(output_dtype=na.DT_F16, gated=gated, gate_activation=na.EP_SILU)
+        assert op.compute([na.tensor(y)], [na.tensor(x), na.tensor(w, dtype=na.DT_Q4_1, shape=[N, K])]) == na.OK
+        outs.append(host(y))
+    assert np.abs(outs[0].astype(np.float32)).max() > 0
+    assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))
