@@ -4019,7 +4019,6 @@ extern "C" int nnops_hip_gemm_q4_1(const NnopsGemmQ41Args* g, void* workspace, s
 int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutArgs& pass, void* workspace,
                                     size_t ws_bytes, hipStream_t stream)
 {
-    const TimingDisarm disarm;
     if (!g.trans_b || g.m <= 2 || g.n <= 0 || g.m > INT32_MAX || g.n > INT32_MAX || g.k > INT32_MAX ||
         g.a == nullptr || g.b == nullptr || g.lda < g.k || g.ldb_bytes < (g.k + 31) / 32 * 20 || (g.ldb_bytes & 3) ||
         ((uintptr_t)g.b & 3) || workspace == nullptr || ((uintptr_t)workspace & 15) != 0 || pass.src == nullptr) {
@@ -4030,6 +4029,8 @@ int nnops_amd::gemm_q4_1_split_pass(const NnopsGemmQ41Args& g, const NnopsFpOutA
     if (route == Q41PassRoute::none) {
         return NNOPS_UNSUPPORTED;
     }
+    // (a call that is left to another route leaves it armed timing events too)
+    const TimingDisarm disarm;
     FpOut fo;
     if (const int rc = make_fp_out(&pass, fo); rc != NNOPS_OK) {
         return rc;

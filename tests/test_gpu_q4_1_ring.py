@@ -220,3 +220,23 @@ def test_q4_1_weight_at_the_end_of_its_buffer(M, K, N, gated):
         outs.append(host(y))
     assert np.abs(outs[0].astype(np.float32)).max() > 0
     assert np.array_equal(outs[0].view(np.uint8), outs[1].view(np.uint8))
+
+
+@pytest.mark.parametrize("M,N", [(17, 4096), (512, 28672)])
+def test_q4_1_gated_linear_timed(M, N):
+    """Armed timing events reach the operator's first launch, on the route
+    whose partials the pass sums (17 rows) and on the fused tiles."""
+    import torch
+    announce(f"q4_1 timed gated M={M}")
+    K = 1024
+    x, blk = dev(dg.normal(M, (M, K)).astype(np.float16)), dev(dg.q4_1_blocks(N, N, K))
+    y = torch.zeros((M, N // 2), dtype=torch.float16, device="cuda")
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    e1.record()          # in this order their own span is not positive
+    e0.record()
+    torch.cuda.synchronize()
+    assert na.lib().nnops_hip_time_next_launch(C.c_void_p(e0.cuda_event), C.c_void_p(e1.cuda_event)) == na.OK
+    op = na.Linear(output_dtype=na.DT_F16, gated=True, gate_activation=na.EP_SILU)
+    assert op.compute([na.tensor(y)], [na.tensor(x), na.tensor(blk, dtype=na.DT_Q4_1, shape=[N, K])]) == na.OK
+    torch.cuda.synchronize()
+    assert e0.elapsed_time(e1) > 0.0
