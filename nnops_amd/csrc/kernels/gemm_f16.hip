@@ -80,15 +80,32 @@ struct F16Plan {
     size_t part_off = 0, total = 0;
 };
 
-// From 3 rows over [N][K] rows of B (4096 x 4096: 3 rows 13.7 us against the
-// GEMV's 19.6, 16 rows 13.7 against 21.4; 2 rows stay with the GEMV, 9.7) and
-// from 17 over a [K][N] B, whose transposed copy the GEMV needs not (17 to 63
+// Few rows over [N][K] rows of B that the GEMV is the faster for: 1 and 2, and
+// 3 and 4 (one pass of it) over a short k or a long one with many columns. GEMV
+// against ring, us, weights in the cache and from HBM:
+//   2 x 4096 x 4096            9.7 / 13.7
+//   3 x 512 x 1000      4.6 /  5.9    4.6 /  5.9
+//   3 x 1024 x 1024     5.3 /  6.0    7.1 /  6.7
+//   3 x 1536 x 100      5.8 /  6.5    5.8 /  6.4
+//   3 x 1792 x 4096                  12.5 /  9.6
+//   3 x 4096 x 4096    13.1 / 12.3   19.3 / 14.9
+//   3 x 1536 x 14336   12.5 / 11.8   16.4 / 13.4
+//   3 x 8192 x 11008                 48.2 / 46.5
+//   3 x 8192 x 14336   41.0 / 40.9   53.6 / 57.9
+inline bool gemv_f16_faster(const NnopsGemmFpArgs& g)
+{
+    return g.m < 3 || (g.m <= 4 && ((g.k < 1792 && g.n <= 8192) || (g.k >= 8192 && g.n > 11008)));
+}
+
+// From 3 rows over [N][K] rows of B (4096 x 4096: 16 rows 13.7 us against the
+// GEMV's 21.4) and from 17 over a [K][N] B, whose transposed copy the GEMV needs not (17 to 63
 // rows on gemm_fp_tile, in f32: 475 us). room: the workspace that K splits may
 // use. by_rows: the plan by the call's rows alone, whose workspace is enough.
 F16Plan plan_f16(const NnopsGemmFpArgs& g, size_t room = SIZE_MAX, bool by_rows = false)
 {
     F16Plan f;
-    if (!g.in_f16 || g.m < (g.trans_b ? 3 : 17) || 2 * g.k > INT32_MAX || g.m > INT32_MAX || g.n > INT32_MAX) {
+    if (!g.in_f16 || (g.trans_b ? gemv_f16_faster(g) : g.m < 17) || 2 * g.k > INT32_MAX || g.m > INT32_MAX ||
+        g.n > INT32_MAX) {
         return f;
     }
     NnopsGemmI8Args x{};
@@ -126,7 +143,11 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, size_t room = SIZE_MAX, bool by_rows 
     } else {
         f.ring = plan_ring(x, a, x.lda, b, ldb, false, std::max(1, splits_in(room, off, g.m, g.n)));
     }
-    if (f.ring.mode != RING_FP && f.ring.mode != RING_PART) {
+    // up to 8 rows, two passes of the GEMV, over a k too short to split and with
+    // a destination that needs the pass over partials (5 x 768 x 1001: GEMV 7.2
+    // us, ring and pass 8.0)
+    const bool short_pass = g.trans_b && g.m <= 8 && g.k < 1024 && f.ring.mode == RING_PART;
+    if (short_pass || (f.ring.mode != RING_FP && f.ring.mode != RING_PART)) {
         f.ring = RingPlan{};
         f.stage_b = false;
         return f;

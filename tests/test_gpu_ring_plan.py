@@ -113,7 +113,7 @@ def test_u8_zero_points_short_stage(M, K, N, trans_b):
     assert np.array_equal(host(c), want)
 
 
-@pytest.mark.parametrize("M,K,N", [(20, 48, 33), (130, 1040, 1001), (40, 8208, 78), (3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
+@pytest.mark.parametrize("M,K,N", [(3, 512, 100), (4, 1792, 260), (8, 768, 1001), (20, 48, 33), (130, 1040, 1001), (40, 8208, 78), (3, 4096, 68), (16, 96, 40), (17, 1024, 132), (40, 11008, 260), (64, 4096, 1024),
                                    (500, 128, 4000), (500, 128, 4100), (384, 128, 16000), (500, 64, 11004),
                                    (1000, 48, 11000)])
 @pytest.mark.parametrize("trans_b", [True, False])

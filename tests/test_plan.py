@@ -35,6 +35,15 @@ def i8_plan(M, K, N, ws=ALL, trans_b=True, ldb=None, ldc=None, b=0, **fields):
     return p
 
 
+def f16_plan(M, K, N, ws=ALL, trans_b=True, c=0):
+    g = na.GemmFpArgs()
+    g.c, g.m, g.n, g.k = c, M, N, K
+    g.lda, g.ldb, g.ldc, g.trans_b, g.in_f16, g.out_f16, g.alpha = K, K if trans_b else N, N, int(trans_b), 1, 1, 1.0
+    p = L.GemmPlan()
+    assert na.lib().nnops_hip_gemm_fp_plan(C.byref(g), ws, C.byref(p)) == na.OK
+    return p
+
+
 # pitches of the last token of M sequences, 4096 wide: up to 4096 tokens each
 @pytest.mark.parametrize("lda", [4096, 4194304, 4227136, 8388608, 8454144, 16777216, 33554432, 134217728])
 @pytest.mark.parametrize("M", [17, 130, 300, 512])
@@ -126,3 +135,12 @@ def test_f16_refuses_a_small_workspace(M, K, N):
     assert need >= M * N * 4
     for ws in (0, M * N * 4 - 1):
         assert na.lib().nnops_hip_gemm_fp(C.byref(g), FAR, ws, None) == na.NOT_INITIALIZED
+
+
+@pytest.mark.parametrize("M,K,N,ring", [
+    (2, 4096, 4096, False), (3, 512, 1000, False), (4, 1024, 4096, False), (3, 1776, 8192, False), (4, 1792, 4096, True),
+    (3, 1536, 14336, True), (4, 4096, 4096, True), (3, 8192, 8192, True), (4, 8192, 14336, False),
+    (5, 512, 1024, True), (5, 512, 100, False), (8, 768, 1001, False), (9, 768, 1001, True), (8, 4096, 1001, True)])
+def test_f16_few_rows(M, K, N, ring):
+    """Where the GEMV is the faster, a call of few rows does not take the ring."""
+    assert (f16_plan(M, K, N).tile_m > 0) == ring
