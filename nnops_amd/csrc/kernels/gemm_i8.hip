@@ -1764,11 +1764,17 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, const PlanFor& f = PlanFor{})
     if (!w.ring.trb && ring) {
         w.ring = plan(false);
     }
-    // few rows that need the general output pass, over a short k: one launch of
-    // gemm_i8_mfma (0.3 us per 64 bytes of k) before the ring and its reduce
-    // (34 x 1024 x 677: 11.3 against 12.2 us)
-    if (!f.by_rows && w.ring.mode == RING_PART && !w.ring.trb && w.ring.splits == 1 && g.m < 64 &&
-        0.3f * (float)(g.k / 64) < w.ring.us) {
+    // few rows over a short k, B's rows k-contiguous: gemm_i8_mfma before the
+    // ring, where the general output pass is needed (one launch, 0.3 us per 64
+    // bytes of k, before the ring and its reduce: 34 x 1024 x 677 11.3 against
+    // 12.2 us) and where an integer destination is written without a split (us,
+    // gemm_i8_mfma / ring, s8: 17 x 256 x 1024 3.4 / 3.8, 17 x 384 x 4096 4.4 /
+    // 4.5, 17 x 512 x 4096 5.2 / 5.0, 48 x 768 x 1024 5.0 / 5.2, 17 x 1024 x 1024
+    // 6.8 / 6.1; an f16 one 17 x 256 x 1024 8.2 / 4.3)
+    const bool short_k = w.ring.mode == RING_PART
+                             ? w.ring.splits == 1 && 0.3f * (float)(g.k / 64) < w.ring.us
+                             : w.ring.mode != RING_FP && (g.k <= 384 || (g.k < 1024 && g.n <= 1024));
+    if (!f.by_rows && !w.ring.trb && g.m < 64 && short_k) {
         w.ring = RingPlan{};
     }
     if (w.ring.mode == RING_PART) {

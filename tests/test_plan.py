@@ -144,3 +144,14 @@ def test_f16_refuses_a_small_workspace(M, K, N):
 def test_f16_few_rows(M, K, N, ring):
     """Where the GEMV is the faster, a call of few rows does not take the ring."""
     assert (f16_plan(M, K, N).tile_m > 0) == ring
+
+
+@pytest.mark.parametrize("M,K,N,kind,ring", [
+    (17, 256, 1024, na.OUT_S8, False), (63, 384, 4096, na.OUT_S32, False), (17, 448, 4096, na.OUT_S8, True),
+    (48, 960, 1024, na.OUT_S8, False), (48, 1024, 1024, na.OUT_S8, True), (64, 256, 1024, na.OUT_S8, True),
+    (17, 256, 1024, na.OUT_F16, True), (17, 256, 1024, na.OUT_F32, True)])
+def test_i8_few_rows_short_k(M, K, N, kind, ring):
+    """Where gemm_i8_mfma is the faster, few rows do not take the ring; over a
+    [K,N] B, which it would have to copy, they do."""
+    assert (i8_plan(M, K, N, out_kind=kind).tile_m > 0) == ring
+    assert i8_plan(M, K, N, out_kind=kind, trans_b=False).in_place
