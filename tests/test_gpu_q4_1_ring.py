@@ -1,7 +1,9 @@
 """The blocks-along-K Q4_1 ring at the sizes where its plan changes: every
-tile shape with ragged edges, K splits whose last one is longer, row counts
-just past the skinny kernel, the output pass over the splits' partials (plain
-and gated), and calls without a workspace.
+tile shape with ragged edges, whole and split over K, with whole and short last
+stages, K splits whose last one is longer, row counts just past the skinny
+kernel, the output pass over the splits' partials (plain and gated), and calls
+without a workspace. plan_cases.py has the shapes whose tile counts, held to the
+plan by test_plan.py.
 
 Bar: the Q4_1 tolerance (2e-3, normalized), against the oracle with weights
 decoded to f16 (the decode's rounding, 2^-12 of a weight, is in both; an f32
@@ -18,34 +20,37 @@ import oracle
 import datagen as dg
 import nnops_amd as na
 from nnops_amd import ops
+import plan_cases as pc
 from gpu_util import dev, host, announce, norm_err, oracle_rows
+from test_plan import q41_plan, L
 
 pytestmark = pytest.mark.gpu
 
 TOL = 2e-3
 
-# (M, K, N): the tile and split that the plan takes
+# (M, K, N): the tile and the K splits that the plan takes
 SHAPES = [
-    (3, 320, 100),          # fewer rows than a tile, K % 256 != 0
-    (5, 32, 40),            # one block of k in all
-    (48, 1696, 1000),       # half a stage last
-    (300, 4128, 260),       # the same, split
+    (3, 320, 100),          # 32 x 128, fewer rows than a tile, K % 256 != 0
+    (5, 32, 40),            # 32 x 128, one block of k in all
+    (48, 1696, 1000),       # 32 x 128 in 6, half a stage last
+    (300, 4128, 260),       # the same in 8
     (1000, 96, 14080),      # 256 x 256
     (17, 256, 130),         # 32 x 128, unsplit (4 stages of k)
-    (31, 4160, 1025),       # 32 x 128, 65 stages over the splits
-    (33, 4096, 260),        # 64 x 128, split
-    (77, 4096, 1024),       # 96 x 128, split
-    (97, 1088, 516),        # 17 stages, two tiles of rows
-    (128, 14336, 256),
-    (130, 512, 8192),       # 64 x 256
-    (300, 4096, 300),
-    (260, 256, 28700),      # 128 x 256
+    (31, 4160, 1025),       # 32 x 128, 65 stages over 16 splits
+    (33, 4096, 260),        # 32 x 128 in 16, one row past a tile
+    (77, 4096, 1024),       # 32 x 128 in 8
+    (77, 4096, 4096),       # 96 x 128 in 8
+    (97, 1088, 516),        # 32 x 128, 17 stages over 4 splits, four tiles of rows
+    (128, 14336, 256),      # 32 x 128 in 16
+    (130, 512, 8192),       # 64 x 128
+    (300, 4096, 300),       # 32 x 128 in 8
+    (260, 256, 28700),      # 96 x 128
 ]
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
 @pytest.mark.parametrize("out_f16", [True, False])
-def test_q4_1_ring_tiles(M, K, N, out_f16):
+def test_q4_1_ring_shapes(M, K, N, out_f16):
     import torch
     announce(f"q4_1 ring {M}x{K}x{N} f16={out_f16}")
     x = dg.normal(M + K, (M, K)).astype(np.float16)
@@ -57,6 +62,25 @@ def test_q4_1_ring_tiles(M, K, N, out_f16):
     want = oracle_rows(lambda r0, r1: oracle.gemm_q4_1(x, blk, N, trans_b=True, rows=(r0, r1),
                                                        w_round_f16=True)[r0:r1], M, band=4)
     assert norm_err(got[:, :N], want) <= TOL
+
+
+# (the partials of a split do not depend on the destination's type)
+@pytest.mark.parametrize("M,K,N,want,splits,out_f16",
+                         [(*c, f16) for c in pc.Q41_TILES for f16 in ((True, False) if c[4] == 1 else (True,))])
+def test_q4_1_ring_tiles(M, K, N, want, splits, out_f16):
+    import torch
+    announce(f"q4_1 ring tile {M}x{K}x{N} f16={out_f16}")
+    p = q41_plan(M, K, N)
+    assert (p.tile_m, p.tile_n) == want and p.splits == splits
+    x = dg.normal(M + K, (M, K)).astype(np.float16)
+    blk = dg.q4_1_blocks(N + K, N, K)
+    c = torch.zeros((M, N), dtype=torch.float16 if out_f16 else torch.float32, device="cuda")
+    na.gemm_q4_1(dev(x), dev(blk), c, n=N, trans_b=True)
+    rows = pc.edge_rows(M, p.tile_m, 101)
+    xr = np.ascontiguousarray(x[rows])
+    want_rows = oracle_rows(lambda r0, r1: oracle.gemm_q4_1(xr, blk, N, trans_b=True, rows=(r0, r1),
+                                                            w_round_f16=True)[r0:r1], len(rows), band=4)
+    assert norm_err(host(c)[rows].astype(np.float32), want_rows) <= TOL
 
 
 @pytest.mark.parametrize("M,K,N2", [(17, 4096, 520), (40, 4096, 2050), (128, 2048, 1032), (200, 4096, 516)])
@@ -107,15 +131,17 @@ def test_q4_1_ring_without_workspace(M):
     assert norm_err(host(c).astype(np.float32), want) <= TOL
 
 
-@pytest.mark.parametrize("M,K,n", [(300, 256, 14336), (512, 96, 16200)])
+@pytest.mark.parametrize("M,K,n,want", pc.Q41_GATED)
 @pytest.mark.parametrize("kw", [dict(), dict(gate_limit=1.5), dict(add_to=True)])
 @pytest.mark.parametrize("f16", [True, False])
-def test_q4_1_gated_tall_tiles(M, K, n, kw, f16):
-    """The fused gated form on its 256-row tiles (ragged rows and columns, the
-    plain SwiGLU and the general combine), bit for bit the product and then
-    the pass."""
+def test_q4_1_gated_tiles(M, K, n, want, kw, f16):
+    """The fused gated form on its 128- and 256-row tiles (ragged rows and
+    columns, the plain SwiGLU and the general combine), bit for bit the product
+    and then the pass."""
     import torch
-    announce(f"q4_1 gated tall {M}x{K}x{n} {kw} f16={f16}")
+    announce(f"q4_1 gated {M}x{K}x{n} {kw} f16={f16}")
+    plan = q41_plan(M, K, 2 * n, L.PLAN_GATED_PASS)
+    assert (plan.tile_m, plan.tile_n) == want and plan.fused
     x, blk = dev(dg.normal(M, (M, K)).astype(np.float16)), dev(dg.q4_1_blocks(n, 2 * n, K))
     tdt = torch.float16 if f16 else torch.float32
     bias = (0.1 * torch.randn(2 * n, device="cuda")).to(tdt)

@@ -1,6 +1,8 @@
-"""The LDS-ring GEMM at the sizes where its plan changes: every tile shape,
-ragged last tiles in both directions, the smallest row counts that take it,
-64-byte k steps, K splits, and a workspace too small for the splits.
+"""The LDS-ring GEMM at the sizes where its plan changes: every tile shape with
+whole and short last stages of k, ragged last tiles in both directions, the
+smallest row counts that take it, K splits, and a workspace too small for the
+splits. plan_cases.py has the shapes whose tile counts, held to the plan by
+test_plan.py.
 
 int8: bit-exact against the oracle. f16: the normalized error of one f16
 rounding (2^-11 of the value) and of an f32 sum over K <= 11008 terms in any
@@ -17,64 +19,76 @@ import datagen as dg
 import nnops_amd as na
 from nnops_amd import ops
 from gpu_util import dev, host, announce, norm_err, oracle_rows, pitched
-from test_plan import i8_plan
+import plan_cases as pc
+from test_plan import i8_plan, f16_plan
 
 pytestmark = pytest.mark.gpu
 
-# (M, K, N): the tile that the shape's plan takes
+# (M, K, N). An odd width of a packed [K,N] weight is copied, not read in place.
 SHAPES = [
-    (17, 704, 68),          # 64 x 64, half a stage last
-    (63, 8192, 132),        # 64 x 64, K split
-    (65, 4096, 260),        # 64 x 64 split, one row past a tile
+    (17, 704, 68),          # gemm_i8_mfma
+    (63, 8192, 132),        # 64 x 64, 16 K splits
+    (65, 4096, 260),        # 64 x 64, 8 splits, one row past a tile
     (500, 256, 4000),       # 128 x 64
-    (130, 4160, 1028),      # split, the last stage half as deep
-    (20, 32, 36),           # one slice of k in all
-    (65, 4128, 260),        # 32 k in the last stage, split
+    (130, 4160, 1028),      # 64 x 64, 5 splits, the last stage half as deep
+    (20, 32, 36),           # gemm_i8_mfma, one slice of k in all
+    (65, 4128, 260),        # 32 k in the last stage, 8 splits
     (333, 1120, 1024),      # 96 k in the last stage
-    (40, 8160, 257),        # split, N % 4 == 1
+    (40, 8160, 257),        # 16 splits, N % 4 == 1
     (200, 288, 4003),       # N % 4 == 3
-    (1000, 96, 16130),      # N % 4 == 2, 256 x 256
-    (500, 256, 4100),       # 128 x 128, last tile 4 columns wide
-    (300, 2048, 1024),      # split over several tiles of rows
+    (1000, 96, 16130),      # N % 4 == 2, 256 x 256, a short stage only
+    (500, 256, 4100),       # 128 x 128, last tile 4 columns wide, f16 through partials
+    (300, 2048, 1024),      # 64 x 64, partials in 3 splits
     (384, 256, 16000),      # 192 x 128
-    (500, 128, 16100),      # 256 x 128
-    (640, 128, 11776),      # 128 x 256
-    (500, 128, 11004),      # 128 x 192
-    (1000, 96, 11008),      # 256 x 192
-    (1000, 128, 16132),     # 256 x 256
+    (500, 128, 16100),      # 256 x 128, one stage, through partials
+    (640, 128, 11776),      # 128 x 256, one stage
+    (500, 128, 11004),      # 128 x 192, one stage, through partials
+    (1000, 96, 11008),      # 256 x 192 (256 x 256 over a [K,N] B), a short stage only
+    (1000, 128, 16132),     # 256 x 256, one stage, through partials
 ]
+
+
+def run_i8(M, K, N, trans_b, out, rows):
+    """One call against the oracle at the given rows (a row's result depends on
+    that row only). s8: the fused requant; s8_tokens: with a scale per row,
+    partials and the reduce; f16: the fused dequantizing output."""
+    seed = M + K + N
+    a = dg.act_s8(seed, (M, K))
+    w = dg.ints(seed + 1, (N, K), -127, 127)
+    sb = dg.uniform(seed + 2, (N,), 0.001, 0.01)
+    kind, okind, dt = {"f16": (na.OUT_F16, oracle.OUT_F16, np.float16),
+                       "s32": (na.OUT_S32, oracle.OUT_S32, np.int32)}.get(out, (na.OUT_S8, oracle.OUT_S8, np.int8))
+    s_a = dg.uniform(seed + 3, (M,), 0.01, 0.03) if out == "s8_tokens" else 0.02
+    bias = dg.ints(seed + 4, (N,), -5000, 5000, np.int32) if out != "f16" else None
+    act = (na.ACT_RELU, oracle.ACT_RELU) if out == "s8" else (na.ACT_NONE, oracle.ACT_NONE)
+    c = dev(np.zeros((M, N), dt))
+    b = w if trans_b else np.ascontiguousarray(w.T)
+    na.gemm_i8(dev(a), dev(b), c, trans_b=trans_b, out_kind=kind, bias=None if bias is None else dev(bias),
+               s_a=dev(s_a) if out == "s8_tokens" else s_a, s_b=dev(sb), s_out=0.4, act=act[0])
+    got = host(c)
+    for r in rows:
+        want = oracle.gemm_i8(a[r:r + 1], w, trans_b=True, bias=bias, out_kind=okind,
+                              s_a=s_a[r:r + 1] if out == "s8_tokens" else s_a, s_b=sb, s_out=0.4, act=act[1])
+        assert np.array_equal(got[r:r + 1].view(np.uint8), want.view(np.uint8)), r
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("out", ["s8", "s8_tokens", "f16"])
-def test_i8_tiles(M, K, N, trans_b, out):
-    """s8: the fused requant; s8 with a scale per row: partials and the
-    reduce; f16: the fused dequantizing output."""
+def test_i8_shapes(M, K, N, trans_b, out):
     announce(f"ring i8 {M}x{K}x{N} tb={trans_b} {out}")
-    seed = M + K + N
-    a = dg.act_s8(seed, (M, K))
-    w = dg.ints(seed + 1, (N, K), -127, 127)
-    sb = dg.uniform(seed + 2, (N,), 0.001, 0.01)
-    kind, dt = (na.OUT_F16, np.float16) if out == "f16" else (na.OUT_S8, np.int8)
-    s_a = dg.uniform(seed + 3, (M,), 0.01, 0.03) if out == "s8_tokens" else 0.02
-    bias = dg.ints(seed + 4, (N,), -5000, 5000, np.int32) if out != "f16" else None
-    c = dev(np.zeros((M, N), dt))
-    b = w if trans_b else np.ascontiguousarray(w.T)
-    na.gemm_i8(dev(a), dev(b), c, trans_b=trans_b, out_kind=kind, bias=None if bias is None else dev(bias),
-               s_a=dev(s_a) if out == "s8_tokens" else s_a, s_b=dev(sb), s_out=0.4,
-               act=na.ACT_RELU if out == "s8" else na.ACT_NONE)
-    got = host(c)
+    run_i8(M, K, N, trans_b, out,
+           sorted({r for e in (0, 64, 128, 192, 256, 384, 512, M) for r in range(e - 2, e + 2) if 0 <= r < M}))
 
-    def rows(r0, r1):
-        return oracle.gemm_i8(a[r0:r1], w, trans_b=True, bias=bias,
-                              out_kind=oracle.OUT_F16 if out == "f16" else oracle.OUT_S8,
-                              s_a=s_a[r0:r1] if out == "s8_tokens" else s_a, s_b=sb, s_out=0.4,
-                              act=oracle.ACT_RELU if out == "s8" else oracle.ACT_NONE)
-    # the rows around every tile edge (a row's result depends on that row only)
-    edges = sorted({r for e in (0, 64, 128, 192, 256, 384, 512, M) for r in range(e - 2, e + 2) if 0 <= r < M})
-    for r in edges:
-        assert np.array_equal(got[r:r + 1].view(np.uint8), rows(r, r + 1).view(np.uint8)), r
+
+@pytest.mark.parametrize("M,K,N,nk,kn", pc.I8_TILES)
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("out", ["s8", "s8_tokens", "s32", "f16"])
+def test_i8_tiles(M, K, N, nk, kn, trans_b, out):
+    announce(f"ring i8 tile {M}x{K}x{N} tb={trans_b} {out}")
+    p = i8_plan(M, K, N, trans_b=trans_b)
+    assert (p.tile_m, p.tile_n) == (nk if trans_b else kn)
+    run_i8(M, K, N, trans_b, out, pc.edge_rows(M, p.tile_m, 41))
 
 
 # [K,N] weights of odd width at a 16-byte pitch: read in place, the last k
@@ -118,7 +132,20 @@ def test_u8_zero_points_short_stage(M, K, N, trans_b):
                                    (1000, 48, 11000)])
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("out_f16", [True, False])
-def test_f16_tiles(M, K, N, trans_b, out_f16):
+def test_f16_shapes(M, K, N, trans_b, out_f16):
+    run_f16(M, K, N, trans_b, out_f16)
+
+
+@pytest.mark.parametrize("M,K,N,want", pc.F16_TILES)
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("out_f16", [True, False])
+def test_f16_tiles(M, K, N, want, trans_b, out_f16):
+    p = f16_plan(M, K, N, trans_b=trans_b)
+    assert (p.tile_m, p.tile_n) == want
+    run_f16(M, K, N, trans_b, out_f16)
+
+
+def run_f16(M, K, N, trans_b, out_f16):
     import torch
     announce(f"ring f16 {M}x{K}x{N} tb={trans_b} f16={out_f16}")
     a = dg.normal(M + K, (M, K)).astype(np.float16)

@@ -8,6 +8,7 @@ import pytest
 
 import nnops_amd as na
 from nnops_amd import _lib as L
+import plan_cases as pc
 
 ALL = 1 << 62       # a workspace with room for any plan
 
@@ -155,3 +156,47 @@ def test_i8_few_rows_short_k(M, K, N, kind, ring):
     [K,N] B, which it would have to copy, they do."""
     assert (i8_plan(M, K, N, out_kind=kind).tile_m > 0) == ring
     assert i8_plan(M, K, N, out_kind=kind, trans_b=False).in_place
+
+
+def tile(p):
+    return p.tile_m, p.tile_n
+
+
+@pytest.mark.parametrize("M,K,N,nk,kn", pc.I8_TILES)
+def test_i8_tile_cases(M, K, N, nk, kn):
+    """The GPU tests' shapes take the tiles that they are there for, with every
+    destination that is fused and through partials (a scale per row)."""
+    for trans_b, want in ((True, nk), (False, kn)):
+        for fields in (dict(), dict(out_kind=na.OUT_S32), dict(out_kind=na.OUT_F16), dict(s_a=FAR)):
+            p = i8_plan(M, K, N, trans_b=trans_b, **fields)
+            assert tile(p) == want and p.in_place == (not trans_b) and p.fused == ("s_a" not in fields)
+
+
+@pytest.mark.parametrize("M,K,N,want", pc.F16_TILES)
+def test_f16_tile_cases(M, K, N, want):
+    for trans_b in (True, False):
+        p = f16_plan(M, K, N, trans_b=trans_b)
+        assert tile(p) == want and p.fused == (N % 8 == 0)
+
+
+@pytest.mark.parametrize("M,K,N,want,splits", pc.Q41_TILES)
+def test_q4_1_tile_cases(M, K, N, want, splits):
+    p = q41_plan(M, K, N)
+    assert tile(p) == want and p.splits == splits and p.fused == (splits == 1)
+
+
+@pytest.mark.parametrize("M,K,n,want", pc.Q41_GATED)
+def test_q4_1_gated_cases(M, K, n, want):
+    p = q41_plan(M, K, 2 * n, L.PLAN_GATED_PASS)
+    assert tile(p) == want and p.fused
+
+
+def test_every_tile_has_its_cases():
+    """Nine int8 and f16 tiles (seven of them in place over a [K,N] B), seven
+    Q4_1 ones and two gated ones, each with whole stages and a short last one."""
+    def forms(cases, k_stage, i):
+        return {(c[i], c[1] % k_stage != 0) for c in cases}
+    assert len(forms(pc.I8_TILES, 128, 3)) == len(forms(pc.F16_TILES, 64, 3)) == 18
+    assert len(forms(pc.I8_TILES, 128, 4)) == 14
+    assert len({(c[3], c[4] > 1, c[1] % 64 != 0) for c in pc.Q41_TILES}) == 26
+    assert len(forms(pc.Q41_GATED, 64, 3)) == 4
