@@ -88,7 +88,9 @@ def _stream_ptr(stream):
     if _RAW_STREAM is None:
         import torch
         torch.cuda.current_stream()          # initialises the device runtime
-        _RAW_STREAM = (torch._C._cuda_getCurrentRawStream, torch.cuda.current_device)
+        # (a private name: a torch without it gives the Stream object's)
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        _RAW_STREAM = (raw or (lambda dev: torch.cuda.current_stream(dev).cuda_stream), torch.cuda.current_device)
     raw, device = _RAW_STREAM
     return raw(device())
 

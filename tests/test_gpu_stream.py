@@ -31,3 +31,16 @@ def test_current_stream():
             stream.synchronize()
         assert np.array_equal(host(c), want)
     assert (ops._stream_ptr(side) or 0) == side.cuda_stream
+
+
+def test_current_stream_without_the_private_name(monkeypatch):
+    """A torch whose raw stream lookup has another name: the Stream object's
+    handle."""
+    import torch
+    announce("current stream, public names only")
+    monkeypatch.setattr(ops, "_RAW_STREAM", None)
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    side = torch.cuda.Stream()
+    for stream in (side, torch.cuda.default_stream()):
+        with torch.cuda.stream(stream):
+            assert (ops._stream_ptr(None) or 0) == stream.cuda_stream
