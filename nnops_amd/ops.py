@@ -59,6 +59,7 @@ def tensor(t, *, dtype=None, shape=None, scale=1.0, zero_point=0, scale_data=Non
         if arr is None:
             continue
         if hasattr(arr, "data_ptr"):
+            keep.append(arr)
             setattr(x, name, arr.data_ptr())
         else:
             import numpy as np
@@ -70,7 +71,7 @@ def tensor(t, *, dtype=None, shape=None, scale=1.0, zero_point=0, scale_data=Non
         x.granularity = granularity
     elif scale_data is not None or zero_point_data is not None:
         x.granularity = 1
-    x._keep = keep + [t]  # the buffers (device tensor, host tables) must outlive the call
+    x._keep = keep + [t]  # the buffers (the tensor, the tables) must outlive the call
     return x
 
 

@@ -379,3 +379,18 @@ def test_q4_1_codec_rejects_before_any_launch():
     assert lib.nnops_hip_q4_1_quantize(None, 0, 2, 64, 64, 16, 40, None) == na.INVALID_ARGUMENT
     assert lib.nnops_hip_q4_1_quantize(None, 0, 0, 64, 64, None, 40, None) == na.OK              # empty
     assert lib.nnops_hip_q4_1_dequantize(16, 36, 2, 64, 16, 0, 64, None) == na.INVALID_ARGUMENT
+
+
+def test_tensor_keeps_its_tables():
+    """A descriptor holds the tensor and its tables, on the device or the host."""
+    import gc
+    import weakref
+    import torch
+    t = torch.zeros((2, 4), dtype=torch.int8)
+    scales, zps = torch.ones(4), torch.zeros(4, dtype=torch.int32)
+    alive = [weakref.ref(x) for x in (t, scales, zps)]
+    x = na.tensor(t, scale_data=scales, zero_point_data=zps, granularity=2)
+    assert (x.scale_data, x.zero_point_data) == (scales.data_ptr(), zps.data_ptr())
+    del t, scales, zps
+    gc.collect()
+    assert all(r() is not None for r in alive)
