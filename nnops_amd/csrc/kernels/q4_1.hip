@@ -64,6 +64,7 @@ struct Q41Kern {
     FpOut fo;            // the fused gated combine (gemm_q4_1_ring with GATED)
     const float* row_scale;  // SPLIT ring: [M] power-of-two factor of each row of A
     int64_t plane;           // SPLIT ring: bytes from the hi plane of A to the lo plane
+    int64_t b_end;           // rings: the end of the last row's last block, in bytes from b
     int kt_per;              // K splits of the ring (64-k stages) and the skinny kernel (stages per part) each;
                              // the last takes the rest
 };
@@ -2696,7 +2697,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_q4_1_ring(Q41Kern p)
                                        (uint32_t)std::min<int64_t>(a_bytes, 0x7fffffff));
     // ends with the last row's last block: a stage's 64 bytes of a row reach
     // past its blocks, which at a wide pitch may be past the operand
-    const int64_t b_bytes = (int64_t)(p.n - 1 - (GATED ? 0 : n0)) * p.ldb + (int64_t)(p.k / 32) * 20;
+    const int64_t b_bytes = p.b_end - (GATED ? 0 : (int64_t)n0 * p.ldb);
     const QBufRsrc rsb = q_buffer_rsrc(p.b + (GATED ? 0 : (int64_t)n0 * p.ldb) + (int64_t)kt0 * 40,
                                        (uint32_t)std::min<int64_t>(b_bytes - (int64_t)kt0 * 40, 0x7fffffff));
     int a_off[QA], b_off[QB];
@@ -3646,6 +3647,7 @@ inline Q41Kern q41_kern(const NnopsGemmQ41Args& g)
     k.lda = g.lda;
     k.ldc = g.ldc;
     k.ldb = g.ldb_bytes;
+    k.b_end = (g.n - 1) * g.ldb_bytes + g.k / 32 * 20;
     k.out_f16 = g.out_kind == NNOPS_OUT_F16;
     k.bdm = g.b_soa ? g.b_dm : nullptr;
     k.ldbdm = g.b_soa ? g.ldb_dm : 0;
@@ -4137,6 +4139,7 @@ extern "C" int nnops_hip_gemm_q4_1_fused(const NnopsGemmQ41Args* g, const NnopsF
     k.k = (int)g->k;
     k.lda = g->lda;
     k.ldb = g->ldb_bytes;
+    k.b_end = (g->n - 1) * g->ldb_bytes + g->k / 32 * 20;
     k.fo = fo;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (pipe_gemv) {
