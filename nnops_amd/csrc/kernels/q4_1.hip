@@ -3474,18 +3474,25 @@ inline Q41RingPlan plan_q41_ring(const NnopsGemmQ41Args& g, int max_splits)
 }
 
 // The fused gated tiles' time: 128 or 256 rows x 128 outputs, one workgroup per
-// CU, and the combine. At 2 x 14336 x 4096 the tall tiles take 512 rows in one
-// round (139 us, 161 in the 128-row tiles' two), 256 rows or fewer the low
-// ones (85 against 113 us). Infinite where the tile's offsets do not fit (its
-// weight rows, N / 2 apart, are the fused entry's own check).
+// CU; per round of 256 of them the first stages and the combine (12 or 17 us) and
+// the steps, which take less where the last round leaves CUs idle (0.75 of it up
+// to 160 of the 256). Within 11 % of 70 shapes (64 to 1300 rows, K 1024 to 14336,
+// 512 to 11008 outputs). At 2 x 14336 x 4096 the tall tiles take 512 rows in one
+// round (134 us, 170 in the 128-row tiles' two). With every round at the full
+// step time (1.17, 1.95) calls that fill part of the CUs went to K splits and a
+// pass, 593 x 2 x 4592 x 11008 178 us against 160 here. Infinite where the tile's
+// offsets do not fit (its weight rows, N / 2 apart, are the fused entry's own
+// check).
 inline float gated_us(const NnopsGemmQ41Args& g, int bm)
 {
     if (!q41_tile_fits(g, bm, 1)) {
         return INFINITY;
     }
     const int64_t tiles = ((g.m + bm - 1) / bm) * ((g.n / 2 + 127) / 128);
-    const float steps = (float)((g.k + 63) / 64);
-    return (float)((tiles + 255) / 256) * (bm == 256 ? steps * 1.95f + 14.0f : steps * 1.17f + 6.0f);
+    const int64_t full = tiles / 256, rest = tiles % 256;
+    const float last = rest == 0 ? 0.0f : 0.75f + 0.25f * std::max(0.0f, (float)(rest - 160) * (1.0f / 96.0f));
+    const float steps = (float)((g.k + 63) / 64) * (bm == 256 ? 1.94f : 1.09f);
+    return ((float)full + last) * steps + (float)(full + (rest != 0 ? 1 : 0)) * (bm == 256 ? 17.0f : 12.0f);
 }
 
 inline bool gated_tall(const NnopsGemmQ41Args& g)
@@ -3600,6 +3607,21 @@ inline Q41RingPlan choose_q41_ring(const NnopsGemmQ41Args& g, size_t ws_bytes, b
     return r;
 }
 
+// The time of a gated product by the plan r and its pass: unsplit, the products
+// are staged as f32 (8 us with the second launch, and their bytes), and of the
+// tiles that share CUs in pairs only those past 256 take longer (380 x 2 x 5504 x
+// 14336, 344 of 96 x 128: 187 us, the fused tiles 196).
+inline float q41_staged_us(const NnopsGemmQ41Args& g, const Q41RingPlan& r)
+{
+    if (r.splits > 1) {
+        return r.us;
+    }
+    const int64_t tiles = ((g.m + r.bm - 1) / r.bm) * ((g.n + r.bn - 1) / r.bn);
+    const bool pairs = r.bn == 128 && tiles > 256 && tiles <= 512;
+    return r.us * (pairs ? (0.5f + (float)tiles * (0.5f / 256.0f)) / 1.55f : 1.0f) + 8.0f +
+           8.0f * (float)g.m * (float)g.n / 3.5e6f;
+}
+
 // How the output pass's call runs: the skinny kernel's or the ring's partials
 // (r) summed by the pass, or neither (the fused gated tiles, or the product
 // and then the pass).
@@ -3618,8 +3640,7 @@ inline Q41PassRoute q41_pass_route(const NnopsGemmQ41Args& g, bool gated, size_t
     }
     if (gated) {
         // the gated form's fused tiles where they are the faster
-        const float staged = r.splits > 1 ? 0.0f : 3.0f + 8.0f * (float)g.m * (float)g.n / 3.5e6f;
-        if (std::min(gated_us(g, 128), gated_us(g, 256)) <= r.us + staged) {
+        if (std::min(gated_us(g, 128), gated_us(g, 256)) <= q41_staged_us(g, r)) {
             return Q41PassRoute::none;
         }
     }

@@ -200,3 +200,11 @@ def test_every_tile_has_its_cases():
     assert len(forms(pc.I8_TILES, 128, 4)) == 14
     assert len({(c[3], c[4] > 1, c[1] % 64 != 0) for c in pc.Q41_TILES}) == 26
     assert len(forms(pc.Q41_GATED, 64, 3)) == 4
+
+
+@pytest.mark.parametrize("M,K,n", [(593, 11008, 4592), (593, 11008, 4593), (700, 11008, 3300), (384, 4096, 8192)])
+def test_q4_1_gated_tiles_past_half_the_cus(M, K, n):
+    """The fused tiles where they fill most of one round: 160 us against 178 in K
+    splits and a pass (593 rows)."""
+    p = q41_plan(M, K, 2 * n, L.PLAN_GATED_PASS)
+    assert p.fused and p.tile_m
