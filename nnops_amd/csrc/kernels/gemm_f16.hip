@@ -141,7 +141,7 @@ F16Plan plan_f16(const NnopsGemmFpArgs& g, size_t room = SIZE_MAX, bool by_rows 
             f.ring.mode = RING_FP;
         }
     } else {
-        f.ring = plan_ring(x, a, x.lda, b, ldb, false, std::max(1, splits_in(room, off, g.m, g.n)));
+        f.ring = plan_ring(x, a, x.lda, b, ldb, false, std::max(1, splits_in(room, off, g.m, g.n)), true);
     }
     // up to 8 rows, two passes of the GEMV, over a k too short to split and with
     // a destination that needs the pass over partials (5 x 768 x 1001: GEMV 7.2

@@ -1746,12 +1746,12 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, const PlanFor& f = PlanFor{})
     // a [K,N] B goes to the ring in place when it takes it and no column
     // sums of B are needed (they are summed over the staged copy's rows)
     const bool need_rb = g.a_u8 || g.zp_a != nullptr || g.zp_a_scalar != 0;
-    // (from 17 rows: 24 x 11008 x 4096 s8 15.8 us on 64 x 64 tiles in four
+    // (from 17 rows: 24 x 11008 x 4096 s8 14.1 us on 64 x 64 tiles in four
     // splits, 52 us on gemm_i8_mfma's 64 workgroups of the whole K)
     const bool ring = g.m > 16 && f.ring;
     auto plan = [&](bool trb) {
         return f.by_rows ? plan_ring_by_rows(g, a, lda, b, ldb, trb, true)
-                         : plan_ring(g, a, lda, b, ldb, trb, std::max(1, splits_in(f.room, off, g.m, g.n)));
+                         : plan_ring(g, a, lda, b, ldb, trb, std::max(1, splits_in(f.room, off, g.m, g.n)), false);
     };
     if (!g.trans_b && !need_rb && ring) {
         w.ring = plan(true);
@@ -1765,14 +1765,14 @@ WsPlan plan_workspace(const NnopsGemmI8Args& g, const PlanFor& f = PlanFor{})
         w.ring = plan(false);
     }
     // few rows over a short k, B's rows k-contiguous: gemm_i8_mfma before the
-    // ring, where the general output pass is needed (one launch, 0.3 us per 64
-    // bytes of k, before the ring and its reduce: 34 x 1024 x 677 11.3 against
+    // ring, where the general output pass is needed (one launch, 2.2 us and 0.3 per
+    // 64 bytes of k, before the ring and its reduce: 34 x 1024 x 677 11.3 against
     // 12.2 us) and where an integer destination is written without a split (us,
     // gemm_i8_mfma / ring, s8: 17 x 256 x 1024 3.4 / 3.8, 17 x 384 x 4096 4.4 /
     // 4.5, 17 x 512 x 4096 5.2 / 5.0, 48 x 768 x 1024 5.0 / 5.2, 17 x 1024 x 1024
     // 6.8 / 6.1; an f16 one 17 x 256 x 1024 8.2 / 4.3)
     const bool short_k = w.ring.mode == RING_PART
-                             ? w.ring.splits == 1 && 0.3f * (float)(g.k / 64) < w.ring.us
+                             ? w.ring.splits == 1 && 2.2f + 0.3f * (float)(g.k / 64) < w.ring.us
                              : w.ring.mode != RING_FP && (g.k <= 384 || (g.k < 1024 && g.n <= 1024));
     if (!f.by_rows && !w.ring.trb && g.m < 64 && short_k) {
         w.ring = RingPlan{};

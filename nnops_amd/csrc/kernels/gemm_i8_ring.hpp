@@ -49,7 +49,7 @@ constexpr int kMostSplits = 16;     // K splits at most
 // The ring plan of an int8 call (ring_plan.hip), and the one by its rows alone;
 // an f16 call asks with its K and row pitches in bytes.
 RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, bool trb,
-                   int max_splits);
+                   int max_splits, bool f16);
 RingPlan plan_ring_by_rows(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb,
                            bool trb, bool small_tiles);
 

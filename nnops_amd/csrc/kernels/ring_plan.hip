@@ -4,21 +4,43 @@
 namespace nnops_amd {
 namespace {
 
-// The ring's tile shapes and the time of one 128-byte k step of one
-// workgroup, with one workgroup on every CU (the loop's time over its steps,
-// at 512 x 4096 x 4096 and up, int8 and f16 operands alike: the step moves
-// the same bytes and runs as many matrix-core cycles). The 192-column tiles
-// (not over a [K,N] B in place) are for widths that leave 128 and 256 columns
-// with a last round nearly empty: 1000 x 4096 x 11008 f16 115 -> 105 us on 232
-// tiles of 256 x 192 against 172 of 256 x 256, 512 rows 67 -> 60 (s8 36 -> 33).
+// The ring's tile shapes and the time of one 128-byte k step of one workgroup
+// with one workgroup on every CU, over [N,K] rows of B and over a [K,N] B in
+// place (0: not taken there). The 192-column tiles are for widths that leave 128
+// and 256 columns with a last round nearly empty: 1000 x 4096 x 11008 f16 115 ->
+// 105 us on 232 tiles of 256 x 192 against 172 of 256 x 256, 512 rows 67 -> 60
+// (s8 36 -> 33).
 struct RingTile {
     int bm, bn;
-    float step_us;
+    float step_us, trb_step_us;
 };
 constexpr RingTile kRingTiles[] = {
-    {64, 64, 0.38f},    {128, 64, 0.48f},   {128, 128, 0.68f},  {192, 128, 0.82f},
-    {128, 192, 0.85f}, {256, 128, 1.08f},  {128, 256, 1.08f},  {256, 192, 1.40f}, {256, 256, 1.80f},
+    {64, 64, 0.31f, 0.58f},    {128, 64, 0.40f, 0.48f},  {128, 128, 0.53f, 0.61f},
+    {192, 128, 0.74f, 0.84f},  {128, 192, 0.75f, 0.0f},  {256, 128, 0.89f, 1.04f},
+    {128, 256, 0.90f, 1.04f},  {256, 192, 1.13f, 0.0f},  {256, 256, 1.28f, 1.30f},
 };
+
+// The step time of the 64 x 64 tiles over a [K,N] B that an XCD's L2 holds: their
+// stages read 64 bytes of each row of B, from further away at half the rate.
+constexpr float kTrbSmallStepUs = 0.37f;
+constexpr int64_t kTrbSmallBytes = 6000000;
+
+// The time of `wgs` workgroups of `steps` k steps each: per round of 256 of them
+// what the first stages and the output take, by the tile's area, and the steps,
+// which take less where a last round leaves CUs idle (the matrix cores' clock and
+// the L2s are shared: down to 0.85 of it at half of the CUs, the small tiles
+// 0.91). A grid that is no multiple of the 8 XCDs is not remapped to them, so
+// that the row tiles of one column band read B into several L2s: 8 % more.
+float ring_us(const RingTile& t, float step_us, uint64_t wgs, uint32_t steps, bool bands)
+{
+    const float area = (float)(t.bm * t.bn);
+    const uint64_t full = wgs / 256, rest = wgs % 256;
+    const float low = t.bm * t.bn > 128 * 128 ? 0.85f : 0.91f;
+    const float last = rest == 0 ? 0.0f : low + (1.0f - low) * std::max(0.0f, (float)rest * (1.0f / 128.0f) - 1.0f);
+    const float us = ((float)full + last) * (float)steps * step_us;
+    return (wgs % 8 != 0 && bands && wgs > 128 ? 1.08f * us : us) +
+           (float)(full + (rest != 0 ? 1 : 0)) * (3.0f + area * (4.3f / 65536.0f));
+}
 
 // The fused output mode a call may take (RING_PART: none): row-uniform
 // parameters, no zero-point terms, half-away rounding, N % 4 == 0, 16-byte
@@ -93,30 +115,31 @@ RingPlan plan_ring_by_rows(const NnopsGemmI8Args& g, const int8_t* a, int64_t ld
 // The ring kernel needs K % 32 == 0 (bytes of k: whole matrix-core slices),
 // 16-byte-aligned k-contiguous rows and 32-bit buffer offsets within a row
 // panel.
-// The tile and the K split are the cheapest by
-//   rounds of 256 workgroups x k steps x the tile's step time
-//   + (partials: 3 us, and their bytes written and read at 3.5 TB/s),
-// since every sweep of tiles and splits (int8 and f16, 24 to 4096 rows) was
-// won by a grid just under one workgroup per CU, whichever tile gives it, and
-// a second workgroup on a CU doubles the time: 512 x 4096 x 4096 s8 18.4 us on
-// 256 tiles of 128 x 64, 21 on 128 of 128 x 128, 27 on 512 of 64 x 64, 35 in
-// eight K splits of 256 x 256; 1024 x 4096 x 4096 24.7 us on 256 tiles of
-// 128 x 128, 42 on 256 x 256 in four splits. The estimate is within 20 % of
-// the measured time where the matrix work or the staging bounds it. The partials
-// of K splits stay under 32 MiB (an unsplit call's, where its mode has any, are
-// one M x N array of 4 bytes), a split keeps at least 512 bytes of k, a k of fewer than
-// 16 steps is not split (the reduce costs more than it gains), and a problem
-// of few rows is split over small tiles only, which bounds the partials (and
-// so the workspace) by those of one tile per CU. max_splits: what a workspace
-// has room for (kMostSplits: all that the plan would take). The fused output
-// modes (fused_mode) go without a split.
+// The tile and the K split are the cheapest by ring_us, plus, with partials, 2.4
+// us and 0.38 us per MB of them (0.71 past 8 splits of int8, whose reduce is then
+// gemm_i8_reduce<16>). That was fitted to 852 shapes of 17 to 2048 rows (int8 s8 /
+// s32 / [K,N], f16; k 256 and widths 128 to 14336), each timed in graphs on 3 to
+// 20 tiles and splits, 7792 times in all: within 8 % of them (one standard
+// deviation). Its choices are 0.9 % slower than the best of each shape's and in 3
+// of 100 by more than 10 %; an estimate by rounds and full step times alone had
+// left 1.6 % and 6 of 100, 907 x 1344 x 9680 over a [K,N] B 32.6 us for 21.0 and
+// 929 x 7616 x 4944 f16 108 for 83.
+// The partials of K splits stay under 64 MiB (an unsplit call's, where its mode
+// has any, are one M x N array of 4 bytes), a split keeps at least 512 bytes of
+// k, a k of fewer than 16 steps is not split (the reduce costs more than it
+// gains), and a problem of few rows is split over small tiles only, which bounds
+// the partials (and so the workspace) by those of one tile per CU; tiles of 192
+// and 256 rows that are over twice its rows are not looked at. max_splits:
+// what a workspace has room for (kMostSplits: all that the plan would take). The
+// fused output modes (fused_mode) go without a split.
 // trb: B is the caller's [K,N] (row pitch ldb), read in place (its whole
-// span within 32-bit buffer offsets).
+// span within 32-bit buffer offsets). f16: f16 operands.
 RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const int8_t* b, int64_t ldb, bool trb,
-                   int max_splits)
+                   int max_splits, bool f16)
 {
     RingPlan r;
-    if (g.m < 1 || g.n < 1 || g.m > INT32_MAX || g.n > INT32_MAX - 3 || g.k > INT32_MAX - 127 || g.k < 32 || g.k % 32 != 0 || !aligned16(a, lda) || !aligned16(b, ldb)) {
+    if (g.m < 1 || g.n < 1 || g.m > INT32_MAX || g.n > INT32_MAX - 3 || g.k > INT32_MAX - 127 || g.k < 32 ||
+        g.k % 32 != 0 || !aligned16(a, lda) || !aligned16(b, ldb)) {
         return r;
     }
     if (trb && (g.k * ldb + g.n >= (int64_t)INT32_MAX || ldb < g.n)) {
@@ -125,20 +148,26 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
     const int fused = fused_mode(g);
     const uint32_t m = (uint32_t)g.m, n = (uint32_t)g.n, kt = (uint32_t)((g.k + 127) / 128);
     const float out_bytes = 4.0f * (float)m * (float)n;
-    const uint32_t most = std::min({(uint32_t)max_splits, kt / 4u, (uint32_t)(32.0f * 1024 * 1024 / out_bytes)});
+    const uint32_t most = std::min({(uint32_t)max_splits, kt / 4u, (uint32_t)(64.0f * 1024 * 1024 / out_bytes)});
     const int split_area = m <= 256 ? 256 * 128 : m <= 384 ? 192 * 128 : 256 * 256;
     float best = 0.0f;
     for (const RingTile& t : kRingTiles) {
-        if ((trb && t.bn == 192) || t.bm * lda >= (int64_t)INT32_MAX ||
+        float step_us = trb ? t.trb_step_us : t.step_us;
+        if (step_us == 0.0f || (t.bm > 128 && (uint32_t)t.bm > 2 * m) || t.bm * lda >= (int64_t)INT32_MAX ||
             (!trb && t.bn * ldb >= (int64_t)INT32_MAX)) {
             continue;
         }
-        const uint64_t tiles = (uint64_t)((m + t.bm - 1) / (uint32_t)t.bm) * ((n + t.bn - 1) / (uint32_t)t.bn);
-        auto consider = [&](uint32_t sp, uint64_t rounds) {
+        if (trb && t.bm * t.bn == 64 * 64 && g.k * g.n < kTrbSmallBytes) {
+            step_us = kTrbSmallStepUs;
+        }
+        const uint32_t row_tiles = (m + (uint32_t)t.bm - 1) / (uint32_t)t.bm;
+        const uint64_t tiles = (uint64_t)row_tiles * ((n + (uint32_t)t.bn - 1) / (uint32_t)t.bn);
+        auto consider = [&](uint32_t sp) {
             const uint32_t steps = kt - (sp - 1) * (kt / sp);       // the last split's, the longest
             const bool part = sp > 1 || fused == RING_PART;
-            const float us = (float)rounds * (float)steps * t.step_us +
-                             (part ? 3.0f + 2.0f * (float)sp * out_bytes / 3.5e6f : 0.0f);
+            const float byte_us = !f16 && sp > 8 ? 0.71e-6f : 0.38e-6f;
+            const float us = ring_us(t, step_us, tiles * sp, steps, row_tiles > 1) +
+                             (part ? 2.4f + (float)sp * out_bytes * byte_us : 0.0f);
             if (r.bm == 0 || us < best) {
                 best = us;
                 r.bm = t.bm;
@@ -147,15 +176,17 @@ RingPlan plan_ring(const NnopsGemmI8Args& g, const int8_t* a, int64_t lda, const
                 r.mode = part ? RING_PART : fused;
             }
         };
-        consider(1, (tiles + 255) / 256);
+        consider(1);
         if (tiles <= 128 && kt >= 16 && t.bm * t.bn <= split_area) {
-            // the split that fills the CUs, and half of it
-            const uint32_t sp = std::min(most, 256u / (uint32_t)tiles);
-            if (sp > 1) {
-                consider(sp, 1);
+            // the split that fills the CUs, parts of it, and the least
+            const uint32_t top = std::min(most, 256u / (uint32_t)tiles);
+            for (const uint32_t sp : {top, top / 2, top / 3}) {
+                if (sp > 2) {
+                    consider(sp);
+                }
             }
-            if (sp > 3) {
-                consider(sp / 2, 1);
+            if (top >= 2) {
+                consider(2);
             }
         }
     }

@@ -93,8 +93,7 @@ def test_i8_tiles(M, K, N, nk, kn, trans_b, out):
 
 # [K,N] weights of odd width at a 16-byte pitch: read in place, the last k
 # row's last columns in a dword that N ends inside
-@pytest.mark.parametrize("M,K,N,tile_m", [(17, 768, 257, 64), (40, 1120, 1001, 64), (333, 4096, 1002, 64),
-                                          (500, 1152, 5002, 128), (700, 1056, 8001, 192), (1000, 416, 16001, 256)])
+@pytest.mark.parametrize("M,K,N,tile_m", pc.I8_IN_PLACE_ODD)
 def test_i8_in_place_odd_columns(M, K, N, tile_m):
     announce(f"ring i8 in place {M}x{K}x{N}")
     plan = i8_plan(M, K, N, trans_b=False, ldb=(N + 15) // 16 * 16, ldc=N, out_kind=na.OUT_S32)

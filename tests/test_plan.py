@@ -172,6 +172,12 @@ def test_i8_tile_cases(M, K, N, nk, kn):
             assert tile(p) == want and p.in_place == (not trans_b) and p.fused == ("s_a" not in fields)
 
 
+@pytest.mark.parametrize("M,K,N,tile_m", pc.I8_IN_PLACE_ODD)
+def test_i8_in_place_odd_cases(M, K, N, tile_m):
+    p = i8_plan(M, K, N, trans_b=False, ldb=(N + 15) // 16 * 16, out_kind=na.OUT_S32)
+    assert p.in_place and p.tile_m == tile_m
+
+
 @pytest.mark.parametrize("M,K,N,want", pc.F16_TILES)
 def test_f16_tile_cases(M, K, N, want):
     for trans_b in (True, False):
@@ -200,6 +206,27 @@ def test_every_tile_has_its_cases():
     assert len(forms(pc.I8_TILES, 128, 4)) == 14
     assert len({(c[3], c[4] > 1, c[1] % 64 != 0) for c in pc.Q41_TILES}) == 26
     assert len(forms(pc.Q41_GATED, 64, 3)) == 4
+
+
+@pytest.mark.parametrize("M,K,N,trans_b,want,splits", [
+    (907, 1344, 9680, False, (256, 256), 1),        # 21 us; two rounds of 192 x 128 33
+    (1551, 1024, 5904, False, (256, 256), 1),       # 18; 25
+    (858, 6144, 11008, False, (256, 256), 1),       # 75; 86
+    (218, 14336, 4240, True, (256, 128), 7),        # 31; 41 in 5 splits of 128 x 192
+    (97, 11008, 1232, True, (64, 64), 6)])          # 12.5; 15.2 in 12 splits of 128 x 64
+def test_i8_cheapest(M, K, N, trans_b, want, splits):
+    """Shapes that an estimate without the CUs' fill, the [K,N] steps and the
+    reduce of many splits had given slower tiles."""
+    p = i8_plan(M, K, N, trans_b=trans_b)
+    assert tile(p) == want and p.splits == splits
+
+
+@pytest.mark.parametrize("M,K,N,splits", [(997, 13056, 4608, 3), (414, 14336, 10096, 3), (929, 7616, 4944, 3)])
+def test_f16_splits_past_32_mib(M, K, N, splits):
+    """Partials of up to 64 MiB where they are the faster: 126 us in 3 splits
+    against 158 unsplit, 159 against 192 in 2, 83 against 108 unsplit."""
+    p = f16_plan(M, K, N)
+    assert tile(p) == (256, 256) and p.splits == splits and p.workspace_bytes <= 64 << 20
 
 
 @pytest.mark.parametrize("M,K,n", [(593, 11008, 4592), (593, 11008, 4593), (700, 11008, 3300), (384, 4096, 8192)])
