@@ -9,7 +9,8 @@
 namespace nnops_amd {
 namespace {
 
-// The same for 2-byte elements (an f16 [K][N] B staged as [N][Kp]).
+// dst[c][r] = src[r][c] over 64 x 64 tiles in LDS, rows R to Rp of dst's rows
+// 0 (an f16 [K][N] B staged as [N][Kp]). Bound: HBM.
 __global__ __launch_bounds__(256) void transpose_b16(const uint16_t* src, int64_t lds_, int R, int C,
                                                     uint16_t* dst, int64_t ldd, int Rp)
 {
@@ -98,9 +99,10 @@ inline bool gemv_f16_faster(const NnopsGemmFpArgs& g)
 }
 
 // From 3 rows over [N][K] rows of B (4096 x 4096: 16 rows 13.7 us against the
-// GEMV's 21.4) and from 17 over a [K][N] B, whose transposed copy the GEMV needs not (17 to 63
-// rows on gemm_fp_tile, in f32: 475 us). room: the workspace that K splits may
-// use. by_rows: the plan by the call's rows alone, whose workspace is enough.
+// GEMV's 21.4), but where the GEMV is the faster, and from 17 over a [K][N] B,
+// whose transposed copy the GEMV needs not (17 to 63 rows on gemm_fp_tile, in
+// f32: 475 us). room: the workspace that K splits may use. by_rows: the plan by
+// the call's rows alone, whose workspace is enough.
 F16Plan plan_f16(const NnopsGemmFpArgs& g, size_t room = SIZE_MAX, bool by_rows = false)
 {
     F16Plan f;

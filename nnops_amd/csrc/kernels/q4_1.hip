@@ -893,7 +893,8 @@ __global__ __launch_bounds__(256) void gemv_q4_1_pipe(Q41Kern p)
 // 14336, N = 4096: 1024 workgroups of 40 KiB, four per CU). Bound: HBM and the
 // decode, as the K = 4096 form. The register form it replaces there
 // (gemv_q4_1_rows) loops over K with two loads in flight per row. K = 14336,
-// N = 4096: M = 1 16.1 -> 11.6 us, M = 2 21.9 -> 14.2; K = 11008: 15.8 -> 11.3.
+// N = 4096: M = 1 16.6 -> 11.1 us, M = 2 21.3 -> 13.3; K = 11008: 15.0 -> 10.1 and
+// 18.8 -> 12.2 (twelve weights in turn, from HBM).
 // ---------------------------------------------------------------------------
 template <int MT, int KW>
 __global__ __launch_bounds__(256) void gemv_q4_1_parts(Q41Kern p)
@@ -2643,7 +2644,7 @@ __device__ __forceinline__ v8h decode8_f16(uint32_t lo0, uint32_t lo1, v2h d2, v
 // pass: 108 against 98 us at 512 x 14336 x 4096, the pass's arithmetic then
 // running with the matrix cores idle; the gated form saves the larger
 // staging.) 512 x 2 x 14336 x 4096: 173 us on 128-row tiles with a branching
-// combine, 161 with the straight-line one, 139 on 256-row tiles.
+// combine, 161 with the straight-line one, 134 on 256-row tiles.
 // TAIL: K % 64 == 32. (A form of its own: with the last stage's code in every
 // kernel the K loop's schedule lost 2 %, 495 x 11008 x 11008 171 -> 174.5 us.)
 template <int OUT, int NS, int WM, int WN = 4, bool GATED = false, bool SPLIT = false, int BM = 128, int BN = 256,
@@ -3332,8 +3333,6 @@ inline bool use_gemv(const NnopsGemmQ41Args& g)
     return g.m <= 2 || (!g.a_f16 && g.m <= kF32GemvRows);
 }
 
-// The blocks-along-N ring: f16 A with 16-byte rows, K % 64 == 0, 16-byte B
-// rows, and every stage offset within a buffer resource's 31-bit range
 // The skinny MFMA GEMM (gemv_q4_1_skinny): blocks along K, f16 A with 16-byte
 // rows, 3 <= M <= 48 (launches of 16 rows; with f16 A past 16 rows only where
 // the ring's K splits have no workspace), K % 256 == 0, 16-byte weight rows,
@@ -3361,6 +3360,8 @@ inline bool bcm_ok(const NnopsGemmQ41Args& g)
     return g.b_soa && !g.trans_b && g.a_f16 && g.k % 8 == 0 && (g.lda % 8) == 0 && ((uintptr_t)g.a & 15) == 0;
 }
 
+// The blocks-along-N ring: f16 A with 16-byte rows, K % 64 == 0, 16-byte B
+// rows, and every stage offset within a buffer resource's 31-bit range.
 inline bool kn_ring_ok(const NnopsGemmQ41Args& g)
 {
     return !g.trans_b && g.a_f16 && g.k % 64 == 0 && (g.lda % 8) == 0 && ((uintptr_t)g.a & 15) == 0 &&
